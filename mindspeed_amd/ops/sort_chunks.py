@@ -51,9 +51,13 @@ class _SortChunks(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out, grad_probs, _grad_map):
         (inverse_map,) = ctx.saved_tensors
-        if grad_out is None:
-            return None, None, None, None
         gp = grad_probs.contiguous() if ctx.has_probs and grad_probs is not None else None
+        if grad_out is None:
+            if gp is None:
+                return None, None, None, None
+            # the rows had no part in the loss: the probabilities go back as rows of one element
+            gp_in, _ = K.gather_rows(gp.view(-1, 1), None, inverse_map)
+            return None, None, None, gp_in.view(gp.shape)
         gi, gp_in = K.gather_rows(grad_out.contiguous(), gp, inverse_map)
         return gi, None, None, (gp_in if gp is not None else None)
 

@@ -126,6 +126,28 @@ def test_sort_chunks_rows_left_out_are_zeros(hidden, dtype, pdt, device):
     assert torch.equal(gx.cpu(), exp_g) and torch.equal(gprobs.cpu(), exp_gp)
 
 
+@pytest.mark.parametrize("pdt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(300,), (300, 1)])
+def test_sort_chunks_gradient_of_the_probabilities_alone(shape, pdt, device):
+    """A loss that reads the moved probabilities and not the rows: their gradient comes back by the same map (exact), the
+    rows get none."""
+    say("sort_chunks probs alone", shape, pdt)
+    gen = torch.Generator().manual_seed(11)
+    sizes, order = torch.tensor([70, 0, 41, 130, 59]), torch.tensor([3, 1, 0, 4, 2])
+    p, gp = (torch.rand(shape, generator=gen).to(pdt) for _ in range(2))
+    starts = torch.cumsum(sizes, 0) - sizes
+    source = torch.cat([torch.arange(starts[i], starts[i] + sizes[i]) for i in order.tolist()])
+    exp = torch.empty_like(gp)
+    exp[source] = gp
+    for form in ("lists", "device"):
+        xd = torch.randn(300, 24, generator=gen).to(device).requires_grad_(True)
+        pd = p.to(device).requires_grad_(True)
+        chunks = (sizes.tolist(), order.tolist()) if form == "lists" else (sizes.to(device), order.to(device))
+        _, out_p = ops.sort_chunks_by_idxs(xd, *chunks, pd)
+        out_p.backward(gp.to(device))
+        assert xd.grad is None and pd.grad.shape == p.shape and torch.equal(pd.grad.cpu(), exp)
+
+
 @pytest.mark.parametrize("dtype,pdt", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32),
                                        (torch.float32, torch.float32)])
 @pytest.mark.parametrize("nchunks,rows,hidden", [(64, 8192, 512), (1500, 6000, 24), (2600, 40000, 8), (7, 300, 13)])

@@ -265,6 +265,19 @@ def test_shapes_propagate_on_meta_tensors():
     assert xc.grad.shape == (T, H) and pc.grad.shape == (T,)
 
 
+def test_sort_chunks_backward_of_either_output_on_meta_tensors():
+    """Each output of the chunk sort carries a gradient by itself: a loss on the moved probabilities alone reaches them."""
+    x = torch.empty(24, 16, dtype=torch.bfloat16, device="meta", requires_grad=True)
+    sizes, order = (torch.empty(4, dtype=torch.int64, device="meta") for _ in range(2))
+    for shape in ((24,), (24, 1)):
+        p = torch.empty(shape, dtype=torch.float32, device="meta", requires_grad=True)
+        out, out_p = ops.sort_chunks_by_idxs(x, sizes, order, p)
+        (gp,) = torch.autograd.grad(out_p, p, torch.empty_like(out_p), retain_graph=True)
+        assert gp.shape == p.shape and gp.dtype == p.dtype
+        gx, gp = torch.autograd.grad(out, (x, p), torch.empty_like(out), allow_unused=True)
+        assert gx.shape == x.shape and gp is None
+
+
 def test_caller_side_modules_run_on_meta_tensors():
     """The expert module (one-node and op-by-op bodies, with activation recomputation), ``BF16GMMFunction`` and the fused
     chunk sort's own names carry shapes and gradients on meta tensors: no device is needed to trace them."""
