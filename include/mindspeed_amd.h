@@ -318,7 +318,8 @@ int ms_sort_chunks(ms_stream_t stream, const void *input, const int64_t *split_s
                    int dtype, const void *probs, int probs_dtype, void *out, void *out_probs,
                    int32_t *row_map);
 /* The same with the map in the other direction: inverse_map int32 [rows], entry r = output row of source row r
- * (-1 for a source row that no named chunk holds).  Output rows that no chunk fills are written as zeros. */
+ * (-1 for a source row that no named chunk holds; of a chunk named more than once, the row of its first copy).  Output
+ * rows that no chunk fills are written as zeros. */
 int ms_sort_chunks_inverse(ms_stream_t stream, const void *input, const int64_t *split_sizes,
                            const int64_t *sorted_idxs, int64_t num_chunks, int64_t rows, int64_t hidden,
                            int dtype, const void *probs, int probs_dtype, void *out, void *out_probs,

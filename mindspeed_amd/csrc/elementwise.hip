@@ -163,23 +163,25 @@ __device__ __forceinline__ void move_scalar(const void *in, void *out, int bytes
 // experts x ranks, a few thousand at most), finds the position of each of its output rows by bisection, and
 // copies the rows with `lanes` threads per row.  Output rows past the sum of the sizes get row_map = -1; malformed
 // chunk indices count as empty chunks.  Such rows are left alone, or written as zeros with `zero_rest`.
-// inverse_map (optional): entry r = output row of source row r, -1 where no chunk that sorted_idxs names holds it.  With
-// it the way back is a gather that knows which rows to zero, so neither direction needs a pass of zeros over its output
-// first: 16384 x 7168 bf16 rows in 64 chunks, both directions, 238 -> 172 us (5.5 TB/s of copied bytes).
+// inverse_map (optional): entry r = output row of source row r, -1 where no chunk that sorted_idxs names holds it; of a
+// chunk that is named more than once, the row of its first copy (every workgroup scans for itself, so which copy counts
+// must not depend on the order of its threads).  With it the way back is a gather that knows which rows to zero, so
+// neither direction needs a pass of zeros over its output first: 16384 x 7168 bf16 rows in 64 chunks, both directions, 238 -> 172 us (5.5 TB/s of copied bytes).
 template <typename VecT>
 __global__ __launch_bounds__(1024) void sort_chunks_kernel(
     const VecT *__restrict__ in, VecT *__restrict__ out, const int64_t *__restrict__ split_sizes,
     const int64_t *__restrict__ sorted_idxs, int num_chunks, int rows, int vecs_per_row, int lanes,
     const void *__restrict__ probs, void *__restrict__ out_probs, int probs_bytes, int32_t *__restrict__ row_map,
     int32_t *__restrict__ inverse_map, int zero_rest) {
-    // src_start[num_chunks + 1], dst_start[num_chunks + 1], scratch[32], then 16-bit src_of[num_chunks], pos_of[num_chunks]
+    // src_start[num_chunks + 1], dst_start[num_chunks + 1], scratch[32], pos_of[num_chunks], then 16-bit src_of[num_chunks]
+    // (4096 chunks must fit in the 64 KB that a launch has without asking for more)
     extern __shared__ int lds[];
-    constexpr unsigned short kNone = 0xffff;      // (num_chunks is at most 4096)
+    constexpr int kNone = 0xffff;
     int *src_start = lds;
     int *dst_start = src_start + num_chunks + 1;
     int *scratch = dst_start + num_chunks + 1;
-    unsigned short *src_of = reinterpret_cast<unsigned short *>(scratch + 32);
-    unsigned short *pos_of = src_of + num_chunks;
+    int *pos_of = scratch + 32;
+    unsigned short *src_of = reinterpret_cast<unsigned short *>(pos_of + num_chunks);
     const int tid = threadIdx.x;
     const int nthreads = blockDim.x;
     for (int i = tid; i < num_chunks; i += nthreads) pos_of[i] = kNone;
@@ -188,16 +190,16 @@ __global__ __launch_bounds__(1024) void sort_chunks_kernel(
     for (int c0 = 0; c0 < num_chunks; c0 += nthreads) {
         const int i = c0 + tid;
         int size = 0, moved = 0;
-        unsigned short src = kNone;
+        int src = kNone;
         if (i < num_chunks) {
             const int64_t sz = split_sizes[i];
             size = static_cast<int>(sz < 0 ? 0 : (sz > rows ? rows : sz));
             const int64_t sidx = sorted_idxs[i];
             if (sidx >= 0 && sidx < num_chunks) {
-                src = static_cast<unsigned short>(sidx);
+                src = static_cast<int>(sidx);
                 const int64_t ms = split_sizes[sidx];
                 moved = static_cast<int>(ms < 0 ? 0 : (ms > rows ? rows : ms));
-                pos_of[src] = static_cast<unsigned short>(i);
+                atomicMin(&pos_of[src], i);
             }
         }
         const int s_ex = carry_s + block_exclusive_scan(size, scratch);
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(1024) void sort_chunks_kernel(
         if (i < num_chunks) {
             src_start[i] = s_ex;
             dst_start[i] = d_ex;
-            src_of[i] = src;
+            src_of[i] = static_cast<unsigned short>(src);
         }
         if (tid == nthreads - 1) {
             scratch[16] = s_ex + size;
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(1024) void sort_chunks_kernel(
     const int r = blockIdx.x * (nthreads / lanes) + local_row;
     if (r >= rows) return;
     // row r counted along `from`, seen along `to`: the last chunk that starts at or before it, and where that chunk lies there
-    auto locate = [&](const int *from, const int *to, const unsigned short *other) {
+    auto locate = [&](const int *from, const int *to, const auto *other) {
         int lo = 0, hi = num_chunks + 1;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
@@ -390,7 +392,7 @@ int launch_sort_chunks(hipStream_t stream, const void *in, void *out, const int6
     // fat workgroups repeat the scan of the chunk sizes less often; keep one per compute unit
     int threads = 1024;
     while (threads > 256 && ceil_div(rows, threads / lanes) < 256) threads >>= 1;
-    const size_t lds = (3 * static_cast<size_t>(num_chunks) + 2 + 32) * sizeof(int);
+    const size_t lds = (3 * static_cast<size_t>(num_chunks) + 2 + 32) * sizeof(int) + static_cast<size_t>(num_chunks) * sizeof(unsigned short);
     hipLaunchKernelGGL(sort_chunks_kernel<VecT>, dim3(static_cast<unsigned>(ceil_div(rows, threads / lanes))), dim3(threads),
                        lds, stream, static_cast<const VecT *>(in), static_cast<VecT *>(out), split_sizes, sorted_idxs,
                        static_cast<int>(num_chunks), static_cast<int>(rows), static_cast<int>(vecs), lanes, probs,

@@ -9,7 +9,8 @@ tensors; nothing is read back to the host.  Given as host lists they are checked
 (``sorted_idxs`` a permutation, the sizes summing to the row count, which the
 reference's ``split`` / ``cat`` require too); device tensors cannot be checked
 without a read-back: rows that a partial list leaves out are written as zeros,
-in the outputs and in the gradients.
+in the outputs and in the gradients, and a chunk that the list names more than
+once gets the gradient of its first copy.
 """
 from __future__ import annotations
 

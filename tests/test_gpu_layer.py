@@ -126,6 +126,31 @@ def test_sort_chunks_rows_left_out_are_zeros(hidden, dtype, pdt, device):
     assert torch.equal(gx.cpu(), exp_g) and torch.equal(gprobs.cpu(), exp_gp)
 
 
+@pytest.mark.parametrize("order", [[0, 0], [0, 1, 0], [2, 1, 2, 0], [1] * 70, [3, 0, 3, 3, 1, 0],
+                                   list(range(1, 4096)) + [2047]])
+def test_sort_chunks_gradient_of_a_repeated_chunk(order, device):
+    """Chunk lists on the device that name a chunk more than once: every copy is written forward, and the chunk's rows get
+    the gradient of the first copy, whole, whichever workgroup computes them (exact: copies)."""
+    say("sort_chunks repeated", len(order), order[:6])
+    gen = torch.Generator().manual_seed(len(order))
+    n, hidden = len(order), 520
+    size = 90 if n < 100 else 2
+    rows = n * size
+    x, g = (torch.randn(rows, hidden, generator=gen) for _ in range(2))
+    p, gp = (torch.rand(rows, generator=gen) for _ in range(2))
+    source = torch.cat([torch.arange(c * size, (c + 1) * size) for c in order])
+    exp_g, exp_gp = torch.zeros_like(x), torch.zeros_like(p)
+    for c in set(order):
+        first = order.index(c) * size
+        exp_g[c * size:(c + 1) * size] = g[first:first + size]
+        exp_gp[c * size:(c + 1) * size] = gp[first:first + size]
+    xd, pd = x.to(device).requires_grad_(True), p.to(device).requires_grad_(True)
+    out, out_p = ops.sort_chunks_by_idxs(xd, torch.full((n,), size).to(device), torch.tensor(order).to(device), pd)
+    assert torch.equal(out.detach().cpu(), x[source]) and torch.equal(out_p.detach().cpu(), p[source])
+    gx, gprobs = torch.autograd.grad((out, out_p), (xd, pd), (g.to(device), gp.to(device)))
+    assert torch.equal(gx.cpu(), exp_g) and torch.equal(gprobs.cpu(), exp_gp)
+
+
 @pytest.mark.parametrize("pdt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [(300,), (300, 1)])
 def test_sort_chunks_gradient_of_the_probabilities_alone(shape, pdt, device):
