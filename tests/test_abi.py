@@ -3,6 +3,7 @@ host-side argument validation works without a GPU (no compute calls here)."""
 import ctypes
 import glob
 import os
+import random
 import re
 
 import pytest
@@ -97,33 +98,78 @@ def test_tile_order_visits_every_tile_once():
     assert lib.ms_gmm_tile_order(0, 4, 0, ctypes.byref(row), ctypes.byref(col)) != 0
 
 
+def _cdiv(a, b):
+    return -(-a // b)
+
+
+def _slots_needed_split_on_rows(counts, m, k, n):
+    """Slots per XCD of the tables the schedule kernel can write for these group sizes (256 x 256 tiles): the common table,
+    the common table with every small tail tile cut in parts, and the per-XCD lists (None where they are not taken)."""
+    cols = _cdiv(n, 256)
+    row_tiles = [_cdiv(c, 256) for c in counts]
+    tiles = sum(row_tiles) * cols
+    zero_fill = _cdiv(m - sum(counts), 256) * cols               # rows past the last group are written as zeros
+    tail_tiles = sum(1 for c in counts if 1 <= (c - 1) % 256 + 1 <= 128 and c > 0) * cols
+    parts = min(256 // tail_tiles, k // 2048, 4) if tail_tiles else 1
+    split = tiles + max(parts - 1, 0) * tail_tiles
+    lists = None
+    if 16 <= len(counts) <= 256 and max(row_tiles) <= 8:
+        load = [0] * 8
+        for rank, t in enumerate(sorted(row_tiles, reverse=True)):
+            load[7 - rank % 8 if rank // 8 % 2 else rank % 8] += t * cols
+        if tiles > 0 and max(load) * 800 <= tiles * 103:
+            lists = max(load) + _cdiv(zero_fill, 8)
+    return _cdiv(tiles + zero_fill, 8), _cdiv(split + zero_fill, 8), lists
+
+
 def test_launch_has_slots_for_every_table_the_schedule_can_write():
-    """Workgroups per XCD of a grouped-matmul launch against the most slots a tile table can need (host arithmetic).
-    Common table: every group's eighth of its tiles, rounded up.  Per-XCD lists with the split on the reduction dim:
-    the XCD with the most groups holds ceil(G / 8) output blocks, e.g. 3 of 17, which is more than an eighth of all
-    tiles when G is not a multiple of 8."""
+    """Workgroups per XCD of a grouped-matmul launch (exactly what is launched) against the slots that the tables of many
+    group lists need, evaluated on the host: ragged, equal and empty groups, fewer rows than groups, rows past the last
+    group, split tail tiles, whole groups per XCD.  The launch carries no workgroup beyond its bound either: a workgroup
+    without a tile still waits for a compute unit."""
     lib = _lib.load()
     slots = ctypes.c_int64(0)
-    cdiv = lambda a, b: -(-a // b)
-    for G in (1, 8, 16, 17, 20, 23, 24, 31, 33, 64, 100, 255, 256):
+
+    def launched(G, m, k, n, group_type, lists, split):
+        assert lib.ms_gmm_launch_slots(G, m, k, n, group_type, lists, split, ctypes.byref(slots)) == 0
+        return slots.value
+
+    # Split on the reduction dim: every group has all its tiles, also an empty one, so the common table needs an eighth of
+    # them.  Per-XCD lists: the XCD with the most groups holds ceil(G / 8) output blocks, e.g. 3 of 17.
+    for G in (1, 8, 16, 17, 20, 23, 24, 31, 33, 64, 100, 255, 256, 4096):
         for k, n in ((2048, 8192), (2880, 2880), (256, 256), (4096, 4096), (8, 8), (1000, 520)):
-            out_tiles = cdiv(k, 256) * cdiv(n, 256)
-            for lists in (0, 1):
-                assert lib.ms_gmm_launch_slots(G, 4096, k, n, 2, lists, 0, ctypes.byref(slots)) == 0
-                need_common = G * cdiv(out_tiles, 8)
-                assert slots.value >= need_common, (G, k, n, lists, slots.value, need_common)
-                if lists:
-                    need_lists = cdiv(G, 8) * out_tiles
-                    assert slots.value >= need_lists, (G, k, n, slots.value, need_lists)
-    # split on rows: at most ceil(m / 256) + G + 1 row tiles (every group and the zero-fill pseudo-group may end in a
-    # partly filled one); with lists the fullest XCD holds at most 1.03 times an eighth of the groups' tiles plus its
-    # eighth of the pseudo-group's, rounded up
-    for G in (8, 17, 64, 256):
-        for m, n in ((8192, 4096), (65536, 2816), (100, 8)):
-            tiles = (cdiv(m, 256) + G + 1) * cdiv(n, 256)
-            assert lib.ms_gmm_launch_slots(G, m, 4096, n, 0, 1, 0, ctypes.byref(slots)) == 0
-            assert slots.value >= cdiv(tiles * 103, 800) + 1
-            assert lib.ms_gmm_launch_slots(G, m, 4096, n, 0, 0, 1, ctypes.byref(slots)) == 0
-            assert slots.value >= cdiv(tiles + 256, 8) + G
+            out_tiles = _cdiv(k, 256) * _cdiv(n, 256)
+            assert launched(G, 4096, k, n, 2, 0, 0) == _cdiv(G * out_tiles, 8)
+            assert launched(G, 4096, k, n, 2, 1, 0) == _cdiv(G, 8) * out_tiles
+
+    # Split on rows: at most ceil(m / 256) + G + 1 row tiles (every group and the zero-fill pseudo-group may end in a partly
+    # filled one) and at most one per row.
+    rng = random.Random(0)
+    with_lists = fullest = 0
+    for trial in range(4000):
+        G = rng.choice([1, 2, 3, 8, 16, 17, 20, 24, 33, 64, 100, 255, 256, 300])
+        k, n = rng.choice([72, 2048, 4096, 14336]), rng.choice([8, 264, 1408, 4096, 28672])
+        kind = rng.randrange(5)
+        if kind == 0:
+            counts = [rng.randrange(0, 3) for _ in range(G)]                  # fewer rows than groups, many empty
+        elif kind == 1:
+            counts = [rng.choice([1, 257, 513, 128, 129]) for _ in range(G)]   # every last tile nearly empty
+        elif kind == 2:
+            counts = [rng.randrange(1, 9) * 256] * G                           # equal groups of whole tiles
+        elif kind == 3:
+            counts = [int(rng.expovariate(1 / 700)) for _ in range(G)]
+        else:
+            counts = [256 * rng.randrange(1, 4) + rng.randrange(256) for _ in range(G)]
+        m = max(sum(counts) + rng.choice([0, 0, 1, 255, 257, 3000]), 1)
+        common, split, lists = _slots_needed_split_on_rows(counts, m, k, n)
+        got = launched(G, m, k, n, 0, 0, 0)
+        assert common <= got, (counts, m, n, common, got)
+        assert got == _cdiv(min(_cdiv(m, 256) + G + 1, m) * _cdiv(n, 256), 8)
+        assert split <= launched(G, m, k, n, 0, 0, 1), (counts, m, k, n, split, slots.value)
+        if lists is not None:
+            with_lists += 1
+            assert max(lists, common) <= launched(G, m, k, n, 0, 1, 0), (counts, m, n, lists, slots.value)
+        fullest = max(fullest, common / got)
+    assert with_lists > 300 and fullest > 0.95           # the lists were met, and the bound is nearly reached
     assert lib.ms_gmm_launch_slots(0, 1, 1, 1, 0, 0, 0, ctypes.byref(slots)) != 0
     assert lib.ms_gmm_launch_slots(8, 1, 1, 1, 1, 0, 0, ctypes.byref(slots)) != 0
