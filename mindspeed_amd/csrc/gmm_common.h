@@ -196,7 +196,7 @@ __device__ __forceinline__ f32x16 mfma16(v16 a, v16 b, f32x16 c) {
 // inside the K loop (up to 500 copies per step of 128 products, and spills).  The compiler therefore does not know that
 // this is a matrix instruction: a caller must leave two instructions between an ordinary vector write of an operand and
 // this (operands that come from LDS reads are covered by the wait the compiler inserts), and wait out the last results
-// with s_nop before ordinary instructions read them.
+// with s_nop before ordinary instructions read them (ready and settle of the K loops).
 template <int DT>
 __device__ __forceinline__ void mfma16x16(v16 a, v16 b, f32x4 &acc) {
     if constexpr (DT == MS_BF16) asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));

@@ -306,18 +306,29 @@ __device__ __forceinline__ const char *uniform(const char *p) {
     return reinterpret_cast<const char *>(lo | hi << 32);
 }
 
+// The accumulators are in their registers at this point of the program, whatever was or will be done with them.
+template <int TM, int TN>
+__device__ __forceinline__ void pin(f32x4 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
+}
+
+// Between the clearing of the accumulators and the first mfma16x16 on them: the two instructions that it has to be away
+// from an ordinary write of its operands (tests/test_matrix_instruction_hazards.py reads the built code for it).
+template <int TM, int TN>
+__device__ __forceinline__ void ready(f32x4 (&acc)[TM][TN]) {
+    pin(acc);
+    asm volatile("s_nop 1" ::: "memory");
+}
+
 // The last matrix instructions must have written their results before ordinary instructions read them (16 passes at most).
 template <int TM, int TN>
 __device__ __forceinline__ void settle(f32x4 (&acc)[TM][TN]) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
+    pin(acc);
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
+    pin(acc);
 }
 
 // K loop of a 256 x 256 tile: 2 x 2 wavefronts of 128 x 128 = 8 x 8 blocks of 16 x 16, K steps of 64 = two 32-wide
@@ -410,6 +421,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
         bf[0][t] = lb.frag(b_cur, 0, t);
         af[0][t] = la.frag(a_cur, 0, t);
     }
+    ready(acc);
     __builtin_amdgcn_sched_barrier(0);
 
     auto k_step = [&](auto tail_c) {
@@ -536,6 +548,7 @@ __device__ __forceinline__ void dma_small_k_loop(const GmmArgs &p, const TileCoo
     MS_TRACE(3);
 #pragma unroll
     for (int f = 0; f < NF; ++f) read_frag(0, 0, f);
+    ready(acc);
     __builtin_amdgcn_sched_barrier(0);
 
     auto k_step = [&](auto tail_c) {
