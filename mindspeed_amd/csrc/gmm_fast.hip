@@ -315,6 +315,19 @@ __device__ __forceinline__ void pin(f32x4 (&acc)[TM][TN]) {
         for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
+// Clears the accumulators, at this point of the program and no earlier: the 256 clearing instructions of a wavefront take
+// half a microsecond, which the way of the first tiles hides once these are requested.  (Cleared ahead of the requests:
+// training layers of 8 experts x 4096 x 14336 with 64 rows each 2214 us instead of 2187, with 256 rows each and a width of
+// 7168 1728 instead of 1707.)
+template <int TM, int TN>
+__device__ __forceinline__ void clear(f32x4 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    pin(acc);
+}
+
 // Between the clearing of the accumulators and the first mfma16x16 on them: the two instructions that it has to be away
 // from an ordinary write of its operands (tests/test_matrix_instruction_hazards.py reads the built code for it).
 template <int TM, int TN>
@@ -347,7 +360,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     const int red_begin = tc.e.red_begin;
     const int red_len = tc.e.red_end - red_begin;
     const int nk = (red_len + BK - 1) / BK;
-    if (nk <= 0) return;
+    if (nk <= 0) return clear(acc);
 
     DmaOperand<A_RED> la;
     DmaOperand<B_RED> lb;
@@ -366,8 +379,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     const int64_t b_step = p.b_stride_red * BK * 2;
     const char *zeros = reinterpret_cast<const char *>((reinterpret_cast<uintptr_t>(p.table->zeros) + 15) & ~uintptr_t(15));
 
-    // LDS: A stages 0, 1, then B stages 0, 1, 2.  Requests run on past the last tile (all-zero tiles that nobody
-    // multiplies): the number of transfers in flight is then the same at every step and one wait count serves all.
+    // LDS: A stages 0, 1, then B stages 0, 1, 2.
     const unsigned lds_a = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr)lds)) + wave * (kXfers * 1024);
     const unsigned lds_b = lds_a + kAStages * kStageTile;
     int a_left = red_len, b_left = red_len;     // reduction indices from the next requested tile's start to the end
@@ -403,7 +415,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     };
 
     // tiles 0 and 1 of both operands (the order of the steady state: B before A)
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < nk && t < 2; ++t) {
 #pragma unroll
         for (int i = 0; i < kXfers; ++i) request_b(std::true_type{}, i);
         next_b();
@@ -411,7 +423,9 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
         for (int i = 0; i < kXfers; ++i) request_a(std::true_type{}, i);
         next_a();
     }
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * kXfers, 0));
+    clear(acc);
+    if (nk > 1) __builtin_amdgcn_s_waitcnt(waitcnt_imm(2 * kXfers, 0));
+    else __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
     __builtin_amdgcn_s_barrier();
     MS_TRACE(3);
     const char *a_cur = lds;                                   // stages of tile kt
@@ -424,7 +438,15 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     ready(acc);
     __builtin_amdgcn_sched_barrier(0);
 
-    auto k_step = [&](auto tail_c) {
+    // WHOLE, TAIL: tile kt + 2 is requested, all of it inside the range or not; DRAIN (kt = nk - 2): there is none; LAST: nor
+    // a tile to read after this one.  (Two all-zero tiles of each operand requested behind every range, so that one wait
+    // count served every step, are as long as a loop of two steps: a training layer of 8 experts x 4096 x 14336 with 64
+    // rows each took 2248 us with them, 2214 without; 222 rows each, 4672 x 5160: 1505 and 1487.)
+    enum { WHOLE, TAIL, DRAIN, LAST };
+    auto k_step = [&](auto kind_c) {
+        constexpr int kind = decltype(kind_c)::value;
+        constexpr std::bool_constant<kind == TAIL> tail_c{};
+        constexpr bool ask = kind == WHOLE || kind == TAIL;
         // slice 0; B's tile kt + 2 is requested
 #pragma unroll
         for (int u = 0; u < 64; ++u) {
@@ -434,34 +456,45 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
                 if (f < 8) bf[1][f] = lb.frag(b_cur, 1, f);
                 else af[1][f - 8] = la.frag(a_cur, 1, f - 8);
             }
-            if (u % 8 == 5) request_b(tail_c, u / 8);
+            if constexpr (ask) {
+                if (u % 8 == 5) request_b(tail_c, u / 8);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
-        next_b();
-        a_cur = a_cur == lds ? lds + kStageTile : lds;
-        b_cur = b_cur == lds + (kAStages + kBStages - 1) * kStageTile ? lds + kAStages * kStageTile : b_cur + kStageTile;
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(kXfers, 0));
-        __builtin_amdgcn_s_barrier();
+        if constexpr (ask) next_b();
+        if constexpr (kind != LAST) {
+            a_cur = a_cur == lds ? lds + kStageTile : lds;
+            b_cur = b_cur == lds + (kAStages + kBStages - 1) * kStageTile ? lds + kAStages * kStageTile : b_cur + kStageTile;
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(ask ? kXfers : 0, 0));
+            __builtin_amdgcn_s_barrier();
+        }
         // slice 1; A's tile kt + 2 is requested, slice 0 of tile kt + 1 is read
 #pragma unroll
         for (int u = 0; u < 64; ++u) {
             mfma(1, u);
-            if (u % 2 == 0 && u < 32) {
-                const int f = u / 2;
-                if (f < 8) bf[0][f] = lb.frag(b_cur, 0, f);
-                else af[0][f - 8] = la.frag(a_cur, 0, f - 8);
+            if constexpr (kind != LAST) {
+                if (u % 2 == 0 && u < 32) {
+                    const int f = u / 2;
+                    if (f < 8) bf[0][f] = lb.frag(b_cur, 0, f);
+                    else af[0][f - 8] = la.frag(a_cur, 0, f - 8);
+                }
             }
-            if (u % 8 == 1) request_a(tail_c, u / 8);
+            if constexpr (ask) {
+                if (u % 8 == 1) request_a(tail_c, u / 8);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
-        next_a();
+        if constexpr (ask) next_a();
     };
     int kt = 0;
     const int nk_full = red_len / BK - 2;       // steps whose requests are whole tiles inside the range
-    for (; kt < nk_full; ++kt) k_step(std::false_type{});
-    for (; kt < nk; ++kt) k_step(std::true_type{});
-    // the transfers of the trailing all-zero tiles must have landed before the stages are reused
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+    for (; kt < nk_full; ++kt) k_step(std::integral_constant<int, WHOLE>{});
+    if (kt + 2 < nk) {
+        k_step(std::integral_constant<int, TAIL>{});
+        ++kt;
+    }
+    if (kt + 1 < nk) k_step(std::integral_constant<int, DRAIN>{});
+    k_step(std::integral_constant<int, LAST>{});      // (no transfer is under way any more: the stages can be reused)
     settle(acc);
 }
 
@@ -489,7 +522,7 @@ __device__ __forceinline__ void dma_small_k_loop(const GmmArgs &p, const TileCoo
     const int red_begin = tc.e.red_begin;
     const int red_len = tc.e.red_end - red_begin;
     const int nk = (red_len + BK - 1) / BK;
-    if (nk <= 0) return;
+    if (nk <= 0) return clear(acc);
 
     OpA la;
     OpB lb;
@@ -543,6 +576,7 @@ __device__ __forceinline__ void dma_small_k_loop(const GmmArgs &p, const TileCoo
         for (int i = 0; i < NXFER; ++i) request(std::true_type{}, i);
         next_tile();
     }
+    clear(acc);
     __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 1) * NXFER, 0));
     __builtin_amdgcn_s_barrier();
     MS_TRACE(3);
@@ -631,10 +665,6 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     std::conditional_t<DMA, Acc16<2 * TM, 2 * TN>, Acc32<TM, TN>> sums;
     auto &acc = sums.v;
     if constexpr (DMA) {
-#pragma unroll
-        for (int i = 0; i < 2 * TM; ++i)
-#pragma unroll
-            for (int j = 0; j < 2 * TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         if constexpr (TBM == 256) dma_k_loop<DT, A_RED, B_RED, SWIGLU>(p, tc, lds, row0, col0, acc);
         else dma_small_k_loop<DT, B_RED, SWIGLU, TBM>(p, tc, lds, row0, col0, acc);
     } else {

@@ -541,3 +541,48 @@ def test_small_tiles_over_reduction_lengths(K, dtype, device):
     scaled = wd * 0.0625                                  # gate values of the size an activation meets
     act = ops.fused_swiglu(ops.npu_gmm_v2(xd, scaled, group_list=cd, group_type=0))
     assert torch.equal(ops.gmm_swiglu(xd, scaled, cd), act)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_large_tiles_over_reduction_lengths_beside_bad_rows(bad, dtype, device):
+    """256-row tiles whose reduction takes no step, one, two, three and more, ending inside a step or with it; every other
+    group (and what lies past the last offset) holds NaN or infinities, which must stay out of the groups beside it.  Small
+    integers: forward, dX, dW, its fp32 form and `+=` are exact."""
+    say("large tiles", bad, dtype)
+    gen = torch.Generator().manual_seed(17)
+    ints = lambda *s: torch.randint(-1, 2, s, generator=gen).double()
+    put = lambda t: t.to(dtype).to(device)
+    # split on the reduction dim: the groups' lengths are the reductions; outputs of one whole tile and a part of another
+    lengths = torch.tensor([0, 5, 1, 9, 63, 1, 64, 70, 65, 3, 127, 64, 128, 65, 129, 2, 191, 7, 192, 1, 193, 64, 256, 30, 257, 33])
+    K, N, M = 264, 520, int(lengths.sum()) + 40
+    ends = torch.cumsum(lengths, 0)
+    x, g = ints(M, K), ints(M, N)
+    x[ends[-1]:], g[ends[-1]:] = bad, bad
+    exp = torch.zeros(lengths.numel(), K, N).double()
+    for e, (end, n) in enumerate(zip(ends.tolist(), lengths.tolist())):
+        if e % 2:
+            x[end - n:end], g[end - n:end] = bad, bad
+        else:
+            exp[e] = x[end - n:end].t() @ g[end - n:end]
+    xd, gd, start = put(x), put(g), ints(*exp.shape)
+    for n in (lengths.numel(), 13):                       # with whole groups dealt out to single XCDs, and without
+        dw = ops.npu_gmm_v2(xd.t(), gd, group_list=lengths[:n].to(device), group_type=2)
+        assert torch.equal(dw[::2].cpu().double(), exp[:n:2])
+        acc = start[:n].float().to(device)
+        ops.npu_groupmatmul_add_fp32(xd, gd, ends[:n].to(device), acc)
+        assert torch.equal(acc[::2].cpu().double(), (start + exp)[:n:2])
+    # split on rows: K is the reduction, in both weight layouts
+    counts = torch.tensor([256, 3, 300, 200, 512, 70])
+    M, N = int(counts.sum()), 264
+    for K in (8, 56, 64, 72, 128, 136, 192, 200, 256, 264):
+        say("large tiles rows", K)
+        x, w = ints(M, K), ints(counts.numel(), K, N)
+        exp = torch.cat([xs @ w[e] for e, xs in enumerate(x.split(counts.tolist()))])
+        keep = torch.repeat_interleave(torch.arange(counts.numel()) % 2 == 0, counts)
+        x[~keep], w[1::2] = bad, bad
+        xd, wd = put(x), put(w)
+        wt = put(w.transpose(1, 2).contiguous()).transpose(1, 2)
+        for weight in (wd, wt):
+            y = ops.npu_gmm_v2(xd, weight, group_list=counts.to(device), group_type=0).cpu().double()
+            assert torch.equal(y[keep], exp[keep])
