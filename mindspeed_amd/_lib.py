@@ -15,7 +15,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # MINDSPEED_AMD_LIB names another build of the same library (to compare two builds on one machine)
 LIB_PATH = os.environ.get("MINDSPEED_AMD_LIB") or os.path.join(_HERE, "libmindspeed_amd.so")
 
-ABI_VERSION = 103                # what ms_version() of a matching build returns (argument lists below)
+ABI_VERSION = 104                # what ms_version() of a matching build returns (argument lists below)
 MS_BF16, MS_FP16, MS_FP32 = 0, 1, 2
 MS_INT32, MS_INT64 = 0, 1
 MS_MAX_EXPERTS = 1024

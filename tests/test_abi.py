@@ -2,9 +2,13 @@
 host-side argument validation works without a GPU (no compute calls here)."""
 import ctypes
 import glob
+import hashlib
 import os
 import random
 import re
+import shutil
+import subprocess
+import sys
 
 import pytest
 
@@ -31,6 +35,22 @@ def test_library_exports_every_declared_symbol():
     for name in sorted(declared_symbols()):
         assert hasattr(lib, name), name
     assert lib.ms_version() == _lib.ABI_VERSION
+
+
+def test_the_version_moves_with_the_entry_points(tmp_path):
+    """The names that a version stands for, and what a build of the version before says when it is loaded: that it has to
+    be built again (and not which symbol it lacks)."""
+    names = " ".join(sorted(declared_symbols()))
+    assert (_lib.ABI_VERSION, hashlib.sha256(names.encode()).hexdigest()[:16]) == (104, "357be616bd29ac47")
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    stale = tmp_path / "stale.so"
+    subprocess.run([cc, "-shared", "-fPIC", "-x", "c", "-", "-o", str(stale)], input=f"int ms_version(void) {{ return {_lib.ABI_VERSION - 1}; }}",
+                   text=True, check=True)
+    res = subprocess.run([sys.executable, "-c", "from mindspeed_amd import _lib; _lib.load()"], capture_output=True, text=True,
+                         cwd=ROOT, env=dict(os.environ, MINDSPEED_AMD_LIB=str(stale)))
+    assert res.returncode != 0 and "rebuild it" in res.stderr and "undefined symbol" not in res.stderr
 
 
 def test_workspace_size_and_validation_are_host_only():
