@@ -24,7 +24,8 @@
 //     global loads stay fully coalesced (32 lanes x 16 bytes per memory row).
 //
 // The small tail tiles of a RED A run the same way with more stages (dma_small_k_loop below).  Those of an
-// A of the other kind (the weight gradient) keep 32x32x16 and a register-staged K loop:
+// A of the other kind (the weight gradient of a width that is no multiple of 256) keep 32x32x16 and a register-staged K loop
+// (the transfers' swizzle is made for 512-byte rows; whether one for shorter rows would pay there was not measured):
 //   registers hold tile kt+1 (loaded one K step ago), LDS stage `cur` holds tile kt.
 //   step kt, phase p = 0..3 (one 16-wide slice of the 64-wide K step each):
 //       store part p of tile kt+1 from registers to LDS stage `nxt`
@@ -64,12 +65,9 @@ __device__ __forceinline__ void sg() {
     if constexpr (N > 0) __builtin_amdgcn_sched_group_barrier(MASK, N, ID);
 }
 
-// Bytes of one operand tile in LDS.  RED: [ROWS outer][64 reduction] x 2 bytes.  !RED: [64 reduction][ROWS outer]
-// x 2 bytes with 64 bytes of padding per row (pitch mod 256 == 64 keeps the transposing reads conflict-free).
-template <bool RED, int ROWS>
-constexpr int tile_bytes() { return RED ? ROWS * 128 : 64 * (ROWS * 2 + 64); }
-constexpr int kRedTileBytes = tile_bytes<true, 256>();
-constexpr int kOuterTileBytes = tile_bytes<false, 256>();
+// Bytes of one register-staged operand tile in LDS: [64 reduction][ROWS outer] x 2 bytes with 64 bytes of padding per row.
+template <int ROWS>
+constexpr int tile_bytes() { return 64 * (ROWS * 2 + 64); }
 
 constexpr int kStagePitch = 272;                          // epilogue staging: 128 x 2 bytes + 16 bytes pad
 constexpr int kStagePerWave = 128 * kStagePitch;          // one 128 x 128 16-bit block per wavefront
@@ -83,56 +81,40 @@ __device__ __forceinline__ uint2 lds_read_tr(const char *p) {
     return __builtin_bit_cast(uint2, v);
 }
 
-// One operand of the macro tile (ROWS outer indices x 64 reduction indices):
-// global -> registers -> LDS, and LDS -> MFMA fragments.
-template <bool RED, int ROWS>
+// One operand of a small tile of the weight gradient (ROWS outer indices x 64 reduction indices, contiguous along the
+// outer dim): global -> registers -> LDS, and LDS -> MFMA fragments.
+template <int ROWS>
 struct Operand {
     static constexpr int NL = ROWS / 32;          // 16-byte loads per lane per K step (8, 4 or 2)
-    static constexpr int PITCH = ROWS * 2 + 64;   // !RED: bytes per reduction row in LDS
-    static constexpr int CP = ROWS / 8;           // !RED: 16-byte chunks per reduction row
-    static constexpr int RP = 256 / CP;           // !RED: reduction rows covered by one load of the workgroup
+    static constexpr int PITCH = ROWS * 2 + 64;   // bytes per reduction row in LDS
+    static constexpr int CP = ROWS / 8;           // 16-byte chunks per reduction row
+    static constexpr int RP = 256 / CP;           // reduction rows covered by one load of the workgroup
     unsigned off[NL];   // per-lane global byte offsets of the loads, relative to the tile's base pointer
-    unsigned off0;      // !RED: offset of (reduction index 0, this lane's outer chunk), always valid
+    unsigned off0;      // offset of (reduction index 0, this lane's outer chunk), always valid
     unsigned st_off;    // byte offset of this lane's first LDS store inside the tile
     unsigned frag_off;  // byte offset of this lane's fragment reads inside the tile
     v16 r[NL];
 
-    // outer0: first outer index of the tile; outer_last: clamp bound (RED: last valid outer index,
-    // !RED: last valid start of an 8-wide chunk); wave_outer: this wavefront's first outer index in the tile.
-    __device__ __forceinline__ void init(int64_t stride_outer, int64_t stride_red, int outer0, int outer_last,
-                                         int wave_outer) {
+    // outer0: first outer index of the tile; outer_last: last valid start of an 8-wide chunk; wave_outer: this wavefront's
+    // first outer index in the tile.
+    __device__ __forceinline__ void init(int64_t stride_red, int outer0, int outer_last, int wave_outer) {
         const int tid = threadIdx.x;
         const int lane = tid & 63;
-        if constexpr (RED) {
-            const int ck = tid & 7;
-            const int row = tid >> 3;
+        const int chunk = tid % CP;   // 16-byte chunk along the outer dim
+        const int rrow = tid / CP;    // reduction row within one load of the workgroup
+        int outer = outer0 + chunk * 8;
+        outer = outer > outer_last ? outer_last : outer;
 #pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                int outer = outer0 + row + 32 * i;
-                outer = outer > outer_last ? outer_last : outer;
-                off[i] = static_cast<unsigned>((static_cast<int64_t>(outer - outer0) * stride_outer + ck * 8) * 2);
-            }
-            off0 = 0;
-            st_off = row * 128 + ((ck ^ swz(row)) << 4);
-            const int frow = lane & 31;
-            frag_off = (wave_outer + frow) * 128 + (((lane >> 5) ^ swz(frow)) << 4);
-        } else {
-            const int chunk = tid % CP;   // 16-byte chunk along the outer dim
-            const int rrow = tid / CP;    // reduction row within one load of the workgroup
-            int outer = outer0 + chunk * 8;
-            outer = outer > outer_last ? outer_last : outer;
-#pragma unroll
-            for (int i = 0; i < NL; ++i)
-                off[i] = static_cast<unsigned>((static_cast<int64_t>(i * RP + rrow) * stride_red + (outer - outer0)) * 2);
-            off0 = static_cast<unsigned>((outer - outer0) * 2);
-            st_off = rrow * PITCH + chunk * 16;
-            // transposing read: in each group of 16 lanes, lane L supplies the 4-element segment at
-            // (reduction L/4, outer 4*(L%4)) and receives reduction 0..3 of outer L.
-            const int l16 = lane & 15;
-            const int red = 8 * (lane >> 5) + (l16 >> 2);
-            const int out = wave_outer + 16 * ((lane >> 4) & 1) + 4 * (l16 & 3);
-            frag_off = red * PITCH + out * 2;
-        }
+        for (int i = 0; i < NL; ++i)
+            off[i] = static_cast<unsigned>((static_cast<int64_t>(i * RP + rrow) * stride_red + (outer - outer0)) * 2);
+        off0 = static_cast<unsigned>((outer - outer0) * 2);
+        st_off = rrow * PITCH + chunk * 16;
+        // transposing read: in each group of 16 lanes, lane L supplies the 4-element segment at
+        // (reduction L/4, outer 4*(L%4)) and receives reduction 0..3 of outer L.
+        const int l16 = lane & 15;
+        const int red = 8 * (lane >> 5) + (l16 >> 2);
+        const int out = wave_outer + 16 * ((lane >> 4) & 1) + 4 * (l16 & 3);
+        frag_off = red * PITCH + out * 2;
     }
 
     // base: pointer to element (outer0, red0) of the tile.  Loads i = h*NL/2 .. (h+1)*NL/2 - 1 of this lane.
@@ -145,12 +127,9 @@ struct Operand {
             if constexpr (!TAIL) {
                 r[i] = *reinterpret_cast<const v16 *>(base + off[i]);
             } else {
-                // RED: one chunk of 8 reduction indices per lane (whole or nothing: the reduction extent is a
-                // multiple of 8 on this path); !RED: one reduction index per load.  Masked-out lanes read a
-                // valid address (chunk 0 / reduction index 0) instead.
-                const int q = tid & 7;
-                const bool ok = RED ? (q * 8 < nvalid) : (i * RP + tid / CP < nvalid);
-                const unsigned o = ok ? off[i] : (RED ? off[i] - q * 16 : off0);
+                // one reduction index per load; masked-out lanes read a valid address (reduction index 0) instead
+                const bool ok = i * RP + tid / CP < nvalid;
+                const unsigned o = ok ? off[i] : off0;
                 const v16 v = *reinterpret_cast<const v16 *>(base + o);
                 const v16 z = {0u, 0u, 0u, 0u};
                 r[i] = ok ? v : z;
@@ -160,23 +139,16 @@ struct Operand {
 
     __device__ __forceinline__ void store_half(char *tile, int h) const {
 #pragma unroll
-        for (int i = h * (NL / 2); i < (h + 1) * (NL / 2); ++i) {
-            if constexpr (RED) *reinterpret_cast<v16 *>(tile + st_off + i * 32 * 128) = r[i];
-            else *reinterpret_cast<v16 *>(tile + st_off + i * RP * PITCH) = r[i];
-        }
+        for (int i = h * (NL / 2); i < (h + 1) * (NL / 2); ++i) *reinterpret_cast<v16 *>(tile + st_off + i * RP * PITCH) = r[i];
     }
 
     // Fragment t (32 outer indices) of K slice kk (16 reduction indices): 8 consecutive reduction values
     // of outer index (lane & 31), reduction half (lane >> 5).
     __device__ __forceinline__ v16 frag(const char *tile, int kk, int t) const {
-        if constexpr (RED) {
-            return *reinterpret_cast<const v16 *>(tile + (frag_off ^ ((kk * 2) << 4)) + t * 32 * 128);
-        } else {
-            const char *p = tile + frag_off + kk * 16 * PITCH + t * 64;
-            const uint2 lo = lds_read_tr(p);
-            const uint2 hi = lds_read_tr(p + 4 * PITCH);
-            return v16{lo.x, lo.y, hi.x, hi.y};
-        }
+        const char *p = tile + frag_off + kk * 16 * PITCH + t * 64;
+        const uint2 lo = lds_read_tr(p);
+        const uint2 hi = lds_read_tr(p + 4 * PITCH);
+        return v16{lo.x, lo.y, hi.x, hi.y};
     }
 };
 
@@ -202,7 +174,9 @@ __device__ __forceinline__ void interleave(std::integer_sequence<int, G...>) {
 //   !RED operand: [64 reduction][256 outer], 512-byte rows, chunk c of row r holds memory chunk
 //                 c ^ ((r & 3) << 2) ^ (((r >> 3) & 1) << 1)
 // (the first keeps 8 consecutive rows of one chunk column on 8 different bank groups for ds_read_b128, the second the
-// rows of one ds_read_b64_tr_b16 on different 32-byte bank groups).
+// rows of one ds_read_b64_tr_b16 on different 32-byte bank groups).  Whole kernels still count conflicts: 0.09 (forward),
+// 0.07 (dX) and 0.3 (dW, both operands of the second kind) conflict clocks per clock of LDS instructions (Mixtral shape),
+// of fragment reads, incoming transfers and staged epilogue together; which of them was not taken apart.
 constexpr int kStageTile = 256 * BK * 2;      // bytes of one operand in one stage (32 KB)
 constexpr int kAStages = 2, kBStages = 3;     // 5 x 32 KB: the compute unit's whole 160 KB
 constexpr int kDmaBytes = (kAStages + kBStages) * kStageTile;
@@ -645,8 +619,9 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     constexpr int WAVES_N = 4 / WAVES_M;
     constexpr int TM = TBM / WAVES_M / 32;      // 32-row MFMA blocks per wavefront
     constexpr int TN = BN / WAVES_N / 32;       // 32-column MFMA blocks per wavefront
-    constexpr int A_BYTES = tile_bytes<A_RED, TBM>();            // small tiles only: two register-staged stages
-    constexpr int STAGE = A_BYTES + tile_bytes<B_RED, BN>();
+    constexpr int A_BYTES = tile_bytes<TBM>();  // small tiles of the weight gradient only: two register-staged stages
+    constexpr int STAGE = A_BYTES + tile_bytes<BN>();
+    static_assert(A_RED || !B_RED, "the split on the reduction dim takes both operands along their outer dims");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -674,10 +649,10 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
             for (int j = 0; j < TN; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-        Operand<A_RED, TBM> la;
-        Operand<B_RED, BN> lb;
-        la.init(p.a_stride_row, p.a_stride_red, row0, A_RED ? row_end - 1 : row_end - 8, wm * TM * 32);
-        lb.init(p.b_stride_col, p.b_stride_red, col0, B_RED ? col_end - 1 : col_end - 8, wn * TN * 32);
+        Operand<TBM> la;
+        Operand<BN> lb;
+        la.init(p.a_stride_red, row0, row_end - 8, wm * TM * 32);
+        lb.init(p.b_stride_red, col0, col_end - 8, wn * TN * 32);
         // uniform base pointers of element (outer0, red_begin); advanced by one K step per iteration
         const char *a_ptr = static_cast<const char *>(p.a) +
                             (static_cast<int64_t>(row0) * p.a_stride_row + static_cast<int64_t>(red_begin) * p.a_stride_red) * 2;
@@ -739,9 +714,9 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 
         // instruction counts of one phase (one 16-wide K slice)
         constexpr int NM = TM * TN;                                        // MFMAs
-        constexpr int NRD = (A_RED ? TM : 2 * TM) + (B_RED ? TN : 2 * TN); // LDS fragment reads
-        constexpr int NLA = Operand<A_RED, TBM>::NL / 2;                   // loads / stores of an A part
-        constexpr int NLB = Operand<B_RED, BN>::NL / 2;                    // ... of a B part
+        constexpr int NRD = 2 * TM + 2 * TN;                               // LDS fragment reads
+        constexpr int NLA = Operand<TBM>::NL / 2;                          // loads / stores of an A part
+        constexpr int NLB = Operand<BN>::NL / 2;                           // ... of a B part
 
         int kt = 0;
         // HAS1: tile kt+1 exists (it is in registers); HAS2: tile kt+2 exists; tail2_c: tile kt+2 is the last one.
@@ -797,8 +772,8 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     const int64_t ldc = p.c_stride_row;
     constexpr int WR = TM * 32, WC = TN * 32;       // this wavefront's block of the tile
     if constexpr (OUT == OUT_SAME || OUT == OUT_SWIGLU || OUT == OUT_SWIGLU_GRAD) {
-        // 16-bit output: each wavefront stages its block in its own LDS region (row pitch WC*2 + 16 bytes:
-        // conflict-free for the 8-byte column-slice writes of 16 x 16 blocks and the row reads) and writes it out as
+        // 16-bit output: each wavefront stages its block in its own LDS region (row pitch WC*2 + 16 bytes, so that the
+        // 8-byte column-slice writes of a 16 x 16 block start on different banks in all its rows) and writes it out as
         // 16 bytes per lane, WC*2 contiguous bytes per row.
         constexpr int SP = WC * 2 + 16;
         static_assert(WR * SP <= kStagePerWave, "staging region too small");
@@ -1002,6 +977,7 @@ __global__ __launch_bounds__(256) void gmm16_fast_kernel(const GmmArgs p) {
 template <int DT, int OUT>
 int launch_fast(hipStream_t stream, const GmmArgs &args, bool a_red, bool b_red, unsigned grid, bool lists) {
     const void *fn;
+    MS_REQUIRE(a_red || !b_red, MS_ERR_UNSUPPORTED, "ms_gmm: operand layout not supported");   // (the caller keeps it off this path)
     if constexpr (OUT == OUT_SWIGLU) {
         MS_REQUIRE(a_red && !b_red, MS_ERR_UNSUPPORTED, "ms_gmm_swiglu: operand layout not supported");
         fn = reinterpret_cast<const void *>(&gmm16_fast_kernel<DT, true, false, OUT>);
@@ -1010,11 +986,10 @@ int launch_fast(hipStream_t stream, const GmmArgs &args, bool a_red, bool b_red,
         fn = reinterpret_cast<const void *>(&gmm16_fast_kernel<DT, true, true, OUT>);
     } else if (a_red && b_red) fn = reinterpret_cast<const void *>(&gmm16_fast_kernel<DT, true, true, OUT>);
     else if (a_red) fn = reinterpret_cast<const void *>(&gmm16_fast_kernel<DT, true, false, OUT>);
-    else if (b_red) fn = reinterpret_cast<const void *>(&gmm16_fast_kernel<DT, false, true, OUT>);
     else if (lists) fn = reinterpret_cast<const void *>(&gmm16_fast_kernel<DT, false, false, OUT, true>);
     else fn = reinterpret_cast<const void *>(&gmm16_fast_kernel<DT, false, false, OUT>);
     constexpr int lds_bytes = kDmaBytes;      // covers the small tiles' two stages and the epilogue's staging as well
-    static_assert(kDmaBytes >= 4 * kOuterTileBytes && kDmaBytes >= 4 * kRedTileBytes && kDmaBytes >= kStageBytes,
+    static_assert(kDmaBytes >= 2 * (tile_bytes<128>() + tile_bytes<BN>()) && kDmaBytes >= kStageBytes,
                   "the K loop's LDS must hold every other use of it");
     hipError_t e = set_max_dynamic_lds(fn, lds_bytes);
     MS_REQUIRE(e == hipSuccess, MS_ERR_HIP, "ms_gmm: hipFuncSetAttribute: %s", hipGetErrorString(e));
