@@ -11,6 +11,7 @@ from conftest import rel_l2
 from oracle import moe_oracle as O
 
 import mindspeed_amd.ops as ops
+from mindspeed_amd import _lib
 from mindspeed_amd.dispatcher import dispatch_mlp_combine
 
 pytestmark = pytest.mark.gpu
@@ -46,6 +47,13 @@ def test_swiglu(rows, ffn, dtype, device):
     assert rel_l2(xd2.grad, ex2) <= tol and rel_l2(pd.grad, ep2) <= tol
 
 
+def poison(x, p, device):
+    """Blocks of the sizes that the outputs are about to take, left full of NaN in the allocator: it hands out freed blocks of
+    the same size first, and keeps small and large ones apart."""
+    held = [torch.full_like(t, float("nan"), device=device) for t in (x, p) for _ in range(4)]
+    del held
+
+
 @pytest.mark.parametrize("nchunks,rows,hidden", [(16, 2048, 256), (32, 4096, 128), (5, 77, 10)])
 def test_sort_chunks(nchunks, rows, hidden, device):
     say("sort_chunks", nchunks, rows, hidden)
@@ -79,8 +87,7 @@ def test_sort_chunks_partial_map_on_the_device(device):
     rows, hidden = 1000, 64
     x = torch.randn(rows, hidden, generator=gen)
     p = torch.rand(rows, generator=gen)
-    poison = torch.full((1 << 22,), float("nan"), device=device)       # whatever the allocator hands out next is NaN
-    del poison
+    poison(x, p, device)
     # 1. the sizes cover 900 of the 1000 rows
     sizes = torch.tensor([300, 100, 500]); order = torch.tensor([2, 0, 1])
     xd = x.to(device).requires_grad_(True)
@@ -89,16 +96,20 @@ def test_sort_chunks_partial_map_on_the_device(device):
     assert torch.equal(out.cpu(), want)
     assert torch.equal(outp.cpu(), torch.cat([p[400:900], p[0:300], p[300:400], torch.zeros(100)]))
     g = torch.randn(rows, hidden, generator=gen)
-    out.backward(g.to(device))
+    gd = g.to(device)
+    poison(x, p, device)
+    out.backward(gd)
     exp_g = torch.zeros(rows, hidden)
     exp_g[400:900], exp_g[0:300], exp_g[300:400] = g[0:500], g[500:800], g[800:900]
     assert torch.equal(xd.grad.cpu(), exp_g)
     # 2. chunk 0 named twice, chunk 1 never: 600 output rows are written, the input rows of chunk 1 get no gradient
     sizes = torch.tensor([300, 700]); order = torch.tensor([0, 0])
     xd = x.to(device).requires_grad_(True)
+    poison(x, p, device)
     out, _ = ops.sort_chunks_by_idxs(xd, sizes.to(device), order.to(device))
     assert torch.equal(out.cpu(), torch.cat([x[0:300], x[0:300], torch.zeros(400, hidden)]))
-    out.backward(g.to(device))
+    poison(x, p, device)
+    out.backward(gd)
     got = xd.grad.cpu()
     assert not torch.isnan(got).any() and torch.equal(got[300:], torch.zeros(700, hidden))
 
@@ -118,12 +129,42 @@ def test_sort_chunks_rows_left_out_are_zeros(hidden, dtype, pdt, device):
     exp, exp_p, exp_g, exp_gp = (torch.zeros_like(t) for t in (x, p, x, p))
     exp[:200], exp_p[:200], exp_g[source], exp_gp[source] = x[source], p[source], g[:200], gp[:200]
     xd, pd = x.to(device).requires_grad_(True), p.to(device).requires_grad_(True)
-    poison = torch.full((1 << 22,), float("nan"), device=device)
-    del poison
-    out, out_p = ops.sort_chunks_by_idxs(xd, sizes.to(device), order.to(device), pd)
+    sd, od, gd, gpd = sizes.to(device), order.to(device), g.to(device), gp.to(device)
+    poison(x, p, device)
+    out, out_p = ops.sort_chunks_by_idxs(xd, sd, od, pd)
     assert torch.equal(out.detach().cpu(), exp) and torch.equal(out_p.detach().cpu(), exp_p)
-    gx, gprobs = torch.autograd.grad((out, out_p), (xd, pd), (g.to(device), gp.to(device)))
+    poison(x, p, device)
+    gx, gprobs = torch.autograd.grad((out, out_p), (xd, pd), (gd, gpd))
     assert torch.equal(gx.cpu(), exp_g) and torch.equal(gprobs.cpu(), exp_gp)
+    # the entry points themselves, on outputs that hold NaN: every element is written
+    lib = _lib.load()
+    ptr = lambda t: t.data_ptr()
+    code, pcode = _lib.dtype_code(dtype, "x"), _lib.dtype_code(pdt, "p")
+    stream = _lib.stream_ptr(xd.device)
+    bad = lambda t: torch.full_like(t, float("nan"))
+    out, out_p, gx, gprobs = bad(xd.detach()), bad(pd.detach()), bad(gd), bad(gpd)
+    inverse = torch.full((rows,), 12345, dtype=torch.int32, device=device)
+    _lib.check(lib.ms_sort_chunks_inverse(stream, ptr(xd), ptr(sd), ptr(od), 4, rows, hidden, code, ptr(pd), pcode, ptr(out),
+                                          ptr(out_p), ptr(inverse)), "ms_sort_chunks_inverse")
+    _lib.check(lib.ms_gather_rows_zero(stream, ptr(gd), ptr(inverse), rows, hidden, code, ptr(gx), ptr(gpd), pcode, ptr(gprobs)),
+               "ms_gather_rows_zero")
+    for got, want in ((out, exp), (out_p, exp_p), (gx, exp_g), (gprobs, exp_gp)):
+        assert torch.equal(got.cpu(), want)
+    want = torch.full((rows,), -1, dtype=torch.int32)
+    want[source] = torch.arange(200, dtype=torch.int32)
+    assert torch.equal(inverse.cpu(), want)
+    # and the form with the map from output rows to source rows, which leaves the other rows alone, with its way back
+    out, out_p, gx = bad(xd.detach()), bad(pd.detach()), bad(gd)
+    row_map = torch.full((rows,), 12345, dtype=torch.int32, device=device)
+    _lib.check(lib.ms_sort_chunks(stream, ptr(xd), ptr(sd), ptr(od), 4, rows, hidden, code, ptr(pd), pcode, ptr(out), ptr(out_p),
+                                  ptr(row_map)), "ms_sort_chunks")
+    _lib.check(lib.ms_gather_rows(stream, ptr(gd), ptr(row_map), rows, hidden, code, 1, ptr(gx)), "ms_gather_rows")
+    assert torch.equal(row_map.cpu(), torch.cat([source, torch.full((100,), -1)]).int())
+    assert torch.equal(out[:200].cpu(), exp[:200]) and torch.equal(out_p[:200].cpu(), exp_p[:200]) and torch.equal(gx.cpu()[source], g[:200])
+    assert out[200:].isnan().all() and out_p[200:].isnan().all()
+    rest = torch.ones(rows, dtype=torch.bool)
+    rest[source] = False
+    assert gx.cpu()[rest].isnan().all()
 
 
 @pytest.mark.parametrize("order", [[0, 0], [0, 1, 0], [2, 1, 2, 0], [1] * 70, [3, 0, 3, 3, 1, 0],
