@@ -10,8 +10,8 @@
 // launch's time follows its energy.  Hence the 16x16x32 matrix instruction (same rate as
 // 32x32x16, 14 % less energy per product in a loop of nothing else) and operands that go from
 // global memory to LDS without passing through registers.  The same tile on 32x32x16 with
-// register-staged operands ran 8192 x 4096 x 28672 in 8 groups at 1202 (forward, NN) / 1238
-// (dX, NT) / 1058 (dW, TN) TFLOP/s, this one at 1366 / 1465 / 1128 (bf16, random operands, one box).
+// register-staged operands ran 8192 x 4096 x 28672 in 8 groups at 1189 (forward, NN) / 1231
+// (dX, NT) / 1055 (dW, TN) TFLOP/s, this one at 1369 / 1454 / 1139 (bf16, random operands, one box).
 //
 // LDS layout per operand tile
 //   * operand contiguous along the reduction dim in memory ("RED"): stored as
