@@ -1,6 +1,8 @@
 // Declarations shared by the grouped-matmul translation units.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace ms {
@@ -49,7 +51,6 @@ struct TileTable {
                              // dealt out to single XCDs); `entries` is then unused
     int list_stride;         // entries reserved per list
     int pad[3];
-    int zeros[8];            // always zero: source of out-of-range operand chunks (holds an aligned 16-byte block)
     int begins[16];          // tile_begin of the first 16 entries (INT_MAX past the last): one load finds the entry
     int list_count[8];       // entries in use in every XCD's list
     GroupEntry entries[1];
@@ -78,6 +79,15 @@ struct GmmArgs {
     int partials_per_row;
     // split tail tiles only (OUT_SAME): fp32 partial sums, rows of `cols` floats
     float *split_ws;
+    // tiles found from the group list itself (tile_from_list), without a table; NULL: from the table
+    const int64_t *group_list;
+    const int64_t *b_offsets;   // element offsets of separately allocated weights, or NULL
+    int64_t b_stride_group, c_stride_group;
+    int group_list_type, group_type, num_groups;
+    int m, k;
+    int tile_rows;              // rows per full tile: 64, 128 or 256
+    int small_tails;            // a group's last row tile may be a smaller one
+    int tails_last_below;       // launches of fewer tiles take their small tiles last
 };
 
 struct TileCoord {
@@ -123,6 +133,16 @@ __device__ __forceinline__ int find_entry(const GroupEntry *entries, int n, int 
     return lo + __popcll(__ballot(i < hi && begin <= at)) - 1;
 }
 
+// Tile number j of an entry: of the entry's tiles every XCD (workgroup number modulo 8) takes consecutive ones of the
+// blocked order, the odd ones dealt in turn.
+__device__ __forceinline__ void deal_tile(TileCoord &tc, int j, int num_col_tiles) {
+    const int x = j & 7, odd = tc.e.num_tiles & 7;         // this XCD's place in the entry's dealing, tiles beyond whole eighths
+    const int r = x * (tc.e.num_tiles >> 3) + (x < odd ? x : odd) + (j >> 3);
+    tile_order(r, tc.e.num_row_tiles, num_col_tiles, tc.row_tile, tc.col_tile);
+    tc.tile_rows = (tc.e.tail_rows != 0 && tc.row_tile == tc.e.num_row_tiles - 1) ? tc.e.tail_rows : tc.e.tile_rows;
+    tc.valid = true;
+}
+
 // Map this workgroup to its tile.  Workgroup b runs on XCD b % 8 (round-robin dispatch).  Normally it takes a tile of
 // the entry that holds tile number b, entries laid end to end: of the entry's tiles every XCD then gets an eighth, the
 // odd ones going to the XCDs in turn from entry to entry, so the XCDs' totals differ by one tile whatever the
@@ -166,12 +186,137 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
     tc.e = table->entries[lo];
     const int j = b - tc.e.tile_begin;
     if (j >= tc.e.num_tiles) return tc;
-    const int x = j & 7, odd = tc.e.num_tiles & 7;         // this XCD's place in the entry's dealing, tiles beyond whole eighths
-    const int r = x * (tc.e.num_tiles >> 3) + (x < odd ? x : odd) + (j >> 3);
-    tile_order(r, tc.e.num_row_tiles, tc.e.num_tiles / tc.e.num_row_tiles, tc.row_tile, tc.col_tile);
-    tc.tile_rows = (tc.e.tail_rows != 0 && tc.row_tile == tc.e.num_row_tiles - 1) ? tc.e.tail_rows : tc.e.tile_rows;
-    tc.valid = true;
+    deal_tile(tc, j, tc.e.num_tiles / tc.e.num_row_tiles);
     return tc;
+}
+
+// Rows of the small tile that a remainder of `rem` rows of a group goes to, 0 for a full one.
+__host__ __device__ __forceinline__ int small_tile_rows(int rem) { return rem <= 64 ? 64 : (rem <= 128 ? 128 : 0); }
+
+// Inclusive prefix of v over the 64 lanes of a wavefront (all of them active); 0 must be neutral for op.
+template <typename Op>
+__device__ __forceinline__ unsigned wave_scan(unsigned v, Op op) {
+    const auto from = [](unsigned x, auto ctrl, auto rows) {
+        return static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), decltype(ctrl)::value,
+                                                                 decltype(rows)::value, 0xf, false));
+    };
+    using std::integral_constant;
+    v = op(v, from(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{}));     // row_shr:1
+    v = op(v, from(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{}));     // row_shr:2
+    v = op(v, from(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{}));     // row_shr:4
+    v = op(v, from(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{}));     // row_shr:8
+    v = op(v, from(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{}));     // row_bcast:15 to rows 1 and 3
+    return op(v, from(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{}));  // row_bcast:31 to rows 2 and 3
+}
+
+// The same tile as from a table without per-XCD lists and split tails (gmm_schedule_kernel), found by every wavefront
+// for itself out of a group list of at most 64 groups: lane g holds group g, the running quantities are prefix sums over
+// the lanes, and the entry that holds this workgroup's tile comes out of one ballot.  One load instead of the table's two
+// dependent ones, and no launch in front of the matmul.
+constexpr int kMaxDirectGroups = 64;
+template <bool SPLIT_RED>
+__device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
+    TileCoord tc;
+    tc.valid = false;
+    const int lane = threadIdx.x & 63;
+    const int b = blockIdx.x;
+    const int C = p.num_col_tiles;
+    const unsigned m = static_cast<unsigned>(p.m);
+    const bool mine = lane < p.num_groups;
+    const int64_t v = p.group_list[mine ? lane : p.num_groups - 1];
+    // Group ends as the schedule kernel derives them: never before the previous end, never past m.
+    const unsigned c = !mine || v < 0 ? 0u : (v > p.m ? m : static_cast<unsigned>(v));
+    const bool counts = p.group_list_type != 0;
+    const unsigned end = wave_scan(c, [&](unsigned x, unsigned y) {
+        const unsigned sum = x + y < m ? x + y : m;           // (both at most m < 2^31)
+        return counts ? sum : (x > y ? x : y);
+    });
+    const unsigned prev = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(end), 0x138, 0xf, 0xf, false));  // wave_shr:1
+    const int len = mine ? static_cast<int>(end - prev) : 0;
+    const int T = p.tile_rows, shift = 31 - __builtin_clz(T);
+    GroupEntry &e = tc.e;
+    e = GroupEntry{};
+    e.tile_rows = T;
+    if constexpr (SPLIT_RED) {
+        // every group has the tiles of one output block; groups of above-average length come first
+        const int row_tiles = (p.k + T - 1) >> shift;
+        e.num_tiles = row_tiles * C;
+        const int q = b / e.num_tiles;
+        if (q >= p.num_groups) return tc;
+        const unsigned long long all = __ballot(mine);
+        const unsigned long long first = __ballot(mine && len >= p.m / p.num_groups);
+        const int nfirst = __popcll(first);
+        const unsigned long long set = q < nfirst ? first : all & ~first;
+        const int nth = q < nfirst ? q : q - nfirst;
+        const bool in_set = (set >> lane) & 1;
+        const unsigned long long hit = __ballot(in_set && __popcll(set & ((1ull << lane) - 1ull)) == nth);
+        const int g = __builtin_ctzll(hit);
+        e.row_end = p.k;
+        e.red_begin = __builtin_amdgcn_readlane(static_cast<int>(prev), g);
+        e.red_end = __builtin_amdgcn_readlane(static_cast<int>(end), g);
+        e.c_off = g * p.c_stride_group;
+        e.num_row_tiles = row_tiles;
+        e.tail_rows = p.small_tails ? small_tile_rows(p.k - (row_tiles - 1) * T) : 0;
+        e.tile_begin = q * e.num_tiles;
+    } else {
+        const int row_tiles = (len + T - 1) >> shift;
+        const int tail = p.small_tails && len > 0 ? small_tile_rows(len - (row_tiles - 1) * T) : 0;
+        const unsigned packed = static_cast<unsigned>(row_tiles) | (tail != 0 ? 1u << 25 : 0u);   // (fewer than 2^25 row tiles, at most 64 tails)
+        const unsigned incl = wave_scan(packed, [](unsigned x, unsigned y) { return x + y; });
+        const unsigned sums = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+        const unsigned before = incl - packed;
+        const int all_rt = sums & ((1u << 25) - 1), all_tails = sums >> 25;
+        const int rt_before = before & ((1u << 25) - 1), tails_before = before >> 25;
+        const int total = all_rt * C;
+        e.red_end = p.k;
+        if (b >= total) {                          // rows past the last offset: zero-fill (empty reduction range)
+            const int last_end = __builtin_amdgcn_readlane(static_cast<int>(end), 63);
+            const int rows = p.m - last_end;
+            e.num_row_tiles = (rows + T - 1) >> shift;
+            e.num_tiles = e.num_row_tiles * C;
+            if (b - total >= e.num_tiles) return tc;
+            e.row_begin = last_end;
+            e.row_end = p.m;
+            e.red_end = 0;
+            e.tail_rows = p.small_tails ? small_tile_rows(rows - (e.num_row_tiles - 1) * T) : 0;
+            e.tile_begin = total;
+        } else {
+            const bool tails_last = total < p.tails_last_below;
+            const bool apart = tails_last && tail != 0;              // this lane's small tile is an entry of its own
+            const int full_tiles = row_tiles - (apart ? 1 : 0);
+            const int total_first = tails_last ? (all_rt - all_tails) * C : total;
+            const bool first = b < total_first;
+            const int begin = first ? (tails_last ? rt_before - tails_before : rt_before) * C : total_first + tails_before * C;
+            const int count = first ? full_tiles * C : (apart ? C : 0);
+            const int g = __builtin_ctzll(__ballot(b >= begin && b < begin + count));
+            const int g_prev = __builtin_amdgcn_readlane(static_cast<int>(prev), g);
+            const int g_end = __builtin_amdgcn_readlane(static_cast<int>(end), g);
+            const int g_tail = __builtin_amdgcn_readlane(tail, g);
+            const int g_full = __builtin_amdgcn_readlane(full_tiles, g);
+            const bool full_only = first && tails_last && g_tail != 0;
+            e.row_begin = first ? g_prev : g_prev + g_full * T;
+            e.row_end = full_only ? g_prev + g_full * T : g_end;
+            e.num_row_tiles = first ? g_full : 1;
+            e.tail_rows = full_only ? 0 : g_tail;
+            e.num_tiles = e.num_row_tiles * C;
+            e.tile_begin = __builtin_amdgcn_readlane(begin, g);
+            e.b_off = p.b_offsets != nullptr ? p.b_offsets[g] : g * p.b_stride_group;
+        }
+    }
+    deal_tile(tc, b - e.tile_begin, C);
+    return tc;
+}
+
+// This workgroup's tile, from the group list or from the table.  LISTS as in locate_tile; SPLIT_RED: the launch splits the
+// reduction dim.
+template <bool LISTS, bool SPLIT_RED>
+__device__ __forceinline__ TileCoord locate(const GmmArgs &p) {
+    if (p.group_list != nullptr) return tile_from_list<SPLIT_RED>(p);
+    return locate_tile<LISTS>(p.table);
+}
+// ... where the kernel is not compiled for one kind of split
+__device__ __forceinline__ TileCoord locate_any(const GmmArgs &p) {
+    return p.group_type == 2 ? locate<false, true>(p) : locate<false, false>(p);
 }
 
 constexpr int BM = 256, BN = 256, BK = 64;

@@ -57,6 +57,9 @@ __device__ long long g_tile_trace[kTraceSlots * 8];
 namespace ms {
 namespace {
 
+// What lanes outside the reduction range fetch instead.
+__device__ __attribute__((aligned(16))) const char kZeroChunk[16] = {};
+
 // Instruction-class masks of __builtin_amdgcn_sched_group_barrier.
 constexpr int SG_MFMA = 0x008, SG_VMEM_RD = 0x020, SG_DS_RD = 0x100, SG_DS_WR = 0x200;
 
@@ -351,7 +354,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
                                                                   static_cast<int64_t>(red_begin) * p.b_stride_red) * 2);
     const int64_t a_step = p.a_stride_red * BK * 2;
     const int64_t b_step = p.b_stride_red * BK * 2;
-    const char *zeros = reinterpret_cast<const char *>((reinterpret_cast<uintptr_t>(p.table->zeros) + 15) & ~uintptr_t(15));
+    const char *zeros = kZeroChunk;
 
     // LDS: A stages 0, 1, then B stages 0, 1, 2.
     const unsigned lds_a = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr)lds)) + wave * (kXfers * 1024);
@@ -509,7 +512,7 @@ __device__ __forceinline__ void dma_small_k_loop(const GmmArgs &p, const TileCoo
                                                                   static_cast<int64_t>(red_begin) * p.b_stride_red) * 2);
     const int64_t a_step = p.a_stride_red * BK * 2;
     const int64_t b_step = p.b_stride_red * BK * 2;
-    const char *zeros = reinterpret_cast<const char *>((reinterpret_cast<uintptr_t>(p.table->zeros) + 15) & ~uintptr_t(15));
+    const char *zeros = kZeroChunk;
 
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_ptr)lds));
     int left = red_len;                 // reduction indices from the next requested tile's start to the end
@@ -943,7 +946,7 @@ template <int DT, bool A_RED, bool B_RED, int OUT, bool LISTS = A_RED>
 __global__ __launch_bounds__(256) void gmm16_fast_kernel(const GmmArgs p) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     MS_TRACE(1);
-    const TileCoord tc = locate_tile<LISTS>(p.table);
+    const TileCoord tc = locate<LISTS, !A_RED>(p);
     if (!tc.valid) return;
     MS_TRACE(2);
     if (tc.tile_rows == 256) {
