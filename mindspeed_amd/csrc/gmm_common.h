@@ -50,7 +50,7 @@ struct TileTable {
     int lists_off;           // 0, or the byte offset from the table to eight lists of entries, one per XCD (whole groups
                              // dealt out to single XCDs); `entries` is then unused
     int list_stride;         // entries reserved per list
-    int pad[3];
+    int part_from, part_count, part_shift;   // tiles of the last round that run in parts (LastRound)
     int begins[16];          // tile_begin of the first 16 entries (INT_MAX past the last): one load finds the entry
     int list_count[8];       // entries in use in every XCD's list
     GroupEntry entries[1];
@@ -88,6 +88,7 @@ struct GmmArgs {
     int tile_rows;              // rows per full tile: 64, 128 or 256
     int small_tails;            // a group's last row tile may be a smaller one
     int tails_last_below;       // launches of fewer tiles take their small tiles last
+    int part_cus;               // compute units if the last round may be divided (LastRound), else 0
 };
 
 struct TileCoord {
@@ -133,6 +134,45 @@ __device__ __forceinline__ int find_entry(const GroupEntry *entries, int n, int 
     return lo + __popcll(__ballot(i < hi && begin <= at)) - 1;
 }
 
+// The full tiles that a launch of few rounds leaves for its last, partly filled round (tiles from .. from + count - 1) run as
+// two or four tiles of fewer rows each (1 << shift), as long as these and the launch's small tiles fit one round: such a
+// launch's time goes by its rounds, and a round lasts as long as its longest tile.  16 groups of 768 rows, bf16, us per launch
+// with whole tiles, halves only and halves or quarters (the present rule): K 1536, 1.12 rounds of tiles 80 / 70 / 66, 1.5
+// rounds 81 / 76 / 76, 2.06 rounds 117 / 105 / 101, 0.38 rounds 37 / 31 / 31; K 3072, 1.12 rounds 144 / 124 / 115, 1.5 rounds
+// 148 / 142 / 142, 2.25 rounds 218 / 208 / 206.  From six rounds on (kTailsLastRounds) it is not done: at the board's power
+// limit the compute units that sit out leave the others a higher clock.
+struct LastRound {
+    int from, count, shift;
+};
+__device__ __forceinline__ LastRound divide_last_round(int full, int small, int cus) {
+    const int left = full % cus;
+    const int shift = left == 0 ? 0 : (4 * left + small <= cus ? 2 : (2 * left + small <= cus ? 1 : 0));
+    return LastRound{full - left, shift != 0 ? left : 0, shift};
+}
+// Tile number of workgroup b, and which part of that tile it takes.  The parts of a tile follow each other on one XCD
+// (their weight panel is fetched once), but for the last, incomplete eight tiles.
+__device__ __forceinline__ int tile_of_workgroup(int b, const LastRound &lr, int &part) {
+    const int s = b - lr.from;
+    part = 0;
+    if (s < 0) return b;
+    const int extra = (lr.count << lr.shift) - lr.count;
+    if (s >= lr.count + extra) return b - extra;
+    const int whole = lr.count & ~7, in_whole = whole << lr.shift;
+    if (s < in_whole) {
+        part = (s >> 3) & ((1 << lr.shift) - 1);
+        return lr.from + ((s >> (3 + lr.shift)) << 3) + (s & 7);
+    }
+    const int rest = lr.count & 7;
+    part = (s - in_whole) / rest;
+    return lr.from + whole + (s - in_whole) - part * rest;
+}
+// Turns a full tile into its part; a part without rows is no tile.
+__device__ __forceinline__ void take_part(TileCoord &tc, int part, int shift) {
+    tc.tile_rows >>= shift;
+    tc.e.row_begin += part * tc.tile_rows;
+    tc.valid = tc.e.row_begin + tc.row_tile * tc.e.tile_rows < tc.e.row_end;
+}
+
 // Tile number j of an entry: of the entry's tiles every XCD (workgroup number modulo 8) takes consecutive ones of the
 // blocked order, the odd ones dealt in turn.
 __device__ __forceinline__ void deal_tile(TileCoord &tc, int j, int num_col_tiles) {
@@ -175,18 +215,22 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
         tc.valid = true;
         return tc;
     }
+    const LastRound lr{table->part_from, table->part_count, table->part_shift};
+    int part;
+    const int t = tile_of_workgroup(b, lr, part);
     // Up to 16 entries (8 experts with their tail tiles) their begins lie in the table's header and are fetched at once.
     int lo = 0;
     if (table->num_entries <= 16) {
 #pragma unroll
-        for (int i = 1; i < 16; ++i) lo += table->begins[i] <= b ? 1 : 0;
+        for (int i = 1; i < 16; ++i) lo += table->begins[i] <= t ? 1 : 0;
     } else {
-        lo = find_entry(table->entries, table->num_entries, b);
+        lo = find_entry(table->entries, table->num_entries, t);
     }
     tc.e = table->entries[lo];
-    const int j = b - tc.e.tile_begin;
+    const int j = t - tc.e.tile_begin;
     if (j >= tc.e.num_tiles) return tc;
     deal_tile(tc, j, tc.e.num_tiles / tc.e.num_row_tiles);
+    if (t >= lr.from && t < lr.from + lr.count) take_part(tc, part, lr.shift);
     return tc;
 }
 
@@ -234,6 +278,8 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
     const unsigned prev = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(end), 0x138, 0xf, 0xf, false));  // wave_shr:1
     const int len = mine ? static_cast<int>(end - prev) : 0;
     const int T = p.tile_rows, shift = 31 - __builtin_clz(T);
+    LastRound lr{0, 0, 0};
+    int t = b, part = 0;                           // tile number, and the part of it
     GroupEntry &e = tc.e;
     e = GroupEntry{};
     e.tile_rows = T;
@@ -268,27 +314,29 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
         const int all_rt = sums & ((1u << 25) - 1), all_tails = sums >> 25;
         const int rt_before = before & ((1u << 25) - 1), tails_before = before >> 25;
         const int total = all_rt * C;
+        const bool tails_last = total < p.tails_last_below;
+        const int total_first = tails_last ? (all_rt - all_tails) * C : total;
+        if (tails_last && p.part_cus != 0) lr = divide_last_round(total_first, total - total_first, p.part_cus);
+        t = tile_of_workgroup(b, lr, part);
         e.red_end = p.k;
-        if (b >= total) {                          // rows past the last offset: zero-fill (empty reduction range)
+        if (t >= total) {                          // rows past the last offset: zero-fill (empty reduction range)
             const int last_end = __builtin_amdgcn_readlane(static_cast<int>(end), 63);
             const int rows = p.m - last_end;
             e.num_row_tiles = (rows + T - 1) >> shift;
             e.num_tiles = e.num_row_tiles * C;
-            if (b - total >= e.num_tiles) return tc;
+            if (t - total >= e.num_tiles) return tc;
             e.row_begin = last_end;
             e.row_end = p.m;
             e.red_end = 0;
             e.tail_rows = p.small_tails ? small_tile_rows(rows - (e.num_row_tiles - 1) * T) : 0;
             e.tile_begin = total;
         } else {
-            const bool tails_last = total < p.tails_last_below;
             const bool apart = tails_last && tail != 0;              // this lane's small tile is an entry of its own
             const int full_tiles = row_tiles - (apart ? 1 : 0);
-            const int total_first = tails_last ? (all_rt - all_tails) * C : total;
-            const bool first = b < total_first;
+            const bool first = t < total_first;
             const int begin = first ? (tails_last ? rt_before - tails_before : rt_before) * C : total_first + tails_before * C;
             const int count = first ? full_tiles * C : (apart ? C : 0);
-            const int g = __builtin_ctzll(__ballot(b >= begin && b < begin + count));
+            const int g = __builtin_ctzll(__ballot(t >= begin && t < begin + count));
             const int g_prev = __builtin_amdgcn_readlane(static_cast<int>(prev), g);
             const int g_end = __builtin_amdgcn_readlane(static_cast<int>(end), g);
             const int g_tail = __builtin_amdgcn_readlane(tail, g);
@@ -303,7 +351,8 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
             e.b_off = p.b_offsets != nullptr ? p.b_offsets[g] : g * p.b_stride_group;
         }
     }
-    deal_tile(tc, b - e.tile_begin, C);
+    deal_tile(tc, t - e.tile_begin, C);
+    if (t >= lr.from && t < lr.from + lr.count) take_part(tc, part, lr.shift);
     return tc;
 }
 
