@@ -33,9 +33,8 @@ def experts_computation(hidden_states, split_list, gate_up_weights, down_weights
     The default (``fuse_activation=None``) is the reference's op sequence, one kernel per op, wherever a backward pass
     may follow; under ``torch.no_grad()`` it is the fused form, whose values are the same bit for bit and which then
     skips the fc1 output (2 % faster per forward pass on the Mixtral shape).  With ``fuse_activation`` the activation
-    comes out of the first grouped matmul's epilogue and its backward rides on the epilogue of the second
-    matmul's dX product (same values as the separate kernels', same step time, one buffer and two launches
-    fewer) whenever the operands allow it.  ``gemm_fusion``: the weight gradients are added into the weights' fp32
+    comes out of the first grouped matmul's epilogue (same values as the separate kernels', same step time, one
+    launch fewer) whenever the operands allow it, in one autograd node with the second matmul.  ``gemm_fusion``: the weight gradients are added into the weights' fp32
     ``main_grad`` by the weight-gradient product itself (mindspeed/ops/gmm.py:56-89; one kernel per op then)."""
     if gemm_fusion:
         fc1 = npu_gmm_v2(hidden_states, gate_up_weights, group_list=split_list, group_type=0, gemm_fusion=True,

@@ -21,7 +21,7 @@ import torch
 
 from .. import _lib
 from ._kernels import K
-from .gmm import _beside, _group_list_tensor, gmm_raw
+from .gmm import _beside, _group_list_tensor, _tracing, gmm_raw
 
 __all__ = ["gmm_swiglu", "GmmSwigluFunction", "grouped_mlp", "GroupedMLPFunction"]
 
@@ -112,6 +112,13 @@ def _swiglu_grad_from_fc1(dact, fc1, p):
     return d_fc1, (gp if p is not None else None)
 
 
+def _require_vector_layout(dy, w2, fc1):
+    """The layout conditions of the fused kernels on what the backward pass brings in."""
+    if not _tracing(dy) and (dy.size(1) % 8 or fc1.size(1) % 16 or any(t.data_ptr() % 16 for t in (dy, w2, fc1))):
+        raise _lib.MindSpeedAmdError("grouped_mlp: the fused kernels need the vector-access layout (16-byte aligned "
+                                     "operands, hidden and ffn multiples of 8)")
+
+
 class GroupedMLPFunction(torch.autograd.Function):
     """The whole expert MLP of ``GmmExpertsImpl.forward`` (experts.py:113-160) as one autograd node:
 
@@ -123,8 +130,12 @@ class GroupedMLPFunction(torch.autograd.Function):
     of the backward pass: dW2 runs beside dX2 and the SwiGLU backward, dW1 beside dX1, with one join at the very
     end (measured on the Mixtral shape this is no faster than three nodes that each overlap their own dW, nor than
     no overlap at all: the step is limited by board power, not by idle units).
-    ``fused_kernels``: the activation comes out of the first matmul's epilogue and its backward rides on the
-    epilogue of the dX2 product (16-bit, vector-access layout only); otherwise one kernel per op, any dtype.
+    ``fused_kernels``: the activation comes out of the first matmul's epilogue (16-bit, vector-access layout only);
+    otherwise one kernel per op, any dtype.  Its backward is a kernel of its own either way: on the epilogue of the dX2
+    product (``ms_gmm_swiglu_grad``) its 29 vector instructions per element run on compute units whose matrix cores wait
+    for them, 16 us per 256 x 256 tile, which the stand-alone kernel hides behind its memory traffic.  Measured from 8
+    experts x 16 rows to 64 x 1024, the fused form was slower throughout: 16 experts x 768 rows, 2048 x 1536, 142 against
+    114 us; 64 experts of 1000 rows on average, 2048 x 1408, 629 against 494; 8 experts x 128 rows 44 against 31.
     ``recompute_activation``: ``act`` is not kept; backward rebuilds it from ``fc1`` for dW2.
     """
 
@@ -172,11 +183,11 @@ class GroupedMLPFunction(torch.autograd.Function):
             if dw2 is not None:
                 gmm_raw(act.t(), dy, gl, 2, glt, out=dw2)
         if ctx.fused_kernels:
-            d_fc1, gp = K.gmm_swiglu_grad(dy, w2.contiguous(), fc1, p, gl, glt)
-            gp = gp if p is not None else None
-        else:
-            dact = gmm_raw(dy, w2.transpose(1, 2), gl, 0, glt)
-            d_fc1, gp = _swiglu_grad_from_fc1(dact, fc1, p)
+            w2 = w2.contiguous()
+            _require_vector_layout(dy, w2, fc1)
+        dact = gmm_raw(dy, w2.transpose(1, 2), gl, 0, glt)
+        d_fc1, gp = _swiglu_grad_from_fc1(dact, fc1, p)
+        del dact
         with side.again():                           # dW1 needs d_fc1: the side stream picks up from here
             if dw1 is not None:
                 gmm_raw(x.t(), d_fc1, gl, 2, glt, out=dw1)
@@ -189,8 +200,8 @@ class GroupedMLPFunction(torch.autograd.Function):
 def grouped_mlp(x, w1, w2, group_list, probs=None, *, group_list_type: int = 1, recompute_activation: bool = False,
                 fused_kernels: bool = True):
     """``gmm(silu(gate) * up * probs, w2)`` with ``gate | up = gmm(x, w1)``: the expert MLP as one autograd node.
-    ``w1 [E, K, 2*ffn]``, ``w2 [E, ffn, K']``.  ``fused_kernels`` (default) fuses both SwiGLU passes into the
-    neighbouring grouped matmuls and needs the layout conditions of :func:`gmm_swiglu`; without it every op is
-    its own kernel, for any dtype and layout the grouped matmul takes."""
+    ``w1 [E, K, 2*ffn]``, ``w2 [E, ffn, K']``.  ``fused_kernels`` (default) fuses the activation into the first
+    grouped matmul and needs the layout conditions of :func:`gmm_swiglu`; without it every op is its own kernel,
+    for any dtype and layout the grouped matmul takes."""
     return GroupedMLPFunction.apply(x, w1, w2, group_list, group_list_type, probs, recompute_activation, fused_kernels,
                                     _differentiated(x, w1, w2, probs))
