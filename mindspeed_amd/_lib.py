@@ -69,6 +69,13 @@ _SIGNATURES = {
     "ms_gather_rows": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _int, _int, _c_void_p],
     "ms_chunk_sort_map": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _c_void_p],
 }
+# combined forms for this package's own use (csrc/internal.h); not part of the C ABI
+_INTERNAL = {
+    "msi_routing_map_permute": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _int, _i64, _int, _c_void_p, _c_void_p,
+                                _c_void_p, _c_void_p, _c_void_p, _int, _c_void_p, _c_void_p, _c_void_p, _size_t],
+    "msi_unpermute_grad": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _i64, _i64, _i64, _int, _i64,
+                           _c_void_p, _c_void_p, _c_void_p],
+}
 EXPORTED_SYMBOLS = tuple(_SIGNATURES) + ("ms_last_error",)
 
 _lib = None
@@ -96,7 +103,7 @@ def load():
         if lib.ms_version() != ABI_VERSION:
             raise RuntimeError(f"{LIB_PATH} reports ABI version {lib.ms_version()}, this package binds version "
                                f"{ABI_VERSION}: rebuild it with `python -m mindspeed_amd.build`")
-        for name, argtypes in _SIGNATURES.items():
+        for name, argtypes in (*_SIGNATURES.items(), *_INTERNAL.items()):
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = _int

@@ -1,0 +1,28 @@
+// Entry points for this package's own bindings only: combinations of what include/mindspeed_amd.h declares that save a
+// launch.  Not part of the C ABI that ms_version() stands for.
+#pragma once
+
+#include "../../include/mindspeed_amd.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* ms_moe_routing_map_permute and ms_moe_routing_map_probs in one: permuted_probs [num_rows] in the dtype of probs (both may
+ * be NULL) and sorted_token_ids [num_rows] (may be NULL) are written beside the rows; rows that no map entry leads to get
+ * zeros. */
+int msi_routing_map_permute(ms_stream_t stream, const void *tokens, const void *routing_map, int64_t num_tokens,
+                            int64_t num_experts, int64_t hidden, int dtype, int64_t num_rows, int drop_and_pad,
+                            void *permuted, int32_t *row_id_map, int32_t *sorted_flat, int64_t *tokens_per_expert,
+                            const void *probs, int probs_dtype, void *permuted_probs, int64_t *sorted_token_ids,
+                            void *workspace, size_t workspace_bytes);
+/* ms_moe_token_unpermute_grad, and rows r of grad_permuted with sorted_flat[r] < 0 (may be NULL) written as zeros
+ * (ms_moe_zero_unmapped_rows). */
+int msi_unpermute_grad(ms_stream_t stream, const void *permuted_tokens, const void *grad_unpermuted,
+                       const int32_t *row_id_map, const void *probs, int probs_dtype, int64_t num_tokens, int64_t topk,
+                       int64_t hidden, int dtype, int64_t num_rows, const int32_t *sorted_flat, void *grad_permuted,
+                       void *grad_probs);
+
+#ifdef __cplusplus
+}
+#endif

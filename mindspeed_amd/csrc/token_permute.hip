@@ -18,6 +18,7 @@
 //
 // All kernels are HBM-bound; rows move as 16-byte vectors per lane.
 #include "common.h"
+#include "internal.h"
 
 namespace ms {
 namespace {
@@ -536,17 +537,43 @@ __global__ __launch_bounds__(256) void gather_combine_kernel(
     }
 }
 
+// Rows first .. first + count - 1 (below num_rows) that sorted_flat marks as reached by no map entry, written as zeros by
+// the wavefront: 64 marks are looked at a time, and normally there are none.
+template <typename VecT>
+__device__ __forceinline__ void zero_marked_rows(const int32_t *__restrict__ sorted_flat, VecT *__restrict__ rows, int first,
+                                                 int count, int num_rows, int vecs_per_row) {
+    const int lane = threadIdx.x & 63;
+    for (int r0 = first; r0 < first + count; r0 += 64) {
+        const int r = r0 + lane;
+        unsigned long long marked = __ballot(r < num_rows && sorted_flat[min(r, num_rows - 1)] < 0);
+        for (; marked != 0; marked &= marked - 1) {
+            VecT *dst = rows + static_cast<int64_t>(r0 + __builtin_ctzll(marked)) * vecs_per_row;
+            for (int c = lane; c < vecs_per_row; c += 64) dst[c] = VecT{};
+        }
+    }
+}
+constexpr int kMarkedPerBlock = 1024;     // marks one workgroup of 256 threads looks at
+
 // grad_permuted[row] = w * dY[t]; grad_probs[t,j] = <dY[t], permuted[row]> for row = row_id_map[t*k+j].
 // `lanes` threads (a power of two, one wavefront at most) share a token, so the dot products are folded with
 // lane shuffles and the kernel has no barrier.  Per chunk of U vectors a thread reads dY once and has the
-// loads of up to JB slots' rows in flight together.
+// loads of up to JB slots' rows in flight together.  Workgroups from row_blocks on write the rows that no entry leads to
+// (sorted_flat given): a launch of its own for them took 3 to 5 us of a routing layer's 75 to 95.
 template <typename DT, typename PT, int VEC, int JB, int U, bool COMPACT>
 __global__ __launch_bounds__(256) void unpermute_grad_kernel(
     const typename DT::storage *__restrict__ permuted, const typename DT::storage *__restrict__ grad_out,
     const int32_t *__restrict__ row_id_map, const typename PT::storage *__restrict__ probs,
     typename DT::storage *__restrict__ grad_permuted, typename PT::storage *__restrict__ grad_probs,
-    int num_tokens, int topk, int hidden, int num_rows, int lanes) {
+    int num_tokens, int topk, int hidden, int num_rows, int lanes, const int32_t *__restrict__ sorted_flat, int row_blocks) {
     using S = typename DT::storage;
+    if (static_cast<int>(blockIdx.x) >= row_blocks) {
+        using Vec = std::conditional_t<VEC * sizeof(S) == 16, v16, S>;
+        constexpr int PER_WAVE = kMarkedPerBlock / 4;
+        zero_marked_rows<Vec>(sorted_flat, reinterpret_cast<Vec *>(grad_permuted),
+                              (static_cast<int>(blockIdx.x) - row_blocks) * kMarkedPerBlock + (threadIdx.x >> 6) * PER_WAVE, PER_WAVE,
+                              num_rows, hidden / VEC);
+        return;
+    }
     const int local_row = threadIdx.x / lanes;
     const int lane = threadIdx.x % lanes;
     const int t = blockIdx.x * (256 / lanes) + local_row;
@@ -1097,6 +1124,30 @@ __global__ __launch_bounds__(256) void routing_map_probs_grad_kernel(const int32
     grad_probs[i] = static_cast<unsigned>(r) < static_cast<unsigned>(num_rows) ? grad_permuted_probs[r] : S(0);
 }
 
+// What goes with a permuted row besides its tokens: its probability (moved as it is) and its token's number.  Written by
+// the kernel that moves the row, behind its stores; a launch of its own for them took 2 to 5 us on the device and as long
+// on the host (routing layers of 4096 x 4096 and 2731 x 2048 tokens, forward and backward, with the marks of the gradient
+// kernel: 197 -> 178 and 208 -> 184 us).
+struct RowExtras {
+    const void *probs;          // [T * E] or NULL
+    void *permuted_probs;       // [num_rows], same type
+    int64_t *token_ids;         // [num_rows] or NULL
+    int elem;                   // bytes of a probability
+    __device__ __forceinline__ bool any() const { return token_ids != nullptr || permuted_probs != nullptr; }
+    __device__ __forceinline__ void put(int row, int flat, int token) const {
+        if (token_ids != nullptr) token_ids[row] = token;
+        if (permuted_probs == nullptr) return;
+        if (elem == 4) static_cast<uint32_t *>(permuted_probs)[row] = static_cast<const uint32_t *>(probs)[flat];
+        else static_cast<uint16_t *>(permuted_probs)[row] = static_cast<const uint16_t *>(probs)[flat];
+    }
+    __device__ __forceinline__ void put_unmapped(int row) const {
+        if (token_ids != nullptr) token_ids[row] = 0;
+        if (permuted_probs == nullptr) return;
+        if (elem == 4) static_cast<uint32_t *>(permuted_probs)[row] = 0;
+        else static_cast<uint16_t *>(permuted_probs)[row] = 0;
+    }
+};
+
 // Permuted rows [first, num_rows) that no map entry leads to (the caller's row count exceeds the number of set
 // entries) are written as zeros, shared out over the workgroups of the launch.
 template <typename VecT>
@@ -1140,7 +1191,7 @@ __device__ __forceinline__ void mask_vector_add(int *table, const v16 &w, int fi
 __global__ __launch_bounds__(1024) void routing_map_fused_kernel(
     const v16 *__restrict__ tokens, v16 *__restrict__ permuted, const unsigned char *__restrict__ map, int num_tokens,
     int E, int num_rows, int32_t *__restrict__ row_id_map, int32_t *__restrict__ sorted_flat,
-    int64_t *__restrict__ tokens_per_expert, int vecs_per_row, int lanes) {
+    int64_t *__restrict__ tokens_per_expert, int vecs_per_row, int lanes, const RowExtras extras) {
     extern __shared__ int lds[];     // table[32][256], sums[32], base[16], rows[rows_per_block * E]
     int *table = lds;
     int *sums = lds + 32 * 256;
@@ -1193,7 +1244,10 @@ __global__ __launch_bounds__(1024) void routing_map_fused_kernel(
         int nnz = 0;
         for (int e = 0; e < E; ++e) nnz += sums[e] + sums[16 + e];
         if (blockIdx.x == 0)
-            for (int r = nnz + tid; r < num_rows; r += nthreads) sorted_flat[r] = -1;
+            for (int r = nnz + tid; r < num_rows; r += nthreads) {
+                sorted_flat[r] = -1;
+                extras.put_unmapped(r);
+            }
         if (tokens != nullptr) zero_unmapped_rows(permuted, nnz, num_rows, vecs_per_row);
     }
     __syncthreads();
@@ -1224,8 +1278,10 @@ __global__ __launch_bounds__(1024) void routing_map_fused_kernel(
         }
     }
     __syncthreads();
-    if (!mover) return;
-    scatter_row(v, src, permuted, rows + local_row * E, E, num_rows, lane, lanes, vecs_per_row);
+    if (mover) scatter_row(v, src, permuted, rows + local_row * E, E, num_rows, lane, lanes, vecs_per_row);
+    if (extras.any())               // (behind the rows, whose stores need not wait for the probabilities' way)
+        for (int q = tid; q < own; q += nthreads)
+            if (rows[q] < num_rows) extras.put(rows[q], split + q, t0 + q / E);
 }
 
 // Mask mode for any expert count (no drop-and-pad), two launches.  The map is cut into chunks of `chunk` tokens
@@ -1254,9 +1310,9 @@ __global__ __launch_bounds__(1024) void routing_map_ranked_kernel(
     const VecT *__restrict__ tokens, VecT *__restrict__ permuted, const unsigned char *__restrict__ map, int num_tokens,
     int E, int chunk, int nchunk, const int *__restrict__ hist, int num_rows, int32_t *__restrict__ row_id_map,
     int32_t *__restrict__ sorted_flat, int64_t *__restrict__ tokens_per_expert, int vecs_per_row, int lanes,
-    int rows_per_block) {
+    int rows_per_block, const RowExtras extras) {
     // first[E], pre[E], cnt[E], scratch[32], ntok[rows_per_block], list[rows_per_block * E] (movers only),
-    // own[rows_per_block * E] bytes
+    // row_of[rows_per_block * E] (extras only), own[rows_per_block * E] bytes
     extern __shared__ int lds[];
     int *first = lds;
     int *pre = first + E;
@@ -1264,7 +1320,8 @@ __global__ __launch_bounds__(1024) void routing_map_ranked_kernel(
     int *scratch = cnt + E;
     int *ntok = scratch + 32;
     int *list = ntok + rows_per_block;
-    unsigned char *own = reinterpret_cast<unsigned char *>(list + (tokens != nullptr ? rows_per_block * E : 0));
+    int *row_of = list + (tokens != nullptr ? rows_per_block * E : 0);
+    unsigned char *own = reinterpret_cast<unsigned char *>(row_of + (extras.any() ? rows_per_block * E : 0));
     const int tid = threadIdx.x;
     const int nthreads = blockDim.x;
     const int t0 = blockIdx.x * rows_per_block;
@@ -1312,7 +1369,10 @@ __global__ __launch_bounds__(1024) void routing_map_ranked_kernel(
         __syncthreads();
     }
     if (blockIdx.x == 0)   // rows that nothing maps to (only if the caller's row count exceeds the set entries)
-        for (int r = carry + tid; r < num_rows; r += nthreads) sorted_flat[r] = -1;
+        for (int r = carry + tid; r < num_rows; r += nthreads) {
+            sorted_flat[r] = -1;
+            extras.put_unmapped(r);
+        }
     if (tokens != nullptr) zero_unmapped_rows(permuted, carry, num_rows, vecs_per_row);
     for (int e = tid; e < E; e += nthreads) {
         int next = first[e] + pre[e] + cnt[e];
@@ -1328,11 +1388,14 @@ __global__ __launch_bounds__(1024) void routing_map_ranked_kernel(
                 ++next;
             }
             row_id_map[split + q] = row;
+            if (extras.any()) row_of[q] = row;
         }
     }
     __syncthreads();
-    if (!mover) return;
-    scatter_row(v, src, permuted, list + local_row * E, ntok[local_row], num_rows, lane, lanes, vecs_per_row);
+    if (mover) scatter_row(v, src, permuted, list + local_row * E, ntok[local_row], num_rows, lane, lanes, vecs_per_row);
+    if (extras.any())
+        for (int q = tid; q < own_n; q += nthreads)
+            if (row_of[q] < num_rows) extras.put(row_of[q], split + q, t0 + q / E);
 }
 
 // ---- host helpers -------------------------------------------------------------------
@@ -1558,18 +1621,19 @@ int launch_gather_combine(hipStream_t stream, const void *rows, const int32_t *m
 template <typename DT, typename PT>
 int launch_unpermute_grad(hipStream_t stream, const void *permuted, const void *gy, const int32_t *map,
                           const void *probs, void *gperm, void *gprobs, int64_t T, int64_t k, int64_t H,
-                          int64_t num_rows) {
+                          int64_t num_rows, const int32_t *sorted_flat) {
     using S = typename DT::storage;
     using PS = typename PT::storage;
     constexpr int VEC = 16 / sizeof(S);
     const bool vec_ok = (H % VEC == 0) && aligned16(gy) && aligned16(gperm) && (permuted == nullptr || aligned16(permuted));
     const int64_t vecs = vec_ok ? H / VEC : H;
     const RowLayout rl = row_layout(vecs);
-    const dim3 grid(static_cast<unsigned>(ceil_div(T, rl.rows_per_block)));
+    const int64_t row_blocks = ceil_div(T, rl.rows_per_block);
+    const dim3 grid(static_cast<unsigned>(row_blocks + (sorted_flat != nullptr ? ceil_div(num_rows, kMarkedPerBlock) : 0)));
 #define MS_UG_ARGS                                                                                                   \
     static_cast<const S *>(permuted), static_cast<const S *>(gy), map, static_cast<const PS *>(probs),               \
         static_cast<S *>(gperm), static_cast<PS *>(gprobs), static_cast<int>(T), static_cast<int>(k),                \
-        static_cast<int>(H), static_cast<int>(num_rows), rl.lanes
+        static_cast<int>(H), static_cast<int>(num_rows), rl.lanes, sorted_flat, static_cast<int>(row_blocks)
     // (the same choice as the gather's: list the valid slots of a many-slot or mostly empty map first)
     const bool sparse = k > 2 && 2 * num_rows <= T * k;
     const bool compact = (k > 8 || sparse) && rl.rows_per_block * k <= kCompactMaxLocal;
@@ -1715,10 +1779,10 @@ extern "C" int ms_moe_token_permute_grad(ms_stream_t stream, const void *grad_pe
     return ms_moe_token_unpermute(stream, grad_permuted, row_id_map, nullptr, dtype, T, k, H, dtype, num_rows, grad_tokens);
 }
 
-extern "C" int ms_moe_token_unpermute_grad(ms_stream_t stream_, const void *permuted, const void *grad_out,
-                                           const int32_t *row_id_map, const void *probs, int probs_dtype, int64_t T,
-                                           int64_t k, int64_t H, int dtype, int64_t num_rows, void *grad_permuted,
-                                           void *grad_probs) {
+extern "C" int msi_unpermute_grad(ms_stream_t stream_, const void *permuted, const void *grad_out,
+                                  const int32_t *row_id_map, const void *probs, int probs_dtype, int64_t T, int64_t k,
+                                  int64_t H, int dtype, int64_t num_rows, const int32_t *sorted_flat, void *grad_permuted,
+                                  void *grad_probs) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (int rc = check_common("ms_moe_token_unpermute_grad", T, k, H, dtype)) return rc;
     MS_REQUIRE(probs == nullptr || probs_dtype == dtype || probs_dtype == MS_FP32, MS_ERR_UNSUPPORTED,
@@ -1736,12 +1800,20 @@ extern "C" int ms_moe_token_unpermute_grad(ms_stream_t stream_, const void *perm
                "ms_moe_token_unpermute_grad: NULL tensor pointer");
     switch (dtype) {
 #define MS_UG_CALL(DT_, PT_) \
-    launch_unpermute_grad<DT_, PT_>(stream, permuted, grad_out, row_id_map, probs, grad_permuted, grad_probs, T, k, H, num_rows)
+    launch_unpermute_grad<DT_, PT_>(stream, permuted, grad_out, row_id_map, probs, grad_permuted, grad_probs, T, k, H, num_rows, sorted_flat)
         case MS_BF16: return p32 ? MS_UG_CALL(BF16, FP32) : MS_UG_CALL(BF16, BF16);
         case MS_FP16: return p32 ? MS_UG_CALL(FP16, FP32) : MS_UG_CALL(FP16, FP16);
         default: return MS_UG_CALL(FP32, FP32);
 #undef MS_UG_CALL
     }
+}
+
+extern "C" int ms_moe_token_unpermute_grad(ms_stream_t stream, const void *permuted, const void *grad_out,
+                                           const int32_t *row_id_map, const void *probs, int probs_dtype, int64_t T,
+                                           int64_t k, int64_t H, int dtype, int64_t num_rows, void *grad_permuted,
+                                           void *grad_probs) {
+    return msi_unpermute_grad(stream, permuted, grad_out, row_id_map, probs, probs_dtype, T, k, H, dtype, num_rows, nullptr,
+                              grad_permuted, grad_probs);
 }
 
 // ---- routing-map mode entry points ------------------------------------------------------
@@ -1768,14 +1840,14 @@ template <typename VecT>
 void launch_routing_map_ranked(hipStream_t stream, const void *tokens, void *permuted, const unsigned char *map, int64_t T,
                                int64_t E, int chunk, int nchunk, const int *hist, int64_t num_rows, int32_t *row_id_map,
                                int32_t *sorted_flat, int64_t *tpe, int64_t vecs, int lanes, int threads,
-                               int rows_per_block) {
-    const size_t ints = 3 * static_cast<size_t>(E) + 32 + rows_per_block +
-                        (tokens != nullptr ? static_cast<size_t>(rows_per_block) * E : 0);
+                               int rows_per_block, const ms::RowExtras &extras) {
+    const size_t lists = (tokens != nullptr ? 1 : 0) + (extras.token_ids != nullptr || extras.permuted_probs != nullptr ? 1 : 0);
+    const size_t ints = 3 * static_cast<size_t>(E) + 32 + rows_per_block + lists * rows_per_block * E;
     const size_t lds = ints * sizeof(int) + ((static_cast<size_t>(rows_per_block) * E + 3) & ~static_cast<size_t>(3));
     hipLaunchKernelGGL((ms::routing_map_ranked_kernel<VecT>), dim3(static_cast<unsigned>(ms::ceil_div(T, rows_per_block))),
                        dim3(threads), lds, stream, static_cast<const VecT *>(tokens), static_cast<VecT *>(permuted), map,
                        static_cast<int>(T), static_cast<int>(E), chunk, nchunk, hist, static_cast<int>(num_rows),
-                       row_id_map, sorted_flat, tpe, static_cast<int>(vecs), lanes, rows_per_block);
+                       row_id_map, sorted_flat, tpe, static_cast<int>(vecs), lanes, rows_per_block, extras);
 }
 
 // Mask mode in two launches (chunk histogram, then ranking + row movement).  Returns -1 when the shape does not
@@ -1783,7 +1855,7 @@ void launch_routing_map_ranked(hipStream_t stream, const void *tokens, void *per
 // then takes the sort-based path.
 int routing_map_two_launches(hipStream_t stream, const void *tokens, const unsigned char *map, int64_t T, int64_t E,
                              int64_t row_bytes, int dtype, int64_t num_rows, void *permuted, int32_t *row_id_map,
-                             int32_t *sorted_flat, int64_t *tpe, int *hist) {
+                             int32_t *sorted_flat, int64_t *tpe, int *hist, const ms::RowExtras &extras) {
     using namespace ms;
     int lanes = 1, threads = 1024, rows_per_block;
     int64_t vecs = 1;
@@ -1809,13 +1881,13 @@ int routing_map_two_launches(hipStream_t stream, const void *tokens, const unsig
     MS_CHECK_LAUNCH("routing_map_hist_kernel");
     if (vec_bytes == 16)
         launch_routing_map_ranked<v16>(stream, tokens, permuted, map, T, E, chunk, nchunk, hist, num_rows, row_id_map,
-                                       sorted_flat, tpe, vecs, lanes, threads, rows_per_block);
+                                       sorted_flat, tpe, vecs, lanes, threads, rows_per_block, extras);
     else if (vec_bytes == 4)
         launch_routing_map_ranked<uint32_t>(stream, tokens, permuted, map, T, E, chunk, nchunk, hist, num_rows, row_id_map,
-                                            sorted_flat, tpe, vecs, lanes, threads, rows_per_block);
+                                            sorted_flat, tpe, vecs, lanes, threads, rows_per_block, extras);
     else
         launch_routing_map_ranked<uint16_t>(stream, tokens, permuted, map, T, E, chunk, nchunk, hist, num_rows, row_id_map,
-                                            sorted_flat, tpe, vecs, lanes, threads, rows_per_block);
+                                            sorted_flat, tpe, vecs, lanes, threads, rows_per_block, extras);
     MS_CHECK_LAUNCH("routing_map_ranked_kernel");
     return MS_OK;
 }
@@ -1836,10 +1908,29 @@ extern "C" int ms_moe_routing_map_workspace_size(int64_t T, int64_t E, int drop_
     return MS_OK;
 }
 
-extern "C" int ms_moe_routing_map_permute(ms_stream_t stream_, const void *tokens, const void *routing_map, int64_t T,
-                                          int64_t E, int64_t H, int dtype, int64_t num_rows, int drop_and_pad,
-                                          void *permuted, int32_t *row_id_map, int32_t *sorted_flat,
-                                          int64_t *tokens_per_expert, void *workspace, size_t workspace_bytes) {
+namespace {
+int launch_routing_map_probs(hipStream_t stream, const int32_t *sorted_flat, int64_t num_rows, int64_t E, const void *probs,
+                             int dtype, void *permuted_probs, int64_t *sorted_token_ids) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(num_rows, 256)));
+    // a probability is only moved, never computed with: 2-byte types share one instantiation
+    if (probs != nullptr && dtype == MS_FP32)
+        hipLaunchKernelGGL(routing_map_probs_kernel<uint32_t>, grid, dim3(256), 0, stream, sorted_flat, static_cast<int>(num_rows),
+                           static_cast<int>(E), static_cast<const uint32_t *>(probs), static_cast<uint32_t *>(permuted_probs),
+                           sorted_token_ids);
+    else
+        hipLaunchKernelGGL(routing_map_probs_kernel<uint16_t>, grid, dim3(256), 0, stream, sorted_flat, static_cast<int>(num_rows),
+                           static_cast<int>(E), static_cast<const uint16_t *>(probs), static_cast<uint16_t *>(permuted_probs),
+                           sorted_token_ids);
+    MS_CHECK_LAUNCH("routing_map_probs_kernel");
+    return MS_OK;
+}
+}  // namespace
+
+extern "C" int msi_routing_map_permute(ms_stream_t stream_, const void *tokens, const void *routing_map, int64_t T, int64_t E,
+                                       int64_t H, int dtype, int64_t num_rows, int drop_and_pad, void *permuted,
+                                       int32_t *row_id_map, int32_t *sorted_flat, int64_t *tokens_per_expert,
+                                       const void *probs, int probs_dtype, void *permuted_probs, int64_t *sorted_token_ids,
+                                       void *workspace, size_t workspace_bytes) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const char *fn = "ms_moe_routing_map_permute";
     if (int rc = check_routing(fn, T, E, drop_and_pad)) return rc;
@@ -1850,7 +1941,20 @@ extern "C" int ms_moe_routing_map_permute(ms_stream_t stream_, const void *token
                (long long)num_rows);
     if (tokens != nullptr)
         if (int rc = check_common(fn, T, E, H, dtype)) return rc;
+    MS_REQUIRE(probs == nullptr || probs_dtype == MS_BF16 || probs_dtype == MS_FP16 || probs_dtype == MS_FP32, MS_ERR_UNSUPPORTED,
+               "%s: probs dtype %d is not one of bf16/fp16/fp32", fn, probs_dtype);
+    MS_REQUIRE(num_rows == 0 || (probs == nullptr) == (permuted_probs == nullptr), MS_ERR_INVALID_ARGUMENT,
+               "%s: probs and permuted_probs must be given together", fn);
     if (T == 0) return MS_OK;
+    if (tokens == nullptr && num_rows > 0 && (permuted_probs != nullptr || sorted_token_ids != nullptr)) {
+        // maps only: the kernels' workgroups hold many tokens then, and their LDS has no room for the rows beside
+        if (int rc = ms_moe_routing_map_permute(stream_, nullptr, routing_map, T, E, H, dtype, num_rows, drop_and_pad, permuted,
+                                                row_id_map, sorted_flat, tokens_per_expert, workspace, workspace_bytes))
+            return rc;
+        return launch_routing_map_probs(stream, sorted_flat, num_rows, E, probs, probs_dtype, permuted_probs, sorted_token_ids);
+    }
+    const RowExtras extras{probs, num_rows > 0 ? permuted_probs : nullptr, num_rows > 0 ? sorted_token_ids : nullptr,
+                           probs_dtype == MS_FP32 ? 4 : 2};
     MS_REQUIRE(routing_map && row_id_map && (sorted_flat || num_rows == 0), MS_ERR_INVALID_ARGUMENT,
                "%s: NULL tensor pointer", fn);
     MS_REQUIRE(tokens == nullptr || permuted != nullptr || num_rows == 0, MS_ERR_INVALID_ARGUMENT, "%s: permuted is NULL", fn);
@@ -1872,7 +1976,7 @@ extern "C" int ms_moe_routing_map_permute(ms_stream_t stream_, const void *token
                                dim3(threads), lds, stream, static_cast<const v16 *>(tokens), static_cast<v16 *>(permuted),
                                static_cast<const unsigned char *>(routing_map), static_cast<int>(T), static_cast<int>(E),
                                static_cast<int>(num_rows), row_id_map, sorted_flat, tokens_per_expert,
-                               static_cast<int>(vecs), lanes);
+                               static_cast<int>(vecs), lanes, extras);
             MS_CHECK_LAUNCH("routing_map_fused_kernel");
             return MS_OK;
         }
@@ -1885,7 +1989,7 @@ extern "C" int ms_moe_routing_map_permute(ms_stream_t stream_, const void *token
     if (!drop_and_pad) {
         const int rc = routing_map_two_launches(stream, tokens, static_cast<const unsigned char *>(routing_map), T, E,
                                                 row_bytes_f, dtype, num_rows, permuted, row_id_map, sorted_flat,
-                                                tokens_per_expert, reinterpret_cast<int *>(ws + r.keys_off));
+                                                tokens_per_expert, reinterpret_cast<int *>(ws + r.keys_off), extras);
         if (rc != -1) return rc;
     }
     int32_t *keys = reinterpret_cast<int32_t *>(ws + r.keys_off);
@@ -1902,6 +2006,9 @@ extern "C" int ms_moe_routing_map_permute(ms_stream_t stream_, const void *token
                        static_cast<int>(T), static_cast<int>(E), capacity, static_cast<int>(num_rows), row_id_map, sorted_flat,
                        counts, tokens_per_expert);
     MS_CHECK_LAUNCH("routing_map_rows_kernel");
+    if (extras.permuted_probs != nullptr || extras.token_ids != nullptr)
+        if (int rc = launch_routing_map_probs(stream, sorted_flat, num_rows, E, probs, probs_dtype, permuted_probs, sorted_token_ids))
+            return rc;
     if (tokens == nullptr || num_rows == 0) return MS_OK;
     const int64_t row_bytes = H * dtype_size(dtype);
     // rows that no entry maps to (never in drop-and-pad mode, which fills every expert's block) are zeroed
@@ -1926,6 +2033,14 @@ extern "C" int ms_moe_routing_map_permute(ms_stream_t stream_, const void *token
     return MS_OK;
 }
 
+extern "C" int ms_moe_routing_map_permute(ms_stream_t stream, const void *tokens, const void *routing_map, int64_t T, int64_t E,
+                                          int64_t H, int dtype, int64_t num_rows, int drop_and_pad, void *permuted,
+                                          int32_t *row_id_map, int32_t *sorted_flat, int64_t *tokens_per_expert,
+                                          void *workspace, size_t workspace_bytes) {
+    return msi_routing_map_permute(stream, tokens, routing_map, T, E, H, dtype, num_rows, drop_and_pad, permuted, row_id_map,
+                                   sorted_flat, tokens_per_expert, nullptr, dtype, nullptr, nullptr, workspace, workspace_bytes);
+}
+
 extern "C" int ms_moe_routing_map_probs(ms_stream_t stream_, const int32_t *sorted_flat, int64_t num_rows, int64_t E,
                                         const void *probs, int dtype, void *permuted_probs, int64_t *sorted_token_ids) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
@@ -1937,18 +2052,7 @@ extern "C" int ms_moe_routing_map_probs(ms_stream_t stream_, const int32_t *sort
     MS_REQUIRE((probs == nullptr) == (permuted_probs == nullptr), MS_ERR_INVALID_ARGUMENT,
                "%s: probs and permuted_probs must be given together", fn);
     MS_REQUIRE(sorted_flat != nullptr, MS_ERR_INVALID_ARGUMENT, "%s: NULL tensor pointer", fn);
-    const dim3 grid(static_cast<unsigned>(ceil_div(num_rows, 256)));
-    // a probability is only moved, never computed with: 2-byte types share one instantiation
-    if (probs != nullptr && dtype == MS_FP32)
-        hipLaunchKernelGGL(routing_map_probs_kernel<uint32_t>, grid, dim3(256), 0, stream, sorted_flat, static_cast<int>(num_rows),
-                           static_cast<int>(E), static_cast<const uint32_t *>(probs), static_cast<uint32_t *>(permuted_probs),
-                           sorted_token_ids);
-    else
-        hipLaunchKernelGGL(routing_map_probs_kernel<uint16_t>, grid, dim3(256), 0, stream, sorted_flat, static_cast<int>(num_rows),
-                           static_cast<int>(E), static_cast<const uint16_t *>(probs), static_cast<uint16_t *>(permuted_probs),
-                           sorted_token_ids);
-    MS_CHECK_LAUNCH("routing_map_probs_kernel");
-    return MS_OK;
+    return launch_routing_map_probs(stream, sorted_flat, num_rows, E, probs, dtype, permuted_probs, sorted_token_ids);
 }
 
 extern "C" int ms_moe_routing_map_probs_grad(ms_stream_t stream_, const int32_t *row_id_map, int64_t num_entries,

@@ -192,8 +192,9 @@ _define("moe_token_unpermute(Tensor permuted, Tensor row_id_map, Tensor? probs, 
         _unpermute, lambda p, r, probs, num_tokens, topk: p.new_empty((num_tokens, p.size(1))))
 
 
-def _unpermute_grad(permuted, grad_out, row_id_map, probs, num_tokens, topk, num_rows):
-    """``permuted`` may be an empty tensor when there are no probabilities (it is only read for their gradient)."""
+def _unpermute_grad(permuted, grad_out, row_id_map, probs, num_tokens, topk, num_rows, sorted_flat=None):
+    """``permuted`` may be an empty tensor when there are no probabilities (it is only read for their gradient).
+    ``sorted_flat``: rows that it marks (below 0) are written as zeros."""
     lib = _lib.load()
     dev = grad_out.device
     hidden = grad_out.size(1)
@@ -205,26 +206,28 @@ def _unpermute_grad(permuted, grad_out, row_id_map, probs, num_tokens, topk, num
     mapped = min(rows, num_tokens * topk)
     if rows > mapped:
         grad_permuted.zero_()
+        sorted_flat = None
     work = flop_counter.unpermute_grad_bytes(num_tokens, topk, hidden, grad_out.element_size(), rows, probs is not None)
     with _lib.on(dev), flop_counter.op("unpermute_grad", work, "byte", dev):
-        _lib.check(lib.ms_moe_token_unpermute_grad(
+        _lib.check(lib.msi_unpermute_grad(
             _lib.stream_ptr(dev), _lib.ptr(permuted) if probs is not None else None, _lib.ptr(grad_out),
             _lib.ptr(row_id_map), _lib.ptr(probs), _lib.dtype_code(probs.dtype, "probs") if probs is not None else 0,
             num_tokens, topk, hidden,
-            _lib.dtype_code(grad_out.dtype, "unpermuted_tokens_grad"), mapped, _lib.ptr(grad_permuted),
-            _lib.ptr(grad_probs) if probs is not None else None), "ms_moe_token_unpermute_grad")
+            _lib.dtype_code(grad_out.dtype, "unpermuted_tokens_grad"), mapped, _lib.ptr(sorted_flat),
+            _lib.ptr(grad_permuted), _lib.ptr(grad_probs) if probs is not None else None), "ms_moe_token_unpermute_grad")
     if probs is not None and grad_probs.dtype != probs_dtype:
         grad_probs = grad_probs.to(probs_dtype)
     return grad_permuted, grad_probs
 
 
-def _unpermute_grad_fake(permuted, grad_out, row_id_map, probs, num_tokens, topk, num_rows):
+def _unpermute_grad_fake(permuted, grad_out, row_id_map, probs, num_tokens, topk, num_rows, sorted_flat=None):
     return (grad_out.new_empty((num_rows, grad_out.size(1))),
             torch.empty_like(probs) if probs is not None else grad_out.new_empty(0))
 
 
 _define("moe_token_unpermute_grad(Tensor permuted, Tensor grad_out, Tensor row_id_map, Tensor? probs, "
-        "int num_tokens, int topk, int num_rows) -> (Tensor, Tensor)", _unpermute_grad, _unpermute_grad_fake)
+        "int num_tokens, int topk, int num_rows, Tensor? sorted_flat=None) -> (Tensor, Tensor)", _unpermute_grad,
+        _unpermute_grad_fake)
 
 
 # ---- SwiGLU --------------------------------------------------------------------------------------------------
@@ -268,6 +271,19 @@ _define("swiglu_grad(Tensor grad_y, Tensor x, Tensor? probs) -> (Tensor, Tensor)
 _ROUTING_MAP_WS = {}     # workspace bytes by (tokens, experts, mode): the size query is pure host arithmetic
 
 
+def _routing_map_workspace(num_tokens, num_experts, drop_and_pad, device):
+    key = (num_tokens, num_experts, bool(drop_and_pad))
+    need = _ROUTING_MAP_WS.get(key)
+    if need is None:
+        nbytes = ctypes.c_size_t(0)
+        _lib.check(_lib.load().ms_moe_routing_map_workspace_size(num_tokens, num_experts, int(drop_and_pad),
+                                                                 ctypes.byref(nbytes)), "ms_moe_routing_map_workspace_size")
+        if len(_ROUTING_MAP_WS) > 4096:
+            _ROUTING_MAP_WS.clear()
+        need = _ROUTING_MAP_WS[key] = nbytes.value
+    return _lib.workspace(need, device)
+
+
 def _routing_map_permute(tokens, routing_map, num_rows, drop_and_pad, want_counts):
     """``tokens`` may be None (maps only).  Returns (permuted or empty, row_id_map, sorted_flat, counts or empty)."""
     lib = _lib.load()
@@ -284,16 +300,7 @@ def _routing_map_permute(tokens, routing_map, num_rows, drop_and_pad, want_count
         permuted = torch.empty((num_rows, hidden), dtype=tokens.dtype, device=dev)
     else:
         permuted = torch.empty(0, dtype=torch.float32, device=dev)
-    key = (num_tokens, num_experts, bool(drop_and_pad))
-    need = _ROUTING_MAP_WS.get(key)
-    if need is None:
-        nbytes = ctypes.c_size_t(0)
-        _lib.check(lib.ms_moe_routing_map_workspace_size(num_tokens, num_experts, int(drop_and_pad),
-                                                         ctypes.byref(nbytes)), "ms_moe_routing_map_workspace_size")
-        if len(_ROUTING_MAP_WS) > 4096:
-            _ROUTING_MAP_WS.clear()
-        need = _ROUTING_MAP_WS[key] = nbytes.value
-    ws = _lib.workspace(need, dev)
+    ws = _routing_map_workspace(num_tokens, num_experts, drop_and_pad, dev)
     work = (num_tokens * hidden * elem + num_rows * hidden * elem if tokens is not None else 0) \
         + num_tokens * num_experts * (1 + 4) + num_rows * 4
     with _lib.on(dev), flop_counter.op("permute", work, "byte", dev):
@@ -316,6 +323,43 @@ def _routing_map_permute_fake(tokens, routing_map, num_rows, drop_and_pad, want_
 
 _define("routing_map_permute(Tensor? tokens, Tensor routing_map, int num_rows, bool drop_and_pad, bool want_counts) "
         "-> (Tensor, Tensor, Tensor, Tensor)", _routing_map_permute, _routing_map_permute_fake)
+
+
+def _routing_map_permute_probs(tokens, routing_map, probs, num_rows, drop_and_pad):
+    """Rows, their probabilities and token numbers in one go: (permuted, row_id_map, sorted_flat, permuted_probs or empty,
+    sorted token ids int64)."""
+    lib = _lib.load()
+    dev = routing_map.device
+    num_tokens, num_experts = routing_map.shape
+    hidden = tokens.size(1)
+    row_id_map = torch.empty(num_tokens * num_experts, dtype=torch.int32, device=dev)
+    sorted_flat = torch.empty(num_rows, dtype=torch.int32, device=dev)
+    permuted = torch.empty((num_rows, hidden), dtype=tokens.dtype, device=dev)
+    permuted_probs = torch.empty(num_rows if probs is not None else 0,
+                                 dtype=probs.dtype if probs is not None else torch.float32, device=dev)
+    sorted_indices = torch.empty(num_rows, dtype=torch.int64, device=dev)
+    ws = _routing_map_workspace(num_tokens, num_experts, drop_and_pad, dev)
+    work = (num_tokens + num_rows) * hidden * tokens.element_size() + num_tokens * num_experts * (1 + 4) + num_rows * 12
+    with _lib.on(dev), flop_counter.op("permute", work, "byte", dev):
+        _lib.check(lib.msi_routing_map_permute(
+            _lib.stream_ptr(dev), _lib.ptr(tokens), _lib.ptr(routing_map), num_tokens, num_experts, hidden,
+            _lib.dtype_code(tokens.dtype, "tokens"), num_rows, int(drop_and_pad), _lib.ptr(permuted), _lib.ptr(row_id_map),
+            _lib.ptr(sorted_flat), None, _lib.ptr(probs), _lib.dtype_code(probs.dtype, "probs") if probs is not None else 0,
+            _lib.ptr(permuted_probs) if probs is not None else None, _lib.ptr(sorted_indices), _lib.ptr(ws), ws.numel()),
+            "msi_routing_map_permute")
+    return permuted, row_id_map, sorted_flat, permuted_probs, sorted_indices
+
+
+def _routing_map_permute_probs_fake(tokens, routing_map, probs, num_rows, drop_and_pad):
+    num_tokens, num_experts = routing_map.shape
+    return (tokens.new_empty((num_rows, tokens.size(1))), routing_map.new_empty(num_tokens * num_experts, dtype=torch.int32),
+            routing_map.new_empty(num_rows, dtype=torch.int32),
+            probs.new_empty(num_rows) if probs is not None else routing_map.new_empty(0, dtype=torch.float32),
+            routing_map.new_empty(num_rows, dtype=torch.int64))
+
+
+_define("routing_map_permute_probs(Tensor tokens, Tensor routing_map, Tensor? probs, int num_rows, bool drop_and_pad) "
+        "-> (Tensor, Tensor, Tensor, Tensor, Tensor)", _routing_map_permute_probs, _routing_map_permute_probs_fake)
 
 
 def _routing_map_probs(sorted_flat, probs, num_experts):

@@ -61,6 +61,13 @@ def routing_map_row_maps(routing_map: torch.Tensor, num_rows: int, drop_and_pad:
     moved in the same call.
     """
     _check_map(routing_map)
+    routing_map, num_rows, tokens = _row_map_arguments(routing_map, num_rows, drop_and_pad, tokens)
+    permuted, row_id_map, sorted_flat, counts = K.routing_map_permute(
+        tokens, routing_map, num_rows, bool(drop_and_pad), bool(want_counts))
+    return (permuted if tokens is not None else None), row_id_map, sorted_flat, (counts if want_counts else None)
+
+
+def _row_map_arguments(routing_map, num_rows, drop_and_pad, tokens):
     routing_map = routing_map.contiguous()
     num_tokens, num_experts = routing_map.shape
     num_rows = int(num_rows)
@@ -74,9 +81,7 @@ def routing_map_row_maps(routing_map: torch.Tensor, num_rows: int, drop_and_pad:
         if tokens.size(1) == 0:
             raise RuntimeError("tokens must have a non-empty hidden dimension")
         _lib.dtype_code(tokens.dtype, "tokens")
-    permuted, row_id_map, sorted_flat, counts = K.routing_map_permute(
-        tokens, routing_map, num_rows, bool(drop_and_pad), bool(want_counts))
-    return (permuted if tokens is not None else None), row_id_map, sorted_flat, (counts if want_counts else None)
+    return routing_map, num_rows, tokens
 
 
 # The dispatcher hands ``unpermute`` the same ``routing_map`` tensor it gave ``permute``.  The row maps that
@@ -168,7 +173,6 @@ class MoePermuteMaskMap(torch.autograd.Function):
         _check_map(routing_map, tokens.size(0))
         num_tokens, num_experts = routing_map.shape
         num_rows = _resolve_num_rows(routing_map, num_out_tokens, drop_and_pad)
-        permuted, row_id_map, sorted_flat, _ = routing_map_row_maps(routing_map, num_rows, drop_and_pad, tokens)
         if probs is not None:
             _lib.require_device(probs, "probs")
             if probs.shape != routing_map.shape:
@@ -176,7 +180,9 @@ class MoePermuteMaskMap(torch.autograd.Function):
                                    f"{tuple(routing_map.shape)}")
             _lib.dtype_code(probs.dtype, "probs")
             probs = probs.contiguous()
-        permuted_probs, sorted_indices = K.routing_map_probs(sorted_flat, probs, num_experts)
+        dense_map, num_rows, tokens = _row_map_arguments(routing_map, num_rows, drop_and_pad, tokens)
+        permuted, row_id_map, sorted_flat, permuted_probs, sorted_indices = K.routing_map_permute_probs(
+            tokens, dense_map, probs, num_rows, bool(drop_and_pad))
         if probs is None:
             permuted_probs = None
         ctx.save_for_backward(row_id_map)
@@ -271,12 +277,10 @@ class MoeUnpermuteMaskMap(torch.autograd.Function):
         grad_out = unpermuted_tokens_grad.contiguous()
         # Every mapped row has exactly one entry leading to it and is written by the gradient kernel.  Rows that
         # nothing maps to exist only when the caller's row count exceeds the number of set mask entries; they are
-        # marked in sorted_flat and written as zeros (a launch whose workgroups all return at once when there are none).
+        # marked in sorted_flat and written as zeros by a few workgroups more of the same launch.
         grad_permuted, grad_probs = K.moe_token_unpermute_grad(
             permuted_tokens if probs is not None else grad_out.new_empty(0), grad_out, row_id_map, probs,
-            ctx.num_tokens, ctx.num_experts, ctx.num_rows)
-        if not ctx.all_rows_mapped:
-            K.zero_unmapped_rows(grad_permuted, sorted_flat)
+            ctx.num_tokens, ctx.num_experts, ctx.num_rows, None if ctx.all_rows_mapped else sorted_flat)
         if probs is None or not ctx.needs_input_grad[3]:
             grad_probs = None
         return grad_permuted, None, None, grad_probs, None, None
