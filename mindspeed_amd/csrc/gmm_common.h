@@ -397,6 +397,14 @@ __device__ __forceinline__ void mfma16x16(v16 a, v16 b, f32x4 &acc) {
     else asm("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
+// The same pointer in scalar registers, whatever the compiler knows about its uniformity.
+__device__ __forceinline__ const char *uniform(const char *p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint64_t lo = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
+    const uint64_t hi = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32)));
+    return reinterpret_cast<const char *>(lo | hi << 32);
+}
+
 // LDS swizzle: 16-byte chunk position of (row, chunk) inside the row's 128 bytes.
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 

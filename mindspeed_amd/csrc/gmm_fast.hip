@@ -275,14 +275,6 @@ struct DmaOperand {
     }
 };
 
-// The same pointer in scalar registers, whatever the compiler knows about its uniformity.
-__device__ __forceinline__ const char *uniform(const char *p) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    const uint64_t lo = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
-    const uint64_t hi = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32)));
-    return reinterpret_cast<const char *>(lo | hi << 32);
-}
-
 // The accumulators are in their registers at this point of the program, whatever was or will be done with them.
 template <int TM, int TN>
 __device__ __forceinline__ void pin(f32x4 (&acc)[TM][TN]) {

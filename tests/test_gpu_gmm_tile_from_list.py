@@ -1,6 +1,7 @@
 """Grouped matmuls of up to 64 groups, whose workgroups find their tiles in the group list by themselves, against the same
 groups with empty ones added behind them up to 70, which go through the tile table.  A tile's sums do not depend on how it
-was found, so the results are equal bit for bit."""
+was found, so the results are equal bit for bit; only the fp32 weight gradient may take tiles of another kind with more
+groups, which add up in another order (at most 2e-6 of the sum of magnitudes for the fewer than 2200 products here)."""
 import pytest
 import torch
 
@@ -44,7 +45,11 @@ def _both(shape, gl, gl_pad, m, counted):
     kind = 1 if counted else 0
     assert torch.equal(gmm_raw(x, w, gl, 0, kind), gmm_raw(x, w_pad, gl_pad, 0, kind))
     assert torch.equal(gmm_raw(dy, w.transpose(1, 2), gl, 0, kind), gmm_raw(dy, w_pad.transpose(1, 2), gl_pad, 0, kind))
-    assert torch.equal(gmm_raw(x.t(), dy, gl, 2, kind), gmm_raw(x.t(), dy, gl_pad, 2, kind)[:gl.numel()])
+    dw, dw_pad = gmm_raw(x.t(), dy, gl, 2, kind), gmm_raw(x.t(), dy, gl_pad, 2, kind)[:gl.numel()]
+    if dtype == torch.float32:
+        assert bool(((dw - dw_pad).abs() <= 2e-6 * gmm_raw(x.abs().t(), dy.abs(), gl, 2, kind)).all())
+    else:
+        assert torch.equal(dw, dw_pad)
 
 
 @pytest.mark.parametrize("counted", [True, False], ids=["counts", "offsets"])
