@@ -20,6 +20,9 @@ TRACE_LIB_PATH = os.path.join(HERE, "libmindspeed_amd_trace.so")   # diagnostic 
 MICROBENCH_CSRC = os.path.join(HERE, "csrc_microbench")
 MICROBENCH_LIB_PATH = os.path.join(HERE, "libmindspeed_amd_microbench.so")   # measurement helpers (plain copy kernel)
 
+HOST_SRC = os.path.join(HERE, "csrc_host", "launch.cpp")
+HOST_LIB_PATH = os.path.join(HERE, "_host.so")               # the kernel calls of the Python ops in native code
+
 ARCH = "gfx950"
 # packed-fp32 VALU forms are switched off for every device translation unit.
 HIPCC_FLAGS = [
@@ -112,10 +115,33 @@ def build_microbench(verbose: bool = False) -> str:
     return MICROBENCH_LIB_PATH
 
 
+def build_host(verbose: bool = False) -> str:
+    """The native side of the Python ops (csrc_host/launch.cpp): host code only, against torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    cmd = [os.environ.get("CXX") or "g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden",
+           "-DTORCH_EXTENSION_NAME=_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",      # (what torch's own stream header asks for)
+           *(f"-I{d}" for d in (*include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include")),
+           HOST_SRC, "-o", HOST_LIB_PATH, *(f"-L{d}" for d in library_paths()),
+           "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for {HOST_SRC}:\n{res.stderr}")
+    if verbose:
+        print(f"built {HOST_LIB_PATH}")
+    return HOST_LIB_PATH
+
+
 if __name__ == "__main__":
     if "--trace" in sys.argv:
         build_trace(verbose=True)
     elif "--microbench" in sys.argv:
         build_microbench(verbose=True)
+    elif "--host" in sys.argv:
+        build_host(verbose=True)
     else:
         build(force="--incremental" not in sys.argv, verbose=True)

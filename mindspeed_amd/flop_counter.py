@@ -88,6 +88,11 @@ def timing_active() -> bool:
     return _active is not None and _active.timing
 
 
+def recording() -> bool:
+    """True while a recorder takes note of every op."""
+    return _active is not None
+
+
 class _NoOp:
     __slots__ = ()
 

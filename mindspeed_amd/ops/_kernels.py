@@ -12,6 +12,7 @@ There is no CPU kernel: on CPU tensors the ops raise.
 from __future__ import annotations
 
 import ctypes
+import warnings
 
 import torch
 
@@ -595,12 +596,14 @@ _define("zero_unmapped_rows(Tensor(a!) rows, Tensor sorted_flat) -> ()", _zero_u
 # make_fx, profilers), a tensor subclass, a meta tensor — it goes through the dispatcher op of the same name, which
 # routes to the same function for device tensors and to the fake kernel otherwise.  The direct call saves the boxing
 # and schema matching of a Python-registered op (measured: about a third of the host time of a small layer step).
+# A plain call is made in native code (csrc_host/launch.cpp) where that has a function of the op's name, unless a Recorder
+# wants to bracket it or the function leaves it to this module's (an argument it does not take).
 _len_dispatch_modes = torch._C._len_torch_dispatch_stack
 _len_function_modes = torch._C._len_torch_function_stack
 
 
-def _plain(args) -> bool:
-    if _len_dispatch_modes() or _len_function_modes() or torch.compiler.is_compiling():
+def _plain_arguments(args) -> bool:
+    if _len_dispatch_modes() or _len_function_modes():
         return False
     for a in args:
         if a is None or a.__class__ is int or a.__class__ is bool:
@@ -612,11 +615,37 @@ def _plain(args) -> bool:
             if a.device.type != "cuda":
                 return False
         elif isinstance(a, (list, tuple)):
-            if not _plain(a):
+            if not _plain_arguments(a):
                 return False
         elif isinstance(a, torch.Tensor):
             return False
     return True
+
+
+_plain_check = _plain_arguments      # or the native one, once that is loaded
+
+
+def _plain(args) -> bool:
+    return not torch.compiler.is_compiling() and _plain_check(args)
+
+
+_native = None                       # op name -> native function; filled by the first plain call
+
+
+def _load_native():
+    global _native, _plain_check
+    _lib.load()
+    try:
+        from .. import _host
+    except ImportError as e:
+        warnings.warn(f"the native side of mindspeed_amd's ops cannot be loaded ({e}); calls go through ctypes, which costs "
+                      "4 to 8 us of host time each.  Build it with `python -m mindspeed_amd.build --host`.")
+        _native = {}
+        return _native
+    _host.bind(_lib.LIB_PATH, _lib.MindSpeedAmdError)
+    _plain_check = _host.plain
+    _native = {name: getattr(_host, name) for name in _DEVICE_FNS if hasattr(_host, name)}
+    return _native
 
 
 class _Ops:
@@ -627,9 +656,17 @@ class _Ops:
         op = getattr(self._ns, name)
 
         def call(*args):
-            if _plain(args):
-                return device_fn(*args)
-            return op(*args)
+            if not _plain(args):
+                return op(*args)
+            if not flop_counter.recording():
+                native = (_native if _native is not None else _load_native()).get(name)
+                if native is not None:
+                    out = native(*args)
+                    if out is True:              # (nothing to return)
+                        return None
+                    if out is not None and out is not False:
+                        return out
+            return device_fn(*args)
         call.__name__ = name
         setattr(self, name, call)
 

@@ -113,8 +113,7 @@ def _remember_row_map(routing_map, num_rows, drop_and_pad, row_id_map, sorted_fl
     maps = kept[1]
     # (the last element: index tensors known to agree with the map, as weak references with their version counters)
     known = [] if sorted_indices is None else [(weakref.ref(sorted_indices), sorted_indices._version)]
-    maps[(int(num_rows), bool(drop_and_pad))] = (row_id_map, sorted_flat, torch.cuda.current_stream(routing_map.device),
-                                                 known)
+    maps[(int(num_rows), bool(drop_and_pad))] = (row_id_map, sorted_flat, _lib.stream_ptr(routing_map.device), known)
     while len(maps) > _ROW_MAPS_KEPT:
         maps.pop(next(iter(maps)))
 
@@ -128,9 +127,11 @@ def _recall_row_map(routing_map, num_rows, drop_and_pad):
     if hit is None:
         return None
     row_id_map, sorted_flat, stream, known = hit
-    now = torch.cuda.current_stream(routing_map.device)
-    if now != stream:
-        now.wait_stream(stream)          # everything queued on the producing stream so far, the map's kernel included
+    if _lib.stream_ptr(routing_map.device) != stream:
+        # everything queued on the producing stream so far, the map's kernel included
+        device = routing_map.device
+        torch.cuda.current_stream(device).wait_stream(
+            torch.cuda.ExternalStream(stream, device) if stream else torch.cuda.default_stream(device))
     return row_id_map, sorted_flat, known
 
 
