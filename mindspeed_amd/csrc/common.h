@@ -105,4 +105,35 @@ __device__ __forceinline__ void store_float_as(void *p, int64_t i, int dtype, fl
     }
 }
 
+// ---- prefix sums over the lanes of a wavefront ----------------------------------
+// v moved over the lanes (data-parallel primitives: 8 clocks each, a shuffle through LDS takes a hundred); lanes without a
+// source get 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int lane_move(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+// ... of a value made of 32-bit words
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T lanes_move(const T &v) {
+    static_assert(sizeof(T) % 4 == 0, "scan items are made of 32-bit words");
+    T r;
+#pragma unroll
+    for (int w = 0; w < static_cast<int>(sizeof(T) / 4); ++w)
+        reinterpret_cast<int *>(&r)[w] = lane_move<CTRL, ROWS>(reinterpret_cast<const int *>(&v)[w]);
+    return r;
+}
+// Inclusive prefix of v over the 64 lanes of a wavefront (all of them active); all-zero words must be neutral for op.
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_scan(T v, Op op) {
+    v = op(v, lanes_move<0x111, 0xf>(v));       // row_shr:1
+    v = op(v, lanes_move<0x112, 0xf>(v));       // row_shr:2
+    v = op(v, lanes_move<0x114, 0xf>(v));       // row_shr:4
+    v = op(v, lanes_move<0x118, 0xf>(v));       // row_shr:8
+    v = op(v, lanes_move<0x142, 0xa>(v));       // row_bcast:15 to rows 1 and 3
+    return op(v, lanes_move<0x143, 0xc>(v));    // row_bcast:31 to rows 2 and 3
+}
+// The value of the lane below (0 in lane 0).
+template <typename T>
+__device__ __forceinline__ T lane_below(const T &v) { return lanes_move<0x138, 0xf>(v); }      // wave_shr:1
+
 }  // namespace ms

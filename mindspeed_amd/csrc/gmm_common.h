@@ -1,8 +1,6 @@
 // Declarations shared by the grouped-matmul translation units.
 #pragma once
 
-#include <type_traits>
-
 #include "common.h"
 
 namespace ms {
@@ -237,22 +235,6 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
 // Rows of the small tile that a remainder of `rem` rows of a group goes to, 0 for a full one.
 __host__ __device__ __forceinline__ int small_tile_rows(int rem) { return rem <= 64 ? 64 : (rem <= 128 ? 128 : 0); }
 
-// Inclusive prefix of v over the 64 lanes of a wavefront (all of them active); 0 must be neutral for op.
-template <typename Op>
-__device__ __forceinline__ unsigned wave_scan(unsigned v, Op op) {
-    const auto from = [](unsigned x, auto ctrl, auto rows) {
-        return static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), decltype(ctrl)::value,
-                                                                 decltype(rows)::value, 0xf, false));
-    };
-    using std::integral_constant;
-    v = op(v, from(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{}));     // row_shr:1
-    v = op(v, from(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{}));     // row_shr:2
-    v = op(v, from(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{}));     // row_shr:4
-    v = op(v, from(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{}));     // row_shr:8
-    v = op(v, from(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{}));     // row_bcast:15 to rows 1 and 3
-    return op(v, from(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{}));  // row_bcast:31 to rows 2 and 3
-}
-
 // The same tile as from a table without per-XCD lists and split tails (gmm_schedule_kernel), found by every wavefront
 // for itself out of a group list of at most 64 groups: lane g holds group g, the running quantities are prefix sums over
 // the lanes, and the entry that holds this workgroup's tile comes out of one ballot.  One load instead of the table's two
@@ -275,7 +257,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
         const unsigned sum = x + y < m ? x + y : m;           // (both at most m < 2^31)
         return counts ? sum : (x > y ? x : y);
     });
-    const unsigned prev = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(end), 0x138, 0xf, 0xf, false));  // wave_shr:1
+    const unsigned prev = lane_below(end);
     const int len = mine ? static_cast<int>(end - prev) : 0;
     const int T = p.tile_rows, shift = 31 - __builtin_clz(T);
     LastRound lr{0, 0, 0};

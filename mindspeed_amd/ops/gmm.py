@@ -18,7 +18,7 @@ import torch
 
 from .. import _lib, flop_counter
 from ._kernels import K, _plain
-from .npu_groupmatmul_add import npu_groupmatmul_add_fp32
+from .npu_groupmatmul_add import add_weight_gradient
 
 __all__ = ["npu_gmm", "npu_gmm_v2", "GMMFunction"]
 
@@ -311,8 +311,7 @@ class GMMFunction(torch.autograd.Function):
         # accumulate form of the dW product, here on the side stream beside dX; what autograd gets for the weight is
         # a placeholder (zeros if the parameter asks for it) and the flag the optimizer wrapper looks at is set.
         with _beside(grad_y) as side:
-            offsets = group_list if ctx.group_list_type == 0 else torch.cumsum(group_list, dim=0)
-            npu_groupmatmul_add_fp32(x, grad_y, offsets, original_weight.main_grad)
+            add_weight_gradient(x, grad_y, group_list, ctx.group_list_type, original_weight.main_grad)
         (dx,), _, dbias = module.npu_gmm_backward_fusion([grad_y], [weight], group_list, ctx.group_list_type)
         side.join()
         placeholder = None

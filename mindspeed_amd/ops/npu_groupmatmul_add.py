@@ -13,6 +13,12 @@ __all__ = ["npu_groupmatmul_add_fp32"]
 
 
 def npu_groupmatmul_add_fp32(x, dy, grouplist, grad):
+    add_weight_gradient(x, dy, grouplist, 0, grad)
+    return None
+
+
+def add_weight_gradient(x, dy, grouplist, group_list_type, grad):
+    """The same for either kind of group list (0: cumulative offsets, 1: counts)."""
     from .gmm import gmm_raw  # deferred: gmm.py imports this module
 
     if grad.dtype != torch.float32:
@@ -24,5 +30,4 @@ def npu_groupmatmul_add_fp32(x, dy, grouplist, grad):
     num_groups = grouplist.shape[0]
     if grad.numel() != num_groups * x.shape[-1] * dy.shape[-1]:
         raise ValueError(f"grad has {grad.numel()} elements, expected {num_groups}x{x.shape[-1]}x{dy.shape[-1]}")
-    gmm_raw(x.transpose(-1, -2), dy, grouplist, 2, 0, out=grad, accumulate=True)
-    return None
+    gmm_raw(x.transpose(-1, -2), dy, grouplist, 2, group_list_type, out=grad, accumulate=True)
