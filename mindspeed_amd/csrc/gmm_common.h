@@ -338,17 +338,15 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
     return tc;
 }
 
-// This workgroup's tile, from the group list or from the table.  LISTS as in locate_tile; SPLIT_RED: the launch splits the
-// reduction dim.
-template <bool LISTS, bool SPLIT_RED>
+// This workgroup's tile, from the group list or from the table (which then has no per-XCD lists): the kernels that are not
+// compiled for one of the two.
+template <bool SPLIT_RED>
 __device__ __forceinline__ TileCoord locate(const GmmArgs &p) {
     if (p.group_list != nullptr) return tile_from_list<SPLIT_RED>(p);
-    return locate_tile<LISTS>(p.table);
+    return locate_tile<false>(p.table);
 }
-// ... where the kernel is not compiled for one kind of split
-__device__ __forceinline__ TileCoord locate_any(const GmmArgs &p) {
-    return p.group_type == 2 ? locate<false, true>(p) : locate<false, false>(p);
-}
+// ... nor for one kind of split
+__device__ __forceinline__ TileCoord locate_any(const GmmArgs &p) { return p.group_type == 2 ? locate<true>(p) : locate<false>(p); }
 
 constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int kTileBytes = BM * BK * 2;                 // 32 KB per operand per stage
