@@ -88,7 +88,7 @@ def cmd_traffic(args):
           f"WRITE_SIZE = {w_read:.0f} (KiB moved each way: {known_kib:.0f})")
     print(f"  -> scale factors: FETCH_SIZE x {f_scale:.3f}, WRITE_SIZE x {w_scale:.3f}\n")
     print(f"{'kernel':84s} {'disp':>5s} {'fetch_MB':>10s} {'write_MB':>10s} {'total_MB':>10s}")
-    record = {}
+    launches = collections.defaultdict(list)      # key -> (dispatches, MB per dispatch) of each of its kernels
     for kernel in fetch:
         if "ms::" not in kernel and "gmm" not in kernel and "kernel" not in kernel:
             continue
@@ -101,7 +101,9 @@ def cmd_traffic(args):
         print(f"{kernel[:84]:84s} {len(f):5d} {f_mb:10.1f} {w_mb:10.1f} {f_mb + w_mb:10.1f}")
         for pattern, key in GEMM_KEYS.items():
             if pattern in kernel:
-                record[key] = int(round((f_mb + w_mb) * 1e6))
+                launches[key].append((len(f), f_mb + w_mb))
+    # (launches with and without a tile table are different kernels of one key)
+    record = {key: int(round(sum(n * mb for n, mb in parts) / sum(n for n, _ in parts) * 1e6)) for key, parts in launches.items()}
     if args.out:
         data = {}
         if os.path.exists(args.out):
