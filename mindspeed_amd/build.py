@@ -86,12 +86,18 @@ def build(force: bool = True, verbose: bool = False) -> str:
     return LIB_PATH
 
 
-def build_trace(verbose: bool = False) -> str:
+def compile_trace() -> str:
+    """The one translation unit of its own that the diagnostic library has."""
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    return _compile(os.path.join(CSRC, "gmm_fast.hip"), True, ("-DMS_TRACE_TILES",), "_trace")
+
+
+def build_trace(verbose: bool = False, force: bool = True) -> str:
     """The diagnostic variant of the library: the grouped-matmul fast kernels compiled with MS_TRACE_TILES (every
     workgroup records time stamps of its phases, read back with ms_trace_read; see profile_tools timeline).  Not
     loaded by anything else; select it with MINDSPEED_AMD_LIB."""
     os.makedirs(OBJ_DIR, exist_ok=True)
-    objs = [_compile(s, True, ("-DMS_TRACE_TILES",), "_trace") if s.endswith("gmm_fast.hip") else _compile(s, False)
+    objs = [_compile(s, force, ("-DMS_TRACE_TILES",), "_trace") if s.endswith("gmm_fast.hip") else _compile(s, False)
             for s in sources()]
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", TRACE_LIB_PATH, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
