@@ -53,7 +53,7 @@ FORMS = {"rows of x": (0, None, False), "reduction of w": (None, 0, False), "col
          "both, w transposed": (0, 1, True)}
 
 
-@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("form", FORMS)
 def test_split_on_rows(form, dtype):
     x_back, w_back, transposed = FORMS[form]
@@ -68,7 +68,7 @@ def test_split_on_rows(form, dtype):
     assert torch.equal(out, want.to(dtype))
 
 
-@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("x_back,w_back", [(1, None), (None, 0), (1, 0)])
 def test_split_on_the_reduction(x_back, w_back, dtype):
     gen = torch.Generator(device="cuda").manual_seed(7)
@@ -78,3 +78,18 @@ def test_split_on_the_reduction(x_back, w_back, dtype):
     xs, ys = _seen(x, x_back).t().split(COUNTS), _seen(dy, w_back).split(COUNTS)
     want = torch.stack([a.t() @ b for a, b in zip(xs, ys)])
     assert torch.equal(out, want.to(dtype))
+
+
+def test_the_fused_forms_refuse_them():
+    """The kernels with the activation in their epilogue come in the vector-access form only."""
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x, w = _numbers(gen, torch.bfloat16, M, KDIM), _numbers(gen, torch.bfloat16, len(COUNTS), KDIM, 2 * N)
+    act, gl = torch.empty(M, N, dtype=x.dtype, device="cuda"), torch.tensor(COUNTS, device="cuda")
+    xp, xs = _matrix(x, 0)
+    need = ctypes.c_size_t(0)
+    _lib.check(lib.ms_gmm_workspace_size(len(COUNTS), M, 0, ctypes.byref(need)), "ms_gmm_workspace_size")
+    work = _lib.workspace(need.value, x.device)
+    rc = lib.ms_gmm_swiglu(_lib.stream_ptr(x.device), xp, *xs, w.data_ptr(), *w.stride(), None, 2 * N, act.data_ptr(), N, None, 0,
+                           gl.data_ptr(), 1, len(COUNTS), M, KDIM, N, _lib.MS_BF16, work.data_ptr(), work.numel())
+    assert rc != 0 and b"vector-access layout" in lib.ms_last_error()
