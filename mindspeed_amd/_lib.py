@@ -11,6 +11,8 @@ import threading
 
 import torch
 
+from . import build as _build
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # MINDSPEED_AMD_LIB names another build of the same library (to compare two builds on one machine)
 LIB_PATH = os.environ.get("MINDSPEED_AMD_LIB") or os.path.join(_HERE, "libmindspeed_amd.so")
@@ -69,7 +71,8 @@ _SIGNATURES = {
     "ms_gather_rows": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _int, _int, _c_void_p],
     "ms_chunk_sort_map": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _c_void_p],
 }
-# combined forms for this package's own use (csrc/internal.h); not part of the C ABI
+# combined forms for this package's own use (csrc/internal.h); not part of the C ABI that the version stands for: msi_interface()
+# names the declarations that a build was made from
 _INTERNAL = {
     "msi_routing_map_permute": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _int, _i64, _int, _c_void_p, _c_void_p,
                                 _c_void_p, _c_void_p, _c_void_p, _int, _c_void_p, _c_void_p, _c_void_p, _size_t],
@@ -84,6 +87,11 @@ _lock = threading.Lock()
 
 class MindSpeedAmdError(RuntimeError):
     """A C-ABI entry point returned a non-zero status."""
+
+
+def _declared_interface():
+    """Hash of the declarations in the source tree, None for a package without one."""
+    return _build.interface_hash() if all(os.path.exists(f) for f in _build.INTERFACE_HEADERS) else None
 
 
 def load():
@@ -103,6 +111,13 @@ def load():
         if lib.ms_version() != ABI_VERSION:
             raise RuntimeError(f"{LIB_PATH} reports ABI version {lib.ms_version()}, this package binds version "
                                f"{ABI_VERSION}: rebuild it with `python -m mindspeed_amd.build`")
+        if not hasattr(lib, "msi_interface"):
+            raise RuntimeError(f"{LIB_PATH} lacks entry points of this package: rebuild it with `python -m mindspeed_amd.build`")
+        lib.msi_interface.argtypes, lib.msi_interface.restype = [], ctypes.c_char_p
+        theirs, ours = lib.msi_interface().decode(), _declared_interface()
+        if ours is not None and theirs != ours:
+            raise RuntimeError(f"{LIB_PATH} was built for entry points {theirs}, the headers beside this package declare {ours}: "
+                               "rebuild it with `python -m mindspeed_amd.build`")
         for name, argtypes in (*_SIGNATURES.items(), *_INTERNAL.items()):
             fn = getattr(lib, name)
             fn.argtypes = argtypes

@@ -1,12 +1,15 @@
 """Build recipe for libmindspeed_amd.so (hipcc, gfx950 only, in-tree).
 
 ``python -m mindspeed_amd.build`` compiles every ``csrc/*.hip`` translation
-unit for gfx950 and links them into ``mindspeed_amd/libmindspeed_amd.so``.
+unit for gfx950 and links them into ``mindspeed_amd/libmindspeed_amd.so``,
+and builds the native side of the Python ops (``_host.so``) that calls it.
 hipcc cross-compiles, so this works on a host without a GPU.
 """
 from __future__ import annotations
 
+import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -46,8 +49,6 @@ def sources():
 def source_hash() -> str:
     """First 16 hex digits of the SHA-256 over the kernel sources (csrc/*.hip, csrc/*.h, the C-ABI header) in name
     order: names the build that measured figures (profiles/*.json) belong to."""
-    import hashlib
-
     h = hashlib.sha256()
     files = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h")))
     files.append(os.path.join(HERE, "..", "include", "mindspeed_amd.h"))
@@ -58,13 +59,31 @@ def source_hash() -> str:
     return h.hexdigest()[:16]
 
 
+INTERFACE_HEADERS = (os.path.join(HERE, "..", "include", "mindspeed_amd.h"), os.path.join(CSRC, "internal.h"))
+
+
+def interface_hash() -> str:
+    """First 16 hex digits of the SHA-256 over the declarations of the library's entry points (comments and spacing left
+    out).  Compiled into the library and into ``_host.so``, which passes its arguments by these declarations: a pair that
+    was not built from the same ones is refused."""
+    h = hashlib.sha256()
+    for f in INTERFACE_HEADERS:
+        with open(f) as fh:
+            h.update(" ".join(re.sub(r"/\*.*?\*/|//[^\n]*", " ", fh.read(), flags=re.S).split()).encode())
+    return h.hexdigest()[:16]
+
+
+def _interface_flag() -> str:
+    return f'-DMS_INTERFACE="{interface_hash()}"'
+
+
 def _compile(src: str, force: bool, extra=(), suffix="") -> str:
     obj = os.path.join(OBJ_DIR, os.path.basename(src)[:-4] + suffix + ".o")
     deps = [src, os.path.join(HERE, "..", "include", "mindspeed_amd.h")]
     deps += [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".h")]
     if not force and os.path.exists(obj) and all(os.path.getmtime(obj) > os.path.getmtime(d) for d in deps):
         return obj
-    cmd = [_hipcc(), *HIPCC_FLAGS, *extra, "-c", src, "-o", obj]
+    cmd = [_hipcc(), *HIPCC_FLAGS, _interface_flag(), *extra, "-c", src, "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{res.stderr}")
@@ -121,8 +140,11 @@ def build_microbench(verbose: bool = False) -> str:
     return MICROBENCH_LIB_PATH
 
 
-def build_host(verbose: bool = False) -> str:
+def build_host(verbose: bool = False, force: bool = True) -> str:
     """The native side of the Python ops (csrc_host/launch.cpp): host code only, against torch's headers."""
+    if not force and os.path.exists(HOST_LIB_PATH) and \
+            all(os.path.getmtime(HOST_LIB_PATH) > os.path.getmtime(d) for d in (HOST_SRC, *INTERFACE_HEADERS)):
+        return HOST_LIB_PATH
     import sysconfig
 
     import torch
@@ -130,7 +152,7 @@ def build_host(verbose: bool = False) -> str:
 
     cmd = [os.environ.get("CXX") or "g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden",
            "-DTORCH_EXTENSION_NAME=_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",      # (what torch's own stream header asks for)
+           _interface_flag(), "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",      # (the last two: what torch's own stream header asks for)
            *(f"-I{d}" for d in (*include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include")),
            HOST_SRC, "-o", HOST_LIB_PATH, *(f"-L{d}" for d in library_paths()),
            "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python"]
@@ -142,12 +164,20 @@ def build_host(verbose: bool = False) -> str:
     return HOST_LIB_PATH
 
 
-if __name__ == "__main__":
-    if "--trace" in sys.argv:
+def main(args) -> None:
+    if "--trace" in args:
         build_trace(verbose=True)
-    elif "--microbench" in sys.argv:
+    elif "--microbench" in args:
         build_microbench(verbose=True)
-    elif "--host" in sys.argv:
+    elif "--host" in args:
         build_host(verbose=True)
-    else:
-        build(force="--incremental" not in sys.argv, verbose=True)
+    else:                                # the library and what calls it: never one of the two alone
+        force = "--incremental" not in args
+        with ThreadPoolExecutor(max_workers=1) as pool:
+            host = pool.submit(build_host, verbose=True, force=force)
+            build(force=force, verbose=True)
+            host.result()
+
+
+if __name__ == "__main__":
+    main(sys.argv[1:])

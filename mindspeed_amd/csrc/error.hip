@@ -6,6 +6,11 @@
 #include <utility>
 
 #include "common.h"
+#include "internal.h"
+
+#ifndef MS_INTERFACE
+#error "MS_INTERFACE: the hash of the declared entry points, as build.py defines it"
+#endif
 
 namespace ms {
 namespace {
@@ -35,3 +40,4 @@ hipError_t set_max_dynamic_lds(const void *fn, int bytes) {
 
 extern "C" const char *ms_last_error(void) { return ms::g_error; }
 extern "C" int ms_version(void) { return 104; }
+extern "C" const char *msi_interface(void) { return MS_INTERFACE; }

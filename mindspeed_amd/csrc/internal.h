@@ -8,6 +8,9 @@
 extern "C" {
 #endif
 
+/* The hash of these declarations and of those in mindspeed_amd.h that the library was built from (build.py: interface_hash):
+ * what a binding that passes arguments by them compares with its own before its first call. */
+const char *msi_interface(void);
 /* ms_moe_routing_map_permute and ms_moe_routing_map_probs in one: permuted_probs [num_rows] in the dtype of probs (both may
  * be NULL) and sorted_token_ids [num_rows] (may be NULL) are written beside the rows; rows that no map entry leads to get
  * zeros. */

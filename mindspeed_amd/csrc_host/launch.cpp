@@ -61,9 +61,13 @@ void bind(const std::string &path, py::object error) {
     if (lib == nullptr) throw std::runtime_error(dlerror());
     auto find = [&](const char *name) {
         void *fn = dlsym(lib, name);
-        if (fn == nullptr) throw std::runtime_error(std::string(path) + " lacks " + name);
+        if (fn == nullptr) throw std::runtime_error(path + " lacks " + name + ": rebuild it with `python -m mindspeed_amd.build`");
         return fn;
     };
+    const std::string theirs = reinterpret_cast<decltype(&msi_interface)>(find("msi_interface"))();
+    if (theirs != MS_INTERFACE)
+        throw std::runtime_error("_host.so was built for entry points " MS_INTERFACE ", " + path + " has " + theirs +
+                                 ": rebuild both with `python -m mindspeed_amd.build`");
 #define MS_FIND(name) api.name = reinterpret_cast<decltype(&::name)>(find(#name));
     MS_FIND(ms_last_error)
     MS_FIND(ms_gmm_workspace_size)

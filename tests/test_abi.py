@@ -193,3 +193,65 @@ def test_launch_has_slots_for_every_table_the_schedule_can_write():
     assert with_lists > 300 and fullest > 0.95           # the lists were met, and the bound is nearly reached
     assert lib.ms_gmm_launch_slots(0, 1, 1, 1, 0, 0, 0, ctypes.byref(slots)) != 0
     assert lib.ms_gmm_launch_slots(8, 1, 1, 1, 1, 0, 0, ctypes.byref(slots)) != 0
+
+
+def _stub(path, interface, version=_lib.ABI_VERSION):
+    """A library with every name that this package binds, built from other declarations."""
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    names = (set(_lib._SIGNATURES) | set(_lib._INTERNAL) | {"ms_last_error"}) - {"ms_version"}
+    code = "".join(f"int {n}(void) {{ return 0; }}\n" for n in sorted(names))
+    code += f"int ms_version(void) {{ return {version}; }}\n"
+    if interface is not None:
+        code += f'const char *msi_interface(void) {{ return "{interface}"; }}\n'
+    subprocess.run([cc, "-shared", "-fPIC", "-x", "c", "-", "-o", str(path)], input=code, text=True, check=True)
+    return str(path)
+
+
+@pytest.mark.parametrize("interface", ["0123456789abcdef", None])
+def test_the_native_side_refuses_a_library_of_other_declarations(interface, tmp_path):
+    """_host.so passes arguments by the declarations it was compiled with: another build's may differ in them without a name
+    missing."""
+    lib = _stub(tmp_path / "other.so", interface)
+    code = f"import torch; from mindspeed_amd import _host; _host.bind({lib!r}, RuntimeError)"
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
+    assert res.returncode != 0 and "rebuild" in res.stderr, res.stderr
+    # ... and the library of this tree is the one it was built with
+    code = "import torch; from mindspeed_amd import _host, _lib; _host.bind(_lib.LIB_PATH, RuntimeError); print('bound')"
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
+    assert res.returncode == 0 and "bound" in res.stdout, res.stderr
+
+
+@pytest.mark.parametrize("interface", ["0123456789abcdef", None])
+def test_the_python_binding_refuses_a_library_of_other_declarations(interface, tmp_path):
+    lib = _stub(tmp_path / "other.so", interface)
+    res = subprocess.run([sys.executable, "-c", "from mindspeed_amd import _lib; _lib.load()"], capture_output=True, text=True,
+                         cwd=ROOT, env=dict(os.environ, MINDSPEED_AMD_LIB=lib))
+    assert res.returncode != 0 and "rebuild it" in res.stderr, res.stderr
+
+
+def test_the_interface_hash_follows_declarations_and_not_comments(tmp_path, monkeypatch):
+    from mindspeed_amd import build
+    copies = []
+    for f in build.INTERFACE_HEADERS:
+        copies.append(str(tmp_path / os.path.basename(f)))
+        shutil.copy(f, copies[-1])
+    before = build.interface_hash()
+    monkeypatch.setattr(build, "INTERFACE_HEADERS", tuple(copies))
+    assert build.interface_hash() == before and _lib.load().msi_interface().decode() == before
+    text = open(copies[1]).read()
+    open(copies[1], "w").write("/* a comment */\n\n" + text + "// and another\n")
+    assert build.interface_hash() == before
+    open(copies[1], "w").write(text.replace("int drop_and_pad", "int64_t drop_and_pad"))
+    assert build.interface_hash() != before
+
+
+@pytest.mark.parametrize("args,force", [([], True), (["--incremental"], False)])
+def test_the_build_command_makes_the_library_and_its_native_side(args, force, monkeypatch):
+    from mindspeed_amd import build
+    made = []
+    monkeypatch.setattr(build, "build", lambda force, verbose: made.append(("library", force)))
+    monkeypatch.setattr(build, "build_host", lambda verbose, force: made.append(("host", force)))
+    build.main(args)
+    assert sorted(made) == [("host", force), ("library", force)]
