@@ -47,11 +47,11 @@ def sources():
 
 
 def source_hash() -> str:
-    """First 16 hex digits of the SHA-256 over the kernel sources (csrc/*.hip, csrc/*.h, the C-ABI header) in name
-    order: names the build that measured figures (profiles/*.json) belong to."""
+    """First 16 hex digits of the SHA-256 over the kernel sources and the native side of the ops (csrc/*.hip, csrc/*.h, the
+    C-ABI header, csrc_host/launch.cpp) in name order: names the build that measured figures (profiles/*.json) belong to."""
     h = hashlib.sha256()
     files = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h")))
-    files.append(os.path.join(HERE, "..", "include", "mindspeed_amd.h"))
+    files += [os.path.join(HERE, "..", "include", "mindspeed_amd.h"), HOST_SRC]
     for f in files:
         h.update(os.path.basename(f).encode())
         with open(f, "rb") as fh:

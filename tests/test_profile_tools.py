@@ -68,6 +68,17 @@ def test_source_hash_follows_the_kernel_sources(tmp_path, monkeypatch):
     assert build.source_hash() != before
 
 
+def test_source_hash_follows_the_native_side_of_the_ops(tmp_path, monkeypatch):
+    """A changed csrc_host/launch.cpp is another build too: small steps are bound by it."""
+    before = build.source_hash()
+    copy = tmp_path / os.path.basename(build.HOST_SRC)
+    copy.write_bytes(open(build.HOST_SRC, "rb").read())
+    monkeypatch.setattr(build, "HOST_SRC", str(copy))
+    assert build.source_hash() == before
+    copy.write_bytes(copy.read_bytes() + b"// changed\n")
+    assert build.source_hash() != before
+
+
 @pytest.mark.gpu
 def test_tile_timeline_on_the_diagnostic_build():
     """The diagnostic build records one time-stamp record per tile: 14336 tiles of the weight-gradient product, each
