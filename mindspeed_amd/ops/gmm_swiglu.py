@@ -112,11 +112,14 @@ def _swiglu_grad_from_fc1(dact, fc1, p):
     return d_fc1, (gp if p is not None else None)
 
 
-def _require_vector_layout(dy, w2, fc1):
-    """The layout conditions of the fused kernels on what the backward pass brings in."""
-    if not _tracing(dy) and (dy.size(1) % 8 or fc1.size(1) % 16 or any(t.data_ptr() % 16 for t in (dy, w2, fc1))):
-        raise _lib.MindSpeedAmdError("grouped_mlp: the fused kernels need the vector-access layout (16-byte aligned "
-                                     "operands, hidden and ffn multiples of 8)")
+def _vector_rows(w):
+    """``w [E, R, C]``, copied where the fast grouped matmul could not read it as it lies (an unaligned base, rows off the
+    16-byte grid, no unit stride).  A transposed view is read in place: a copy of it would be the whole weights."""
+    rows, cols = w.stride(1), w.stride(2)
+    if not _tracing(w) and w.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0 and \
+            ((cols == 1 and rows % 8 == 0) or (rows == 1 and cols % 8 == 0)):
+        return w
+    return w.contiguous()
 
 
 class GroupedMLPFunction(torch.autograd.Function):
@@ -183,8 +186,7 @@ class GroupedMLPFunction(torch.autograd.Function):
             if dw2 is not None:
                 gmm_raw(act.t(), dy, gl, 2, glt, out=dw2)
         if ctx.fused_kernels:
-            w2 = w2.contiguous()
-            _require_vector_layout(dy, w2, fc1)
+            w2 = _vector_rows(w2)
         dact = gmm_raw(dy, w2.transpose(1, 2), gl, 0, glt)
         d_fc1, gp = _swiglu_grad_from_fc1(dact, fc1, p)
         del dact

@@ -187,6 +187,60 @@ def _grouped_mlp_case(counts, K, ffn, dtype, pdt, extra, recompute, fused_kernel
         assert rel_l2(pf.grad, p64.grad) <= tol
 
 
+@pytest.mark.parametrize("name", ["grad_out_off_the_grid", "w2_transposed", "w2_off_the_grid", "hidden_out_36"])
+def test_grouped_mlp_backward_takes_any_layout(name, device):
+    """The backward pass runs the separate kernels, which take what the fused forward does not look at: a gradient that starts
+    off the 16-byte grid, second weights of any layout and width."""
+    say("grouped_mlp backward layout", name)
+    counts, K, ffn, dtype = [33, 0, 70, 9], 64, 128, torch.bfloat16
+    Ko = 36 if name == "hidden_out_36" else 64
+    E, M = len(counts), sum(counts)
+    gen = torch.Generator().manual_seed(31)
+    x = torch.randn(M, K, generator=gen).to(dtype)
+    w1 = (torch.randn(E, K, 2 * ffn, generator=gen) * 0.1).to(dtype)
+    w2 = (torch.randn(E, ffn, Ko, generator=gen) * 0.1).to(dtype)
+    probs = torch.rand(M, generator=gen) + 0.25
+    gy = torch.randn(M, Ko, generator=gen).to(dtype)
+    gl = torch.tensor(counts, dtype=torch.int64)
+
+    def off_the_grid(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=device)[1:]
+        return flat.view(t.shape).copy_(t)
+    w2d, gyd = w2.to(device), gy.to(device)
+    if name == "grad_out_off_the_grid":
+        gyd = off_the_grid(gy)
+    elif name == "w2_transposed":
+        w2d = w2d.transpose(1, 2).contiguous().transpose(1, 2)
+    elif name == "w2_off_the_grid":
+        w2d = off_the_grid(w2)
+    leaves = [t.requires_grad_(True) for t in (x.to(device), w1.to(device), w2d.detach(), probs.to(device))]
+    out = ops.grouped_mlp(leaves[0], leaves[1], leaves[2], gl.to(device), leaves[3])
+    grads = torch.autograd.grad(out, leaves, gyd)
+    exact = [t.double().requires_grad_(True) for t in (x, w1, w2, probs)]
+    fc1 = O.gmm(exact[0], exact[1], gl, group_type=0, group_list_type=1)
+    want = O.gmm(O.swiglu(fc1, exact[3]), exact[2], gl, group_type=0, group_list_type=1)
+    for got, ref in zip((out, *grads), (want, *torch.autograd.grad(want, exact, gy.double()))):
+        assert got.shape == ref.shape and rel_l2(got, ref) <= 1e-2
+
+
+def test_grouped_mlp_backward_reads_transposed_weights_in_place(device):
+    """No copy of the second weights where they are a transposed view: the peak of a backward pass to x alone stays below it."""
+    E, M, K, ffn = 8, 64, 256, 4096
+    x = torch.randn(M, K, device=device).to(torch.bfloat16).requires_grad_(True)
+    w1 = torch.randn(E, K, 2 * ffn, device=device).to(torch.bfloat16)
+    w2 = torch.randn(E, K, ffn, device=device).to(torch.bfloat16).transpose(1, 2)
+    out = ops.grouped_mlp(x, w1, w2, torch.full((E,), M // E, device=device))
+    gy = torch.randn_like(out)
+    torch.autograd.grad(out, x, gy, retain_graph=True)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats(device)
+    before = torch.cuda.memory_allocated(device)
+    torch.autograd.grad(out, x, gy)
+    torch.cuda.synchronize()
+    # (dact, d_fc1, dx and the tile tables: 2 MB; the weights: 16 MB)
+    assert torch.cuda.max_memory_allocated(device) - before < w2.numel() * w2.element_size() // 2
+
+
 def test_inference_skips_the_fc1_output(device):
     """Under ``torch.no_grad()`` the fused forward does not store the fc1 output (the kernel's NULL-output form):
     the activation and the MLP output are bit for bit those of the differentiable call."""
