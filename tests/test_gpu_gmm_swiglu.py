@@ -8,6 +8,8 @@ from oracle import moe_oracle as O
 
 import mindspeed_amd.ops as ops
 from mindspeed_amd.dispatcher import dispatch_mlp_combine, experts_computation
+from mindspeed_amd.ops._kernels import K as K_
+from mindspeed_amd.ops.gmm import gmm_raw
 
 pytestmark = pytest.mark.gpu
 
@@ -24,7 +26,7 @@ CASES = [
     ([300, 212], 72, 136, torch.float16, torch.float32, 0),
     ([1024, 1000, 1048], 512, 1024, torch.bfloat16, torch.float32, 0),       # full tiles, many rounds
     ([40], 8, 8, torch.bfloat16, torch.float32, 0),                          # smallest legal sizes
-    # many small groups with enough tiles for several rounds: whole groups go to single XCDs (per-XCD lists)
+    # more entries than a table's header names, every group with a small tail tile, rows past the last offset
     ([520 + 13 * (i % 7) for i in range(32)], 256, 768, torch.bfloat16, torch.float32, 9),
 ]
 
@@ -112,7 +114,7 @@ MLP_CASES = [
     ([130, 256, 1, 300, 64, 0, 200, 73], 256, 384, torch.bfloat16, torch.bfloat16, 5),
     ([300, 212], 72, 136, torch.float16, torch.float32, 0),
     ([700, 1000, 348], 512, 1024, torch.bfloat16, torch.float32, 0),
-    # many small groups: per-XCD lists in the fused kernels, forward and backward
+    # many small groups of two row tiles, the second nearly full or a small one
     ([430 + 17 * (i % 5) for i in range(24)], 256, 512, torch.bfloat16, torch.float32, 6),
 ]
 
@@ -169,11 +171,8 @@ def _grouped_mlp_case(counts, K, ffn, dtype, pdt, extra, recompute, fused_kernel
     assert torch.equal(out, out_sep)
     assert torch.equal(xf.grad, xs.grad)                   # d_fc1 is bit-identical, so everything behind it is
     assert torch.equal(w1f.grad, w1s.grad) and torch.equal(w2f.grad, w2s.grad)
-    if probs is not None and fused_kernels:
-        # same terms, summed per 64 columns and then over the row instead of in one pass
-        assert rel_l2(pf.grad, ps.grad) <= (1e-5 if pdt == torch.float32 else 1e-2)
-    elif probs is not None:
-        assert torch.equal(pf.grad, ps.grad)               # the very same kernel
+    if probs is not None:
+        assert torch.equal(pf.grad, ps.grad)               # the very same kernel, with fused_kernels or without
 
     x64, w164, w264 = (t.double().requires_grad_(True) for t in (x, w1, w2))
     p64 = None if probs is None else probs.double().requires_grad_(True)
@@ -185,6 +184,35 @@ def _grouped_mlp_case(counts, K, ffn, dtype, pdt, extra, recompute, fused_kernel
     assert rel_l2(w1f.grad, w164.grad) <= tol and rel_l2(w2f.grad, w264.grad) <= tol
     if probs is not None:
         assert rel_l2(pf.grad, p64.grad) <= tol
+
+
+@pytest.mark.parametrize("counts,K,ffn,dtype,pdt,extra", MLP_CASES)
+def test_swiglu_backward_in_the_epilogue(counts, K, ffn, dtype, pdt, extra, device):
+    """``ms_gmm_swiglu_grad``, which the package's own backward does not use (its separate kernels are faster): bit for bit the
+    d_fc1 of those kernels and the probabilities' gradient up to the order of its sums, both against 64 bits."""
+    say("gmm_swiglu_grad case", counts, K, ffn, dtype, pdt, extra)
+    E, M = len(counts), sum(counts) + extra
+    gen = torch.Generator().manual_seed(M + ffn + 2)
+    dy = torch.randn(M, K, generator=gen).to(dtype)
+    w2 = (torch.randn(E, ffn, K, generator=gen) * 0.1).to(dtype)
+    fc1 = torch.randn(M, 2 * ffn, generator=gen).to(dtype)
+    probs = None if pdt is None else (torch.rand(M, generator=gen) + 0.25).to(pdt)
+    gl = torch.tensor(counts, dtype=torch.int64)
+    dyd, w2d, fc1d, gld = (t.to(device) for t in (dy, w2, fc1, gl))
+    pd = None if probs is None else probs.to(device)
+    for kind, lst in ((1, gld), (0, gld.cumsum(0))):
+        d_fc1, gp = K_.gmm_swiglu_grad(dyd, w2d, fc1d, pd, lst, kind)
+        d_sep, gp_sep = K_.swiglu_grad(gmm_raw(dyd, w2d.transpose(1, 2), lst, 0, kind), fc1d, pd)
+        assert torch.equal(d_fc1, d_sep)
+        if pd is not None:
+            # the same fp32 terms, summed per 64 columns and then over the row instead of in one pass, one rounding to pdt
+            assert gp.dtype == pdt and rel_l2(gp, gp_sep) <= (1e-5 if pdt == torch.float32 else 1e-2)
+    fc1_64 = fc1.double().requires_grad_(True)
+    p64 = None if probs is None else probs.double().requires_grad_(True)
+    O.gmm(O.swiglu(fc1_64, p64), w2.double(), gl, group_type=0, group_list_type=1).backward(dy.double())
+    assert rel_l2(d_fc1, fc1_64.grad) <= 1e-2
+    if pd is not None:
+        assert rel_l2(gp, p64.grad) <= 1e-2
 
 
 @pytest.mark.parametrize("name", ["grad_out_off_the_grid", "w2_transposed", "w2_off_the_grid", "hidden_out_36"])
