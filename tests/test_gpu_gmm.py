@@ -99,7 +99,7 @@ GMM_CASES = [
     # forward (4 + 5), 5 x 10 in the weight gradient (one block of 5), and a ragged pair of groups with 5 row tiles each
     (2300, 1280, 2560, 1, "equal"),
     (2100, 768, 1024, 2, "equal"),
-    # many groups of a few row tiles each: whole groups go to single XCDs (lists per XCD) in forward and dX
+    # many groups of a few row tiles each, in fewer rounds of tiles than whole groups are dealt out to XCDs from
     (32768, 256, 1280, 64, "equal"),
     (20000, 320, 768, 24, "equal"),
 ]
@@ -139,7 +139,7 @@ def test_forward_and_backward_vs_oracle(M, K, N, E, kind, dtype, device):
 @pytest.mark.parametrize("E,empty,K,N,rows", [
     (17, (16,), 2048, 4096, 256),          # 16 groups of 256 rows and one empty: the XCD with three groups has 3 x 128 tiles
     (20, (3, 8, 13, 19), 2880, 2880, 192),  # 16 + 4 empty, 12 x 12 output tiles per group
-    (23, (), 1024, 2048, 128),             # no empty group; 23 groups deal out as 3, 3, 3, 3, 3, 3, 3, 2
+    (23, (), 1024, 2048, 128),             # no empty group, few rounds of tiles: found in the group list instead
 ])
 def test_weight_gradient_group_count_not_a_multiple_of_8(E, empty, K, N, rows, device):
     """Split on the reduction dim with whole groups dealt out to single XCDs: the XCD with the most groups holds
@@ -288,7 +288,7 @@ def test_groupmatmul_add_reduction_lengths(K, N, dtype, device):
 
 
 def test_groupmatmul_add_many_groups(device):
-    """The fp32 `+=` form with 24 near-equal groups (whole output blocks dealt out to single XCDs)."""
+    """The fp32 `+=` form with 24 near-equal groups."""
     say("groupmatmul_add many groups")
     counts = [200 + 9 * (i % 7) for i in range(24)]
     M, K, N = sum(counts), 512, 520
@@ -466,8 +466,9 @@ def test_split_tail_tiles_with_rows_past_the_last_offset(device):
 
 
 def test_many_small_groups_take_whole_groups_per_xcd(device):
-    """Near-equal ragged groups of two to five row tiles, 40 of them, and rows past the last offset: the launch deals
-    whole groups out to single XCDs; forward, dX and dW against the oracle, the uncovered rows zero."""
+    """Near-equal ragged groups of two to five row tiles, 40 of them, and rows past the last offset; forward, dX and dW against
+    the oracle, the uncovered rows zero.  (Fewer than six rounds of tiles: launches that do deal whole groups out to single
+    XCDs are in test_gpu_gmm_whole_groups.py.)"""
     say("many small groups")
     gen = torch.Generator().manual_seed(21)
     E, K, N, extra = 40, 384, 1536, 300
@@ -566,7 +567,7 @@ def test_large_tiles_over_reduction_lengths_beside_bad_rows(bad, dtype, device):
         else:
             exp[e] = x[end - n:end].t() @ g[end - n:end]
     xd, gd, start = put(x), put(g), ints(*exp.shape)
-    for n in (lengths.numel(), 13):                       # with whole groups dealt out to single XCDs, and without
+    for n in (lengths.numel(), 13):                       # more groups than a table's header names, and fewer
         dw = ops.npu_gmm_v2(xd.t(), gd, group_list=lengths[:n].to(device), group_type=2)
         assert torch.equal(dw[::2].cpu().double(), exp[:n:2])
         acc = start[:n].float().to(device)
