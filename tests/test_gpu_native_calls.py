@@ -1,6 +1,7 @@
 """The native side of the ops (csrc_host/launch.cpp) against the Python functions of the same names: equal results, equal
 errors, and the same calls left to the dispatcher."""
 import threading
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -12,44 +13,58 @@ from mindspeed_amd.ops._kernels import K
 pytestmark = pytest.mark.gpu
 
 
-def _calls():
+def _inputs():
     gen = torch.Generator(device="cuda").manual_seed(1)
     r = lambda *s, dtype=torch.bfloat16: torch.randn(*s, generator=gen, device="cuda").to(dtype)
-    counts = torch.tensor([30, 0, 64, 6], device="cuda")
-    x, w, dy = r(100, 64), r(4, 64, 128), r(100, 128)
-    tokens, index = r(50, 72), torch.randint(0, 4, (50, 2), generator=gen, device="cuda")
-    permuted, rid, _, _ = kernels._permute(tokens, index, 100, 4, False, False)
-    probs = torch.rand(50, 2, generator=gen, device="cuda")
-    rmap = torch.rand(50, 6, generator=gen, device="cuda") < 0.4
-    rows = int(rmap.sum()) + 3
-    mperm, mrid, mflat, _, _ = kernels._routing_map_permute_probs(tokens, rmap, None, rows, False)
-    mprobs = torch.rand(50, 6, generator=gen, device="cuda")
-    out, acc = torch.zeros(4, 64, 128, device="cuda"), torch.ones(4, 64, 128, device="cuda")
-    return [("gmm", x, w, counts, 0, 1), ("gmm", x.float(), w.float(), counts.cumsum(0), 0, 0), ("gmm", x.t(), dy, counts, 2, 1),
-            ("gmm", dy, w.transpose(1, 2), counts, 0, 1),
-            ("gmm_out", x.t(), dy, counts, 2, 1, out, False), ("gmm_out", x.t(), dy, counts, 2, 1, acc, True),
-            ("gmm_swiglu", x, w, counts, 1, None, True), ("gmm_swiglu", x, w, counts, 1, torch.rand(100, device="cuda"), False),
-            ("moe_token_permute", tokens, index, 100, 4, True, True), ("moe_token_permute", tokens, index.int(), 90, 0, False, True),
-            ("moe_token_permute", tokens, index[:, 0].contiguous(), 50, 4, False, False),
-            ("moe_token_permute_grad", permuted, rid, 50, 2),
-            ("moe_token_unpermute", permuted, rid, None, 50, 2), ("moe_token_unpermute", permuted, rid, probs.half(), 50, 2),
-            ("moe_token_unpermute_grad", permuted, tokens, rid, probs, 50, 2, 100),
-            ("moe_token_unpermute_grad", permuted, tokens, rid, probs.half(), 50, 2, 100),
-            ("moe_token_unpermute_grad", mperm, tokens, mrid, mprobs, 50, 6, rows, mflat),
-            ("moe_token_unpermute_grad", permuted, tokens, rid, None, 50, 2, 130),
-            ("swiglu", dy, None), ("swiglu", dy, torch.rand(100, device="cuda")), ("swiglu_grad", x, dy, None),
-            ("swiglu_grad", x, dy, torch.rand(100, device="cuda").half()),
-            ("routing_map_permute_probs", tokens, rmap, mprobs, rows, False), ("routing_map_permute_probs", tokens, rmap, None, rows, False),
-            ("routing_map_probs_grad", mrid, torch.rand(rows, device="cuda"), 50, 6)]
+    u = lambda *s: torch.rand(*s, generator=gen, device="cuda")
+    i = SimpleNamespace(counts=torch.tensor([30, 0, 64, 6], device="cuda"), x=r(100, 64), w=r(4, 64, 128), dy=r(100, 128),
+                        tokens=r(50, 72), index=torch.randint(0, 4, (50, 2), generator=gen, device="cuda"), probs=u(50, 2),
+                        rmap=u(50, 6) < 0.4, mprobs=u(50, 6), p100=u(100), out=torch.zeros(4, 64, 128, device="cuda"),
+                        acc=torch.ones(4, 64, 128, device="cuda"))
+    i.permuted, i.rid, _, _ = kernels._permute(i.tokens, i.index, 100, 4, False, False)
+    i.rows = int(i.rmap.sum()) + 3
+    i.mperm, i.mrid, i.mflat, _, _ = kernels._routing_map_permute_probs(i.tokens, i.rmap, None, i.rows, False)
+    i.gp = u(i.rows)
+    return i
+
+
+# (op, its arguments out of _inputs()): nothing runs on the device while the tests are collected
+CALLS = {
+    "gmm": lambda i: ("gmm", i.x, i.w, i.counts, 0, 1),
+    "gmm_fp32_offsets": lambda i: ("gmm", i.x.float(), i.w.float(), i.counts.cumsum(0), 0, 0),
+    "gmm_reduction": lambda i: ("gmm", i.x.t(), i.dy, i.counts, 2, 1),
+    "gmm_transposed": lambda i: ("gmm", i.dy, i.w.transpose(1, 2), i.counts, 0, 1),
+    "gmm_out": lambda i: ("gmm_out", i.x.t(), i.dy, i.counts, 2, 1, i.out, False),
+    "gmm_out_accumulate": lambda i: ("gmm_out", i.x.t(), i.dy, i.counts, 2, 1, i.acc, True),
+    "gmm_swiglu": lambda i: ("gmm_swiglu", i.x, i.w, i.counts, 1, None, True),
+    "gmm_swiglu_probs_no_fc1": lambda i: ("gmm_swiglu", i.x, i.w, i.counts, 1, i.p100, False),
+    "permute": lambda i: ("moe_token_permute", i.tokens, i.index, 100, 4, True, True),
+    "permute_int32": lambda i: ("moe_token_permute", i.tokens, i.index.int(), 90, 0, False, True),
+    "permute_top1": lambda i: ("moe_token_permute", i.tokens, i.index[:, 0].contiguous(), 50, 4, False, False),
+    "permute_grad": lambda i: ("moe_token_permute_grad", i.permuted, i.rid, 50, 2),
+    "unpermute": lambda i: ("moe_token_unpermute", i.permuted, i.rid, None, 50, 2),
+    "unpermute_probs": lambda i: ("moe_token_unpermute", i.permuted, i.rid, i.probs.half(), 50, 2),
+    "unpermute_grad": lambda i: ("moe_token_unpermute_grad", i.permuted, i.tokens, i.rid, i.probs, 50, 2, 100),
+    "unpermute_grad_half_probs": lambda i: ("moe_token_unpermute_grad", i.permuted, i.tokens, i.rid, i.probs.half(), 50, 2, 100),
+    "unpermute_grad_marked": lambda i: ("moe_token_unpermute_grad", i.mperm, i.tokens, i.mrid, i.mprobs, 50, 6, i.rows, i.mflat),
+    "unpermute_grad_more_rows": lambda i: ("moe_token_unpermute_grad", i.permuted, i.tokens, i.rid, None, 50, 2, 130),
+    "swiglu": lambda i: ("swiglu", i.dy, None),
+    "swiglu_probs": lambda i: ("swiglu", i.dy, i.p100),
+    "swiglu_grad": lambda i: ("swiglu_grad", i.x, i.dy, None),
+    "swiglu_grad_probs": lambda i: ("swiglu_grad", i.x, i.dy, i.p100.half()),
+    "routing_map_permute": lambda i: ("routing_map_permute_probs", i.tokens, i.rmap, i.mprobs, i.rows, False),
+    "routing_map_permute_no_probs": lambda i: ("routing_map_permute_probs", i.tokens, i.rmap, None, i.rows, False),
+    "routing_map_probs_grad": lambda i: ("routing_map_probs_grad", i.mrid, i.gp, 50, 6),
+}
 
 
 def _flat(result):
     return [result] if isinstance(result, torch.Tensor) else list(result)
 
 
-@pytest.mark.parametrize("i", range(len(_calls()) if torch.cuda.is_available() else 25))
-def test_equals_the_python_function(i):
-    name, *args = _calls()[i]
+@pytest.mark.parametrize("case", CALLS)
+def test_equals_the_python_function(case):
+    name, *args = CALLS[case](_inputs())
     native = (kernels._native if kernels._native is not None else kernels._load_native())[name]
     clones = [a.clone(memory_format=torch.preserve_format) if isinstance(a, torch.Tensor) else a for a in args]
     want, got = kernels._DEVICE_FNS[name](*clones), native(*args)
@@ -93,7 +108,7 @@ def test_which_calls_are_plain():
 
 
 def test_a_recorder_still_sees_the_calls():
-    name, *args = _calls()[0]
+    name, *args = CALLS["gmm"](_inputs())
     with flop_counter.record(timing=False) as rec:
         K.gmm(*args)
     assert [c[0] for c in rec.calls] == ["gmm_fwd"]
@@ -101,7 +116,7 @@ def test_a_recorder_still_sees_the_calls():
 
 def test_current_stream_and_threads():
     """Every call goes to the caller's current stream, also from several threads at once."""
-    name, *args = _calls()[0]
+    name, *args = CALLS["gmm"](_inputs())
     want = K.gmm(*args)
     torch.cuda.synchronize()
     out = {}
