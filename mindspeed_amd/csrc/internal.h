@@ -13,7 +13,7 @@ extern "C" {
 const char *msi_interface(void);
 /* ms_moe_routing_map_permute and ms_moe_routing_map_probs in one: permuted_probs [num_rows] in the dtype of probs (both may
  * be NULL) and sorted_token_ids [num_rows] (may be NULL) are written beside the rows; rows that no map entry leads to get
- * zeros. */
+ * zeros.  Without tokens neither may be asked for. */
 int msi_routing_map_permute(ms_stream_t stream, const void *tokens, const void *routing_map, int64_t num_tokens,
                             int64_t num_experts, int64_t hidden, int dtype, int64_t num_rows, int drop_and_pad,
                             void *permuted, int32_t *row_id_map, int32_t *sorted_flat, int64_t *tokens_per_expert,

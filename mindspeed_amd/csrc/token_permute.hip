@@ -1962,13 +1962,9 @@ extern "C" int msi_routing_map_permute(ms_stream_t stream_, const void *tokens, 
     MS_REQUIRE(num_rows == 0 || (probs == nullptr) == (permuted_probs == nullptr), MS_ERR_INVALID_ARGUMENT,
                "%s: probs and permuted_probs must be given together", fn);
     if (T == 0) return MS_OK;
-    if (tokens == nullptr && num_rows > 0 && (permuted_probs != nullptr || sorted_token_ids != nullptr)) {
-        // maps only: the kernels' workgroups hold many tokens then, and their LDS has no room for the rows beside
-        if (int rc = ms_moe_routing_map_permute(stream_, nullptr, routing_map, T, E, H, dtype, num_rows, drop_and_pad, permuted,
-                                                row_id_map, sorted_flat, tokens_per_expert, workspace, workspace_bytes))
-            return rc;
-        return launch_routing_map_probs(stream, sorted_flat, num_rows, E, probs, probs_dtype, permuted_probs, sorted_token_ids);
-    }
+    // (without tokens the kernels' workgroups hold many positions each, and their LDS has no room for the rows of these beside)
+    MS_REQUIRE(num_rows == 0 || tokens != nullptr || (permuted_probs == nullptr && sorted_token_ids == nullptr), MS_ERR_UNSUPPORTED,
+               "%s: probabilities and token numbers come with the rows only", fn);
     const RowExtras extras{probs, num_rows > 0 ? permuted_probs : nullptr, num_rows > 0 ? sorted_token_ids : nullptr,
                            probs_dtype == MS_FP32 ? 4 : 2};
     MS_REQUIRE(routing_map && row_id_map && (sorted_flat || num_rows == 0), MS_ERR_INVALID_ARGUMENT,

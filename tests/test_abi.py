@@ -91,6 +91,10 @@ def test_workspace_size_and_validation_are_host_only():
     assert rc != 0 and b"topk" in lib.ms_last_error()
     with pytest.raises(_lib.MindSpeedAmdError):
         _lib.check(rc, "ms_moe_token_unpermute")
+    # probabilities and token numbers of routing-map rows come with the rows (no pointer here is ever followed)
+    for probs, permuted_probs, ids in ((64, 64, None), (None, None, 64)):
+        rc = lib.msi_routing_map_permute(None, None, 64, 4, 2, 8, BF16, 4, 0, None, 64, 64, None, probs, FP32, permuted_probs, ids, 64, 1 << 20)
+        assert rc != 0 and b"with the rows only" in lib.ms_last_error()
 
 
 def test_tile_order_visits_every_tile_once():
