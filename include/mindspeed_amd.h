@@ -266,7 +266,9 @@ int ms_gmm_swiglu(ms_stream_t stream, const void *x, int64_t x_stride0, int64_t 
  * with gate = fc1[r, c], up = fc1[r, ffn + c] and dact rounded to dtype first, i.e. the values
  * ms_gmm followed by ms_swiglu_grad produce.  dy [m, k]; weight is the transposed view of
  * W2 [num_groups, ffn, k] (w_stride0 = 1 along k, w_stride1 = k along ffn); fc1 / d_fc1 [m, 2*ffn];
- * probs / grad_probs optional together.  Same layout conditions as ms_gmm_swiglu. */
+ * probs / grad_probs optional together.  Same layout conditions as ms_gmm_swiglu.  It saves the dact
+ * buffer, not time: ms_gmm and ms_swiglu_grad one after the other are faster (16 groups of 768 rows,
+ * 2048 x 1536: 114 against 142 us), and the Python surface runs those. */
 int ms_gmm_swiglu_grad_workspace_size(int64_t num_groups, int64_t m, int64_t ffn, size_t *bytes);
 int ms_gmm_swiglu_grad(ms_stream_t stream, const void *dy, int64_t dy_stride0, int64_t dy_stride1,
                        const void *weight, int64_t w_stride_group, int64_t w_stride0, int64_t w_stride1,

@@ -83,7 +83,7 @@ struct GmmArgs {
     int64_t b_stride_group, c_stride_group;
     int group_list_type, group_type, num_groups;
     int m, k;
-    int tile_rows;              // rows per full tile: 64, 128 or 256
+    int tile_rows;              // rows per full tile, a power of two: 256 for 16-bit operands; 32, 64 or 128 in fp32
     int small_tails;            // a group's last row tile may be a smaller one
     int tails_last_below;       // launches of fewer tiles take their small tiles last
     int part_cus;               // compute units if the last round may be divided (LastRound), else 0

@@ -468,7 +468,8 @@ _define("gmm_swiglu(Tensor x, Tensor weight, Tensor group_list, int group_list_t
 
 def _gmm_swiglu_grad(dy, w2, fc1, probs, group_list, group_list_type):
     """``d_fc1`` (and the probabilities' gradient) from ``dy``: the dX product of the second matmul with the SwiGLU
-    backward on the saved ``fc1`` in its epilogue.  ``w2 [E, ffn, hidden]`` contiguous."""
+    backward on the saved ``fc1`` in its epilogue.  ``w2 [E, ffn, hidden]`` contiguous.  Saves the ``dact`` buffer;
+    ``GroupedMLPFunction`` runs the two kernels apart, which is faster."""
     lib = _lib.load()
     dev = dy.device
     m, two_ffn = fc1.shape
