@@ -181,8 +181,8 @@ def threads_on_one_core():
     the main thread issues the forward pass, then waits while torch's autograd thread issues the backward pass — so
     nothing is lost, and the core never goes idle between the two hand-overs of a step.  With the threads on different
     cores each hand-over wakes an idle core, which on these hosts costs about 70 us: the small configuration's step
-    reads 0.43-0.45 ms that way and 0.29-0.32 ms on one core (whichever placement the scheduler picks decides the
-    figure otherwise: runs of the same loop switch between the two)."""
+    reads 0.27 ms as the scheduler places the threads and 0.17 ms on one core.  (The core is the lowest of
+    the process's share; on another host the step read 0.28 ms and, confined to it, 0.41 ms.)"""
     saved = {}
     for name in os.listdir("/proc/self/task"):
         try:
@@ -534,7 +534,7 @@ def main():
                 ms1, _, _, _ = run_layer(ocfg, device, steps=300, warmup=100, per_kernel=False)
             others[name]["ms_per_step_threads_on_one_core"] = round(ms1, 4)
             others[name]["note"] = ("ms_per_step: threads placed by the scheduler; the step is host-bound and reads "
-                                    "0.27-0.45 ms depending on whether the main and the autograd thread share a core")
+                                    "0.17-0.41 ms depending on the host and on whether the main and the autograd thread share a core")
 
     def graph_section():
         others["plumbing"]["graph_replay_ms_per_step"] = graph_replay_ms(WORKLOADS["plumbing"], device)
