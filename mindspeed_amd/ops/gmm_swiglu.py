@@ -113,8 +113,8 @@ def _swiglu_grad_from_fc1(dact, fc1, p):
 
 
 def _vector_rows(w):
-    """``w [E, R, C]``, copied where the fast grouped matmul could not read it as it lies (an unaligned base, rows off the
-    16-byte grid, no unit stride).  A transposed view is read in place: a copy of it would be the whole weights."""
+    """``w [E, R, C]`` as it lies where the fast grouped matmul can read it (an aligned base, one unit stride, the others on the
+    16-byte grid), so a transposed view without a copy, which would be the whole weights; contiguous otherwise."""
     rows, cols = w.stride(1), w.stride(2)
     if not _tracing(w) and w.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0 and \
             ((cols == 1 and rows % 8 == 0) or (rows == 1 and cols % 8 == 0)):
