@@ -18,10 +18,17 @@
 //     [outer][64 reduction] rows of 128 bytes with an XOR swizzle of the 16-byte
 //     chunks; MFMA fragments are read with ds_read_b128 (bank-conflict free).
 //   * operand contiguous along the outer dim (row of A / column of B): stored as it
-//     lies in memory, [64 reduction][256 outer], and the
-//     MFMA fragments (8 consecutive reduction values per lane) are produced by the
-//     transposing LDS read ds_read_b64_tr_b16.  No register transposition, and the
-//     global loads stay fully coalesced (32 lanes x 16 bytes per memory row).
+//     lies in memory, [64 reduction][256 outer], so the global loads stay fully
+//     coalesced (32 lanes x 16 bytes per memory row).  A lane of a 256-row tile reads
+//     16 bytes = 8 outer indices of each of its 8 reduction indices (ds_read_b128, no
+//     swizzle: 16 lanes read 256 consecutive bytes) and puts the MFMA fragments (8
+//     consecutive reduction values of one outer index) together with v_perm_b32, one per
+//     dword.  Block t then holds every eighth outer index of the wavefront from t on; the
+//     epilogue undoes that.  The transposing read ds_read_b64_tr_b16, which the small
+//     tiles use (their wavefronts cover 64 columns, 8 chunks, not 16), takes twice the LDS
+//     instructions: 8192 x 4096 x 28672 in 8 groups with it and with this, one box, dW 1139
+//     -> 1177 TFLOP/s (1326 -> 1419 on all-zero operands, where power does not limit),
+//     forward 1366 -> 1389.
 //
 // The small tail tiles of a RED A run the same way with more stages (dma_small_k_loop below).  Those of an
 // A of the other kind (the weight gradient of a width that is no multiple of 256) keep 32x32x16 and a register-staged K loop
@@ -174,9 +181,9 @@ __device__ __forceinline__ void interleave(std::integer_sequence<int, G...>) {
 // to c.
 //   RED operand:  [256 outer][64 reduction], 128-byte rows (whole cache lines), chunk c of row r holds memory chunk
 //                 c ^ (r & 7)
-//   !RED operand: [64 reduction][256 outer], 512-byte rows, chunk c of row r holds memory chunk
+//   !RED operand: [64 reduction][256 outer], 512-byte rows; WIDE: as in memory; else chunk c of row r holds memory chunk
 //                 c ^ ((r & 3) << 2) ^ (((r >> 3) & 1) << 1)
-// (the first keeps 8 consecutive rows of one chunk column on 8 different bank groups for ds_read_b128, the second the
+// (the first keeps 8 consecutive rows of one chunk column on 8 different bank groups for ds_read_b128, the last the
 // rows of one ds_read_b64_tr_b16 on different 32-byte bank groups).  Whole kernels still count conflicts: 0.09 (forward),
 // 0.07 (dX) and 0.3 (dW, both operands of the second kind) conflict clocks per clock of LDS instructions (Mixtral shape),
 // of fragment reads, incoming transfers and staged epilogue together; which of them was not taken apart.
@@ -189,8 +196,9 @@ constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 1
 
 using lds_ptr = char __attribute__((address_space(3))) *;
 
-template <bool RED, int ROWS = 256>
+template <bool RED, int ROWS = 256, bool WIDE = false>
 struct DmaOperand {
+    static_assert(!WIDE || (!RED && ROWS == 256), "the wide form reads 256-byte pieces of 512-byte rows");
     static_assert(RED || ROWS == 256, "the swizzle of an operand that is contiguous along its outer dim is made for 512-byte rows");
     static constexpr int NX = ROWS * BK * 2 / 4 / 1024;     // 1 KB transfers per wavefront and tile (8, 4 or 2)
     unsigned off[NX];       // per-lane global byte offsets of this wavefront's transfers, relative to the tile base
@@ -224,12 +232,16 @@ struct DmaOperand {
 #pragma unroll
             for (int i = 0; i < NX; ++i) {
                 const int rr = key + 2 * i;
-                const int cg = (lane & 31) ^ ((rr & 3) << 2) ^ (((rr >> 3) & 1) << 1);
+                const int cg = WIDE ? lane & 31 : (lane & 31) ^ ((rr & 3) << 2) ^ (((rr >> 3) & 1) << 1);
                 const bool second = cg >= 16;
                 int outer = outer0 + cg * 8 + (second ? split : 0);
                 const int last = outer_last + (second ? split_last : 0);
                 outer = outer > last ? last : outer;
                 off[i] = static_cast<unsigned>((static_cast<int64_t>(rr) * stride_red + (outer - outer0)) * 2);
+            }
+            if constexpr (WIDE) {
+                frag_off = 8 * (lane >> 4) * 512 + wave_outer * 2 + (lane & 15) * 16;
+                return;
             }
             // transposing read: in each group of 16 lanes, lane L supplies the 4-element segment at
             // (reduction L/4, outer 4*(L%4)) and receives reduction 0..3 of outer L; lane group g covers the reduction
@@ -273,7 +285,20 @@ struct DmaOperand {
             return v16{lo.x, lo.y, hi.x, hi.y};
         }
     }
+
+    // WIDE: reduction index 8 * (lane >> 4) + s of slice kk, of the eight outer indices 8 * (lane & 15) .. + 7 of this wavefront.
+    __device__ __forceinline__ v16 raw(const char *tile, int kk, int s) const {
+        static_assert(WIDE, "whole rows are read of the unswizzled layout only");
+        return *reinterpret_cast<const v16 *>(tile + frag_off + kk * 32 * 512 + s * 512);
+    }
 };
+
+// Dword d of the fragments 2q and 2q + 1 from dword q of the raw reads 2d and 2d + 1: the reduction indices 2d and 2d + 1 of one
+// outer index side by side.
+__device__ __forceinline__ void take_apart(v16 (&frag)[8], int d, int q, const v16 &even, const v16 &odd) {
+    frag[2 * q][d] = __builtin_amdgcn_perm(odd[q], even[q], 0x05040100u);
+    frag[2 * q + 1][d] = __builtin_amdgcn_perm(odd[q], even[q], 0x07060302u);
+}
 
 // The accumulators are in their registers at this point of the program, whatever was or will be done with them.
 template <int TM, int TN>
@@ -321,6 +346,18 @@ __device__ __forceinline__ void settle(f32x4 (&acc)[TM][TN]) {
 // kt in registers and all its transfers of tile kt+1 have landed, so behind it tile kt's stages are free (the transfers
 // of A's tile kt+2 go there at once; B, with three stages, has its tile kt+2 requested in the first half of the step
 // after the one that freed it) and tile kt+1 can be read.
+// Slots of a slice (64 products) that take raw reads apart, and how many of them lie ahead of slot u: none beside a read, none
+// beside a request (slot busy of every eight) or right behind it.  (Two dwords in every slot from the twelfth on, whatever
+// else is in it: dW 1150 instead of 1177 TFLOP/s, forward 1349 instead of 1389.)
+constexpr bool idle_slot(int u, int busy) { return u >= 11 && u % 8 != busy && u % 8 != busy + 1 && (u >= 32 || u % 2 == 1); }
+constexpr int idle_before(int u, int busy) {
+    int n = 0;
+    for (int w = 0; w < u; ++w) n += idle_slot(w, busy) ? 1 : 0;
+    return n;
+}
+constexpr int kBusyB = 5, kBusyA = 1;       // slots of every eight that request a transfer of B (slice 0) and of A (slice 1)
+static_assert(idle_before(64, kBusyB) >= 32 && idle_before(64, kBusyA) >= 32, "both operands' dwords find their slots");
+
 template <int DT, bool A_RED, bool B_RED, bool SWIGLU>
 __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc, char *lds, int row0, int col0,
                                            f32x4 (&acc)[8][8]) {
@@ -331,8 +368,8 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     const int nk = (red_len + BK - 1) / BK;
     if (nk <= 0) return clear(acc);
 
-    DmaOperand<A_RED> la;
-    DmaOperand<B_RED> lb;
+    DmaOperand<A_RED, 256, !A_RED> la;
+    DmaOperand<B_RED, 256, !B_RED> lb;
     la.init(p.a_stride_row, p.a_stride_red, row0, A_RED ? tc.e.row_end - 1 : tc.e.row_end - 8, wm * 128, wave);
     if constexpr (SWIGLU) {
         static_assert(!SWIGLU || !B_RED, "the fused SwiGLU form reads the weight along its columns");
@@ -382,6 +419,30 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
         const int i = u >> 3, j = (i & 1) ? 7 - (u & 7) : (u & 7);
         mfma16x16<DT>(bf[set][j], af[set][i], acc[i][j]);
     };
+    // What slot u does for the fragments of the next slice to be multiplied (slice kk of the stages a, b, into set `set`): one
+    // read every other slot, B's eight and then A's; of an operand that lies along its outer dim, the pairs of raw reads are
+    // taken apart in idle slots, two dwords in each.
+    v16 ra[8], rb[8];
+    auto next_slice = [&](int u, int set, int kk, const char *a, const char *b, int busy) {
+        if (u % 2 == 0 && u < 32) {
+            const int f = u / 2;
+            if (f < 8) {
+                if constexpr (B_RED) bf[set][f] = lb.frag(b, kk, f);
+                else rb[f] = lb.raw(b, kk, f);
+            } else {
+                if constexpr (A_RED) af[set][f - 8] = la.frag(a, kk, f - 8);
+                else ra[f - 8] = la.raw(a, kk, f - 8);
+            }
+        }
+        if (idle_slot(u, busy)) {
+            const int v = idle_before(u, busy), d = (v >> 2) & 3, q = v & 3;
+            if (v < 16) {
+                if constexpr (!B_RED) take_apart(bf[set], d, q, rb[2 * d], rb[2 * d + 1]);
+            } else if (v < 32) {
+                if constexpr (!A_RED) take_apart(af[set], d, q, ra[2 * d], ra[2 * d + 1]);
+            }
+        }
+    };
 
     // tiles 0 and 1 of both operands (the order of the steady state: B before A)
     for (int t = 0; t < nk && t < 2; ++t) {
@@ -400,10 +461,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     const char *a_cur = lds;                                   // stages of tile kt
     const char *b_cur = lds + kAStages * kStageTile;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        bf[0][t] = lb.frag(b_cur, 0, t);
-        af[0][t] = la.frag(a_cur, 0, t);
-    }
+    for (int u = 0; u < 64; ++u) next_slice(u, 0, 0, a_cur, b_cur, kBusyA);
     ready(acc);
     __builtin_amdgcn_sched_barrier(0);
 
@@ -420,13 +478,9 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
 #pragma unroll
         for (int u = 0; u < 64; ++u) {
             mfma(0, u);
-            if (u % 2 == 0 && u < 32) {
-                const int f = u / 2;
-                if (f < 8) bf[1][f] = lb.frag(b_cur, 1, f);
-                else af[1][f - 8] = la.frag(a_cur, 1, f - 8);
-            }
+            next_slice(u, 1, 1, a_cur, b_cur, kBusyB);
             if constexpr (ask) {
-                if (u % 8 == 5) request_b(tail_c, u / 8);
+                if (u % 8 == kBusyB) request_b(tail_c, u / 8);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -441,15 +495,9 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
 #pragma unroll
         for (int u = 0; u < 64; ++u) {
             mfma(1, u);
-            if constexpr (kind != LAST) {
-                if (u % 2 == 0 && u < 32) {
-                    const int f = u / 2;
-                    if (f < 8) bf[0][f] = lb.frag(b_cur, 0, f);
-                    else af[0][f - 8] = la.frag(a_cur, 0, f - 8);
-                }
-            }
+            if constexpr (kind != LAST) next_slice(u, 0, 0, a_cur, b_cur, kBusyA);
             if constexpr (ask) {
-                if (u % 8 == 1) request_a(tail_c, u / 8);
+                if (u % 8 == kBusyA) request_a(tail_c, u / 8);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -590,20 +638,38 @@ __device__ __forceinline__ void dma_small_k_loop(const GmmArgs &p, const TileCoo
 template <int TM, int TN>
 struct Acc32 {                                  // 32 x 32 blocks
     f32x16 v[TM][TN];
-    static constexpr int MB = 32, ROWS = TM, QUADS = TN * 4;
+    static constexpr int MB = 32, ROWS = TM, QUADS = TN * 4, SIDE = 1;
     __device__ __forceinline__ static int col(int q) { return (q >> 2) * 32 + (q & 3) * 8 + 4 * ((threadIdx.x & 63) >> 5); }
     __device__ __forceinline__ f32x4 quad(int i, int q) const {
         const f32x16 &a = v[i][q >> 2];
         const int e = 4 * (q & 3);
         return f32x4{a[e], a[e + 1], a[e + 2], a[e + 3]};
     }
+    __device__ __forceinline__ static int real_row(int staged) { return staged; }
+    __device__ __forceinline__ static int staged_row(int row) { return row; }
 };
-template <int TM, int TN>
+// Quad q of block row i; staged row i * 16 + (lane & 15) of the wavefront's block is its row of that number, or, if A's outer
+// indices were dealt to the blocks in turn (A_WIDE: block i holds 8 m + i), another one: real_row / staged_row.  B_WIDE the same
+// for the columns: the quads 2e and 2e + 1 of a block row are then the eight columns of B's lane group, side by side.
+template <int TM, int TN, bool A_WIDE = false, bool B_WIDE = false>
 struct Acc16 {                                  // 16 x 16 blocks
     f32x4 v[TM][TN];
-    static constexpr int MB = 16, ROWS = TM, QUADS = TN;
-    __device__ __forceinline__ static int col(int q) { return q * 16 + 4 * ((threadIdx.x & 63) >> 4); }
-    __device__ __forceinline__ f32x4 quad(int i, int q) const { return v[i][q]; }
+    static_assert((!A_WIDE || TM == 8) && (!B_WIDE || TN == 8), "dealing is over eight blocks");
+    static constexpr int MB = 16, ROWS = TM, QUADS = TN, SIDE = B_WIDE ? 2 : 1;      // SIDE: quads that lie side by side
+    __device__ __forceinline__ static int col(int q) {
+        const int g = (threadIdx.x & 63) >> 4;
+        return B_WIDE ? 32 * g + 4 * q : q * 16 + 4 * g;
+    }
+    __device__ __forceinline__ f32x4 quad(int i, int q) const {
+        if constexpr (B_WIDE) {
+            const int j = 4 * (q & 1), e = q >> 1;
+            return f32x4{v[i][j][e], v[i][j + 1][e], v[i][j + 2][e], v[i][j + 3][e]};
+        } else {
+            return v[i][q];
+        }
+    }
+    __device__ __forceinline__ static int real_row(int staged) { return A_WIDE ? 8 * (staged & 15) + (staged >> 4) : staged; }
+    __device__ __forceinline__ static int staged_row(int row) { return A_WIDE ? ((row & 7) << 4) + (row >> 3) : row; }
 };
 
 // One macro tile of TBM x 256 outputs.  TBM = 256: 2x2 wavefronts of 128x128; TBM = 128 / 64: 1x4 wavefronts
@@ -626,13 +692,14 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     const int row0 = tc.e.row_begin + tc.row_tile * BM;   // all but the last row tile of a group are full
     const int row_end = tc.e.row_end;
     constexpr bool SWIGLU = OUT == OUT_SWIGLU;
+    static_assert(A_RED || (OUT != OUT_SWIGLU && OUT != OUT_SWIGLU_GRAD), "the fused epilogues read staged rows as they are");
     constexpr int HALF = BN / 2;                          // activation columns per tile in the fused form
     const int col0 = tc.col_tile * (SWIGLU ? HALF : BN);  // fused: first activation (= gate) column
     const int col_end = p.cols;
     const int red_begin = tc.e.red_begin, red_end = tc.e.red_end;
 
     constexpr bool DMA = TBM == 256 || A_RED;   // operands by transfers straight to LDS
-    std::conditional_t<DMA, Acc16<2 * TM, 2 * TN>, Acc32<TM, TN>> sums;
+    std::conditional_t<DMA, Acc16<2 * TM, 2 * TN, TBM == 256 && !A_RED, TBM == 256 && !B_RED>, Acc32<TM, TN>> sums;
     auto &acc = sums.v;
     if constexpr (DMA) {
         if constexpr (TBM == 256) dma_k_loop<DT, A_RED, B_RED, SWIGLU>(p, tc, lds, row0, col0, acc);
@@ -778,12 +845,16 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll
         for (int i = 0; i < Acc::ROWS; ++i)
 #pragma unroll
-            for (int q = 0; q < Acc::QUADS; ++q) {
-                const f32x4 v = sums.quad(i, q);
-                uint16_t h[4];
+            for (int q = 0; q < Acc::QUADS; q += Acc::SIDE) {
+                __attribute__((aligned(16))) uint16_t h[4 * Acc::SIDE];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) h[e] = DT == MS_BF16 ? BF16::from_float(v[e]) : FP16::from_float(v[e]);
-                *reinterpret_cast<uint2 *>(stg + (i * Acc::MB + qrow) * SP + Acc::col(q) * 2) = *reinterpret_cast<uint2 *>(h);
+                for (int s = 0; s < Acc::SIDE; ++s) {
+                    const f32x4 v = sums.quad(i, q + s);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) h[4 * s + e] = DT == MS_BF16 ? BF16::from_float(v[e]) : FP16::from_float(v[e]);
+                }
+                using Piece = std::conditional_t<Acc::SIDE == 2, v16, uint2>;
+                *reinterpret_cast<Piece *>(stg + (i * Acc::MB + qrow) * SP + Acc::col(q) * 2) = *reinterpret_cast<Piece *>(h);
             }
         __builtin_amdgcn_s_waitcnt(0xC07F);    // own writes only: the region is private to this wavefront
         constexpr int LPR = WC / 8;            // lanes per row (8 columns = 16 bytes each)
@@ -845,7 +916,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
             for (int pass = 0; pass < WR / RPP; ++pass) {
                 const int r = pass * RPP + lane / LPR;
                 const int row = row0 + wm * WR + r;
-                const v16 v = *reinterpret_cast<const v16 *>(stg + r * SP + chunk * 16);
+                const v16 v = *reinterpret_cast<const v16 *>(stg + Acc::staged_row(r) * SP + chunk * 16);
                 if (col_ok && row < row_end) *reinterpret_cast<v16 *>(cbase + static_cast<int64_t>(row) * ldc) = v;
             }
         }
@@ -902,7 +973,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
         auto load_old = [&](f32x4 (&dst)[NP], int i) {
 #pragma unroll
             for (int pass = 0; pass < NP; ++pass) {
-                int row = row0 + wm * WR + i * 32 + pass * RPP + lane / LPR;
+                int row = row0 + wm * WR + Acc::real_row(i * 32 + pass * RPP + lane / LPR);
                 row = row < row_end ? row : row_end - 1;
                 dst[pass] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(lbase + static_cast<int64_t>(row) * ldc));
             }
@@ -922,7 +993,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll
             for (int pass = 0; pass < NP; ++pass) {
                 const int r = pass * RPP + lane / LPR;
-                const int row = row0 + wm * WR + i * 32 + r;
+                const int row = row0 + wm * WR + Acc::real_row(i * 32 + r);
                 f32x4 o = *reinterpret_cast<const f32x4 *>(stg + r * SPF + c4);
                 if constexpr (OUT == ACC_F32) o += old[i & 1][pass];
                 if (col_ok && row < row_end) __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(cbase + static_cast<int64_t>(row) * ldc));
