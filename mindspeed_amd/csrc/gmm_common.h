@@ -49,6 +49,9 @@ struct TileTable {
                              // dealt out to single XCDs); `entries` is then unused
     int list_stride;         // entries reserved per list
     int part_from, part_count, part_shift;   // tiles of the last round that run in parts (LastRound)
+    int in_order;            // split on rows: of the first so many tile numbers every XCD takes consecutive ones (take_together) ..
+    int by_cost;             // 0: `in_order` less the last round's parts, an eighth each; 1: all, by share_begin
+    int share_begin[9];      // first tile number of every XCD's share
     int begins[16];          // tile_begin of the first 16 entries (INT_MAX past the last): one load finds the entry
     int list_count[8];       // entries in use in every XCD's list
     GroupEntry entries[1];
@@ -171,12 +174,32 @@ __device__ __forceinline__ void take_part(TileCoord &tc, int part, int shift) {
     tc.valid = tc.e.row_begin + tc.row_tile * tc.e.tile_rows < tc.e.row_end;
 }
 
+// Tile number b, and the same with every XCD's of the n numbers (b = x, x + 8, ... of XCD x) consecutive.
+__device__ __forceinline__ int share_of_eight(int b, int n) {
+    const int x = b & 7, odd = n & 7;
+    return x * (n >> 3) + (x < odd ? x : odd) + (b >> 3);
+}
+
+// Split on rows: whether every XCD takes consecutive tiles of the whole launch, entries laid end to end, or an eighth of every
+// entry's.  Consecutive ones are blocks of 4 x 8 tiles out of one or two groups, 12 operand panels for the 32 compute units;
+// eighths of small groups are pieces of many (three row tiles by 12 columns: five panels for four and a half tiles).  16 groups
+// of 750 rows, bf16, us per launch with eighths and with consecutive tiles: K 2048, 3072 columns 143 / 139; K 1536, 2048 columns
+// 79 / 70; K 3072 145 / 138; K 2048, 1536 columns 81 / 66.  8 groups of 2048 rows, K 2048, 28 column tiles 379 / 361; 64 groups of
+// 0 to 6600 rows, K 1408 to 2816 360 to 655 / 352 to 640.
+// Not where the XCDs' blocks come back to panels that the last-level cache (256 MB) no longer holds: eight XCDs in as many groups
+// have 8 x 12 panels of 512 K bytes under way, while eighths of one large group share theirs.  8 groups of 2048 rows: K 4096 402 /
+// 408, K 7168 1440 / 1483; a group of 6500 rows beside small ones: K 7168 706 / 733, K 4096 703 / 728.  With at most 5 row
+// tiles in a group (one block) no weight panel is read twice at any K (K 28672, 4 row tiles: 1416 / 1397).
+constexpr int kTogetherTileRows = 256;    // (the fp32 kernels' smaller tiles: eighths)
+constexpr int kOneBlockRowTiles = 5, kTwoBlockRowTiles = 9, kTogetherRed = 3072, kTogetherGroups = 16;
+__device__ __forceinline__ bool take_together(bool all_one_block, bool all_two_blocks, int k, int num_groups) {
+    return all_one_block || (k <= kTogetherRed && (all_two_blocks || num_groups >= kTogetherGroups));
+}
+
 // Tile number j of an entry: of the entry's tiles every XCD (workgroup number modulo 8) takes consecutive ones of the
-// blocked order, the odd ones dealt in turn.
-__device__ __forceinline__ void deal_tile(TileCoord &tc, int j, int num_col_tiles) {
-    const int x = j & 7, odd = tc.e.num_tiles & 7;         // this XCD's place in the entry's dealing, tiles beyond whole eighths
-    const int r = x * (tc.e.num_tiles >> 3) + (x < odd ? x : odd) + (j >> 3);
-    tile_order(r, tc.e.num_row_tiles, num_col_tiles, tc.row_tile, tc.col_tile);
+// blocked order, the odd ones dealt in turn; in_order: the j-th one.
+__device__ __forceinline__ void deal_tile(TileCoord &tc, int j, int num_col_tiles, bool in_order = false) {
+    tile_order(in_order ? j : share_of_eight(j, tc.e.num_tiles), tc.e.num_row_tiles, num_col_tiles, tc.row_tile, tc.col_tile);
     tc.tile_rows = (tc.e.tail_rows != 0 && tc.row_tile == tc.e.num_row_tiles - 1) ? tc.e.tail_rows : tc.e.tile_rows;
     tc.valid = true;
 }
@@ -188,10 +211,10 @@ __device__ __forceinline__ void deal_tile(TileCoord &tc, int j, int num_col_tile
 // them).  Inside the entry an XCD's tiles are consecutive in the blocked order above, so concurrently running
 // workgroups of an XCD share operand panels in that XCD's L2.  With many groups the schedule may instead deal whole
 // groups out to single XCDs (every XCD then has a list of its own): a group's operands are fetched into one L2 instead
-// of eight.
+// of eight.  Split on rows (ROWS), an XCD's tiles may instead be consecutive ones of the whole launch (take_together).
 // LISTS: the kernel may meet per-XCD lists (the fast kernels of the split on rows); the others are compiled without that
 // path, which costs the weight-gradient kernel 0.3 us per tile at its start when it is merely present.
-template <bool LISTS>
+template <bool LISTS, bool ROWS>
 __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
     TileCoord tc;
     tc.valid = false;
@@ -215,7 +238,21 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
     }
     const LastRound lr{table->part_from, table->part_count, table->part_shift};
     int part;
-    const int t = tile_of_workgroup(b, lr, part);
+    int t = tile_of_workgroup(b, lr, part);
+    bool in_order = false;
+    if constexpr (ROWS) {
+        const int n = table->in_order;
+        if (table->by_cost != 0) {
+            const int x = b & 7, slot = b >> 3;
+            const int from = table->share_begin[x], own = table->share_begin[x + 1] - from;
+            in_order = slot < own;
+            t = in_order ? from + slot : n + ((slot - own) << 3) + x;
+        } else {
+            in_order = t < n;
+            const int spread = lr.count != 0 && lr.from < n ? lr.from : n;
+            if (t < spread) t = share_of_eight(t, spread);
+        }
+    }
     // Up to 16 entries (8 experts with their tail tiles) their begins lie in the table's header and are fetched at once.
     int lo = 0;
     if (table->num_entries <= 16) {
@@ -227,7 +264,7 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
     tc.e = table->entries[lo];
     const int j = t - tc.e.tile_begin;
     if (j >= tc.e.num_tiles) return tc;
-    deal_tile(tc, j, tc.e.num_tiles / tc.e.num_row_tiles);
+    deal_tile(tc, j, tc.e.num_tiles / tc.e.num_row_tiles, in_order);
     if (t >= lr.from && t < lr.from + lr.count) take_part(tc, part, lr.shift);
     return tc;
 }
@@ -262,6 +299,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
     const int T = p.tile_rows, shift = 31 - __builtin_clz(T);
     LastRound lr{0, 0, 0};
     int t = b, part = 0;                           // tile number, and the part of it
+    bool in_order = false;
     GroupEntry &e = tc.e;
     e = GroupEntry{};
     e.tile_rows = T;
@@ -300,6 +338,14 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
         const int total_first = tails_last ? (all_rt - all_tails) * C : total;
         if (tails_last && p.part_cus != 0) lr = divide_last_round(total_first, total - total_first, p.part_cus);
         t = tile_of_workgroup(b, lr, part);
+        // (small tiles in between cost half of a full one: with more than a tenth of them equal numbers are no equal shares)
+        if (T == kTogetherTileRows &&
+            take_together(__ballot(row_tiles > kOneBlockRowTiles) == 0, __ballot(row_tiles > kTwoBlockRowTiles) == 0, p.k, p.num_groups) &&
+            (tails_last || 10 * all_tails <= all_rt)) {
+            in_order = t < total_first;
+            const int spread = lr.count != 0 ? lr.from : total_first;
+            if (t < spread) t = share_of_eight(t, spread);
+        }
         e.red_end = p.k;
         if (t >= total) {                          // rows past the last offset: zero-fill (empty reduction range)
             const int last_end = __builtin_amdgcn_readlane(static_cast<int>(end), 63);
@@ -333,7 +379,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
             e.b_off = p.b_offsets != nullptr ? p.b_offsets[g] : g * p.b_stride_group;
         }
     }
-    deal_tile(tc, t - e.tile_begin, C);
+    deal_tile(tc, t - e.tile_begin, C, in_order);
     if (t >= lr.from && t < lr.from + lr.count) take_part(tc, part, lr.shift);
     return tc;
 }
@@ -343,7 +389,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
 template <bool SPLIT_RED>
 __device__ __forceinline__ TileCoord locate(const GmmArgs &p) {
     if (p.group_list != nullptr) return tile_from_list<SPLIT_RED>(p);
-    return locate_tile<false>(p.table);
+    return locate_tile<false, !SPLIT_RED>(p.table);
 }
 // ... nor for one kind of split
 __device__ __forceinline__ TileCoord locate_any(const GmmArgs &p) { return p.group_type == 2 ? locate<true>(p) : locate<false>(p); }

@@ -1013,7 +1013,7 @@ __global__ __launch_bounds__(256) void gmm16_fast_kernel(const GmmArgs p) {
     MS_TRACE(1);
     TileCoord tc;
     if constexpr (DIRECT) tc = tile_from_list<!A_RED>(p);
-    else tc = locate_tile<LISTS>(p.table);
+    else tc = locate_tile<LISTS, A_RED>(p.table);
     if (!tc.valid) return;
     MS_TRACE(2);
     if (tc.tile_rows == 256) {
