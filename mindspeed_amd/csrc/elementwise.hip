@@ -46,7 +46,9 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const typename DT::storage 
     }
 }
 
-// One block per row (so grad_probs can be reduced in the same pass).
+// One block per row (so grad_probs can be reduced in the same pass).  Bound by memory: five arrays of rows x ffn.  Ordinary
+// stores, unlike the forward pass (level there): 8192 rows x 14336, bf16, 207 us with non-temporal ones, 183 with these (6.4 TB/s);
+// 65536 x 1408 139 and 135; 16384 x 2048 51.5 and 51.9.
 template <typename DT, int VEC>
 __global__ __launch_bounds__(256) void swiglu_grad_kernel(const typename DT::storage *__restrict__ gy,
                                                           const typename DT::storage *__restrict__ x,
@@ -86,8 +88,8 @@ __global__ __launch_bounds__(256) void swiglu_grad_kernel(const typename DT::sto
         S *dg = gx + r * 2 * ffn + c;
         S *du = dg + ffn;
         if constexpr (VEC * sizeof(S) == 16) {
-            MS_NT_STORE(*reinterpret_cast<v16 *>(og), reinterpret_cast<v16 *>(dg));
-            MS_NT_STORE(*reinterpret_cast<v16 *>(ou), reinterpret_cast<v16 *>(du));
+            *reinterpret_cast<v16 *>(dg) = *reinterpret_cast<v16 *>(og);
+            *reinterpret_cast<v16 *>(du) = *reinterpret_cast<v16 *>(ou);
         } else {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) { dg[e] = og[e]; du[e] = ou[e]; }

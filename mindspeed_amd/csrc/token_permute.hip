@@ -686,7 +686,10 @@ __device__ __forceinline__ void prefetch_row(VecT (&v)[8], const VecT *__restric
 }
 
 // Write one source row to the rows listed in dest[0 .. count) (entries outside [0, limit) are skipped), `lanes`
-// threads per row, eight vectors per thread at a time; v holds the row's first eight vectors already.
+// threads per row, eight vectors per thread at a time; v holds the row's first eight vectors already.  Ordinary stores:
+// the last-level cache takes the rows (up to 256 MB) faster than HBM does, and what reads them next finds them there.  bf16,
+// us per launch with non-temporal and with these: 8192 tokens x top-8, 2048 wide 66 / 54 (the unpermute that follows 75 / 63),
+// 2048 x top-8, 7168 wide 59 / 48, 4096 x top-2, 4096 wide 20.9 / 20.5 (19.2 / 17.0).
 template <typename VecT>
 __device__ __forceinline__ void scatter_row(VecT (&v)[8], const VecT *__restrict__ src, VecT *__restrict__ permuted,
                                             const int *dest, int count, int limit, int lane, int lanes,
@@ -703,7 +706,7 @@ __device__ __forceinline__ void scatter_row(VecT (&v)[8], const VecT *__restrict
             VecT *dst = permuted + static_cast<int64_t>(row) * vecs_per_row;
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                if (c0 + u * lanes < vecs_per_row) MS_NT_STORE(v[u], dst + c0 + u * lanes);
+                if (c0 + u * lanes < vecs_per_row) dst[c0 + u * lanes] = v[u];
         }
     }
 }
