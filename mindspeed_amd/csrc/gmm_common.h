@@ -50,7 +50,7 @@ struct TileTable {
     int list_stride;         // entries reserved per list
     int part_from, part_count, part_shift;   // tiles of the last round that run in parts (LastRound)
     int in_order;            // split on rows: of the first so many tile numbers every XCD takes consecutive ones (take_together) ..
-    int by_cost;             // 0: `in_order` less the last round's parts, an eighth each; 1: all, by share_begin
+    int by_cost;             // 0: an eighth each (consecutive_tile); 1: by share_begin
     int share_begin[9];      // first tile number of every XCD's share
     int begins[16];          // tile_begin of the first 16 entries (INT_MAX past the last): one load finds the entry
     int list_count[8];       // entries in use in every XCD's list
@@ -190,10 +190,25 @@ __device__ __forceinline__ int share_of_eight(int b, int n) {
 // have 8 x 12 panels of 512 K bytes under way, while eighths of one large group share theirs.  8 groups of 2048 rows: K 4096 402 /
 // 408, K 7168 1440 / 1483; a group of 6500 rows beside small ones: K 7168 706 / 733, K 4096 703 / 728.  With at most 5 row
 // tiles in a group (one block) no weight panel is read twice at any K (K 28672, 4 row tiles: 1416 / 1397).
-constexpr int kTogetherTileRows = 256;    // (the fp32 kernels' smaller tiles: eighths)
 constexpr int kOneBlockRowTiles = 5, kTwoBlockRowTiles = 9, kTogetherRed = 3072, kTogetherGroups = 16;
 __device__ __forceinline__ bool take_together(bool all_one_block, bool all_two_blocks, int k, int num_groups) {
     return all_one_block || (k <= kTogetherRed && (all_two_blocks || num_groups >= kTogetherGroups));
+}
+
+// ... and not where an XCD would have the tiles of a large group and another those of many small ones: full tiles are bound by the
+// matrix cores, small ones by the weights that every one of them streams, and eighths put both on every XCD.  60 groups of 1 to
+// 3100 rows (half of the row tiles small), K 792 / 1584, 18 column tiles: 168 / 174 and 312 / 334 us.  So small tiles are at
+// most a quarter, or no group has twice the average (128 rows each: 298 / 282, 250 each: 399 / 342 and 210 / 185).
+__device__ __forceinline__ bool few_small_tiles(int small, int row_tiles) { return 4 * small <= row_tiles; }
+__device__ __forceinline__ bool much_above_average(int group_row_tiles, int row_tiles, int num_groups) {
+    return static_cast<int64_t>(group_row_tiles) * num_groups > 2 * static_cast<int64_t>(row_tiles);
+}
+
+// Tile number t of the first n, dealt over the XCDs one by one, as one of consecutive ones of its XCD: those in front of the last
+// round's parts, and the tiles that run in parts.
+__device__ __forceinline__ int consecutive_tile(int t, int n, const LastRound &lr) {
+    const int whole = lr.count != 0 ? lr.from : n;
+    return t < whole ? share_of_eight(t, whole) : whole + share_of_eight(t - whole, n - whole);
 }
 
 // Tile number j of an entry: of the entry's tiles every XCD (workgroup number modulo 8) takes consecutive ones of the
@@ -249,8 +264,7 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
             t = in_order ? from + slot : n + ((slot - own) << 3) + x;
         } else {
             in_order = t < n;
-            const int spread = lr.count != 0 && lr.from < n ? lr.from : n;
-            if (t < spread) t = share_of_eight(t, spread);
+            if (in_order) t = consecutive_tile(t, n, lr);
         }
     }
     // Up to 16 entries (8 experts with their tail tiles) their begins lie in the table's header and are fetched at once.
@@ -339,12 +353,11 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
         if (tails_last && p.part_cus != 0) lr = divide_last_round(total_first, total - total_first, p.part_cus);
         t = tile_of_workgroup(b, lr, part);
         // (small tiles in between cost half of a full one: with more than a tenth of them equal numbers are no equal shares)
-        if (T == kTogetherTileRows &&
+        if (p.small_tails && (tails_last || 10 * all_tails <= all_rt) &&
             take_together(__ballot(row_tiles > kOneBlockRowTiles) == 0, __ballot(row_tiles > kTwoBlockRowTiles) == 0, p.k, p.num_groups) &&
-            (tails_last || 10 * all_tails <= all_rt)) {
+            (few_small_tiles(all_tails, all_rt) || __ballot(much_above_average(row_tiles, all_rt, p.num_groups)) == 0)) {
             in_order = t < total_first;
-            const int spread = lr.count != 0 ? lr.from : total_first;
-            if (t < spread) t = share_of_eight(t, spread);
+            if (in_order) t = consecutive_tile(t, total_first, lr);
         }
         e.red_end = p.k;
         if (t >= total) {                          // rows past the last offset: zero-fill (empty reduction range)
