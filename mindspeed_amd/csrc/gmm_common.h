@@ -352,8 +352,8 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
         const int total_first = tails_last ? (all_rt - all_tails) * C : total;
         if (tails_last && p.part_cus != 0) lr = divide_last_round(total_first, total - total_first, p.part_cus);
         t = tile_of_workgroup(b, lr, part);
-        // (small tiles in between cost half of a full one: with more than a tenth of them equal numbers are no equal shares)
-        if (p.small_tails && (tails_last || 10 * all_tails <= all_rt) &&
+        // (all small: nothing to place.  Small tiles in between cost half of a full one: with more than a tenth of them equal numbers are no equal shares)
+        if (p.small_tails && total_first != 0 && (tails_last || 10 * all_tails <= all_rt) &&
             take_together(__ballot(row_tiles > kOneBlockRowTiles) == 0, __ballot(row_tiles > kTwoBlockRowTiles) == 0, p.k, p.num_groups) &&
             (few_small_tiles(all_tails, all_rt) || __ballot(much_above_average(row_tiles, all_rt, p.num_groups)) == 0)) {
             in_order = t < total_first;
