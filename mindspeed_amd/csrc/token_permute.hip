@@ -686,14 +686,19 @@ __device__ __forceinline__ void prefetch_row(VecT (&v)[8], const VecT *__restric
 }
 
 // Write one source row to the rows listed in dest[0 .. count) (entries outside [0, limit) are skipped), `lanes`
-// threads per row, eight vectors per thread at a time; v holds the row's first eight vectors already.  Ordinary stores:
-// the last-level cache takes the rows (up to 256 MB) faster than HBM does, and what reads them next finds them there.  bf16,
-// us per launch with non-temporal and with these: 8192 tokens x top-8, 2048 wide 66 / 54 (the unpermute that follows 75 / 63),
-// 2048 x top-8, 7168 wide 59 / 48, 4096 x top-2, 4096 wide 20.9 / 20.5 (19.2 / 17.0).
-template <typename VecT>
-__device__ __forceinline__ void scatter_row(VecT (&v)[8], const VecT *__restrict__ src, VecT *__restrict__ permuted,
-                                            const int *dest, int count, int limit, int lane, int lanes,
-                                            int vecs_per_row) {
+// threads per row, eight vectors per thread at a time; v holds the row's first eight vectors already.  Ordinary stores as
+// long as the tokens and the permuted rows are no larger than the last-level cache (256 MB) by much: it takes the rows
+// faster than HBM does, and what reads them next finds them there.  Beyond that the rows are in HBM before anything reads
+// them, and non-temporal stores take less time.  bf16, us of the permute and the unpermute that reads its rows, with
+// non-temporal and with ordinary stores (the permute alone, its output then left in the cache to be written back: 14 / 16 to
+// 52 / 57): 3001 tokens x top-4, 2048 wide (61 MB) 32 / 28; 2048 x top-8, 7168 wide (264 MB) 115 / 107; 8192 x top-8: 2048 wide
+// (302 MB) 138 / 121, 2240 wide (330 MB) 142 / 141, 2432 wide (359 MB) 152 / 158, 7168 wide (1057 MB) 439 / 449; 16384 x top-2,
+// 4096 wide (402 MB) 165 / 175.
+constexpr int64_t kCachedRowsBytes = 320ll << 20;
+template <bool CACHED, typename VecT>
+__device__ __forceinline__ void scatter_row_as(VecT (&v)[8], const VecT *__restrict__ src, VecT *__restrict__ permuted,
+                                               const int *dest, int count, int limit, int lane, int lanes,
+                                               int vecs_per_row) {
     for (int c0 = lane; c0 < vecs_per_row; c0 += 8 * lanes) {
         if (c0 != lane) {
 #pragma unroll
@@ -705,10 +710,23 @@ __device__ __forceinline__ void scatter_row(VecT (&v)[8], const VecT *__restrict
             if (static_cast<unsigned>(row) >= static_cast<unsigned>(limit)) continue;   // dropped
             VecT *dst = permuted + static_cast<int64_t>(row) * vecs_per_row;
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (c0 + u * lanes < vecs_per_row) dst[c0 + u * lanes] = v[u];
+            for (int u = 0; u < 8; ++u) {
+                if (c0 + u * lanes >= vecs_per_row) continue;
+                if constexpr (CACHED) dst[c0 + u * lanes] = v[u];
+                else MS_NT_STORE(v[u], dst + c0 + u * lanes);
+            }
         }
     }
+}
+template <typename VecT>
+__device__ __forceinline__ void scatter_row(VecT (&v)[8], const VecT *__restrict__ src, VecT *__restrict__ permuted,
+                                            const int *dest, int count, int limit, int lane, int lanes,
+                                            int vecs_per_row, int num_tokens) {
+    // (decided outside of the loops: beside each other the compiler merges the two kinds of store)
+    if ((static_cast<int64_t>(num_tokens) + limit) * vecs_per_row * static_cast<int64_t>(sizeof(VecT)) <= kCachedRowsBytes)
+        scatter_row_as<true>(v, src, permuted, dest, count, limit, lane, lanes, vecs_per_row);
+    else
+        scatter_row_as<false>(v, src, permuted, dest, count, limit, lane, lanes, vecs_per_row);
 }
 
 // ---- sort and row scatter in one launch ------------------------------------------------
@@ -866,7 +884,7 @@ __global__ __launch_bounds__(1024) void permute_fused_kernel(
     __syncthreads();
 
     if (!mover) return;
-    scatter_row(v, src, permuted, dest + local_row * topk, topk, num_out, lane, lanes, vecs_per_row);
+    scatter_row(v, src, permuted, dest + local_row * topk, topk, num_out, lane, lanes, vecs_per_row, num_tokens);
 }
 
 // The one-launch permute for more than kFusedMaxBins bins (up to MS_MAX_EXPERTS, which is what a call without
@@ -962,7 +980,7 @@ __global__ __launch_bounds__(1024) void permute_fused_bins_kernel(
     }
     __syncthreads();
     if (!mover) return;
-    scatter_row(v, src, permuted, dest + local_row * topk, topk, num_out, lane, lanes, vecs_per_row);
+    scatter_row(v, src, permuted, dest + local_row * topk, topk, num_out, lane, lanes, vecs_per_row, num_tokens);
 }
 
 // Stable scatter and row movement in one launch, behind the histogram launch of the multi-block sort (any bin
@@ -1073,7 +1091,7 @@ __global__ __launch_bounds__(1024) void permute_scatter_rows_kernel(
     }
     __syncthreads();
     if (!mover) return;
-    scatter_row(v, src, permuted, dest + local_row * topk, topk, num_out, lane, lanes, vecs_per_row);
+    scatter_row(v, src, permuted, dest + local_row * topk, topk, num_out, lane, lanes, vecs_per_row, num_tokens);
 }
 
 // ---- routing-map (mask) mode ----------------------------------------------------------
@@ -1297,7 +1315,7 @@ __global__ __launch_bounds__(1024) void routing_map_fused_kernel(
         }
     }
     __syncthreads();
-    if (mover) scatter_row(v, src, permuted, rows + local_row * E, E, num_rows, lane, lanes, vecs_per_row);
+    if (mover) scatter_row(v, src, permuted, rows + local_row * E, E, num_rows, lane, lanes, vecs_per_row, num_tokens);
     if (extras.any())               // (behind the rows, whose stores need not wait for the probabilities' way)
         for (int q = tid; q < own; q += nthreads)
             if (rows[q] < num_rows) extras.put(rows[q], split + q, t0 + q / E);
@@ -1411,7 +1429,7 @@ __global__ __launch_bounds__(1024) void routing_map_ranked_kernel(
         }
     }
     __syncthreads();
-    if (mover) scatter_row(v, src, permuted, list + local_row * E, ntok[local_row], num_rows, lane, lanes, vecs_per_row);
+    if (mover) scatter_row(v, src, permuted, list + local_row * E, ntok[local_row], num_rows, lane, lanes, vecs_per_row, num_tokens);
     if (extras.any())
         for (int q = tid; q < own_n; q += nthreads)
             if (row_of[q] < num_rows) extras.put(row_of[q], split + q, t0 + q / E);
