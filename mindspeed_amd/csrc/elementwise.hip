@@ -47,19 +47,18 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const typename DT::storage 
 }
 
 // One block per row (so grad_probs can be reduced in the same pass).  Bound by memory: five arrays of rows x ffn.  Ordinary
-// stores, unlike the forward pass (level there): 8192 rows x 14336, bf16, 207 us with non-temporal ones, 183 with these (6.4 TB/s);
-// 65536 x 1408 139 and 135; 16384 x 2048 51.5 and 51.9.
-template <typename DT, int VEC>
-__global__ __launch_bounds__(256) void swiglu_grad_kernel(const typename DT::storage *__restrict__ gy,
-                                                          const typename DT::storage *__restrict__ x,
-                                                          const void *__restrict__ probs, int probs_dtype,
-                                                          typename DT::storage *__restrict__ gx,
-                                                          void *__restrict__ gprobs, int ffn) {
+// stores, unlike the forward pass (level there), for an output of up to half of the last-level cache (256 MB), where what reads
+// it next finds it; beyond that, and where it is not read soon, they cost more than they save.  bf16, us of this kernel and one
+// that reads its output, with non-temporal and with ordinary stores: 8192 rows x 3584 (117 MB) 90.6 / 86.5, 16384 x 2048 (134)
+// 98.8 / 95.6, 16384 x 2304 (151) 112.5 / 112.6, 16384 x 3072 (201) 149.6 / 155.1, 65536 x 1408 (369) 269 / 283, 8192 x 14336
+// (470) 371 / 374; passes of training layers: 8192 x 3584 2522 / 2506, 65536 x 1408 3737 / 3758, 8192 x 14336 within 0.3 %.
+constexpr int64_t kCachedGradBytes = 128ll << 20;
+// d_gate and d_up of one row, vector by vector; returns this thread's part of dot(gy, activation).
+template <typename DT, int VEC, bool CACHED>
+__device__ __forceinline__ float swiglu_grad_row(const typename DT::storage *__restrict__ gy, const typename DT::storage *__restrict__ x,
+                                                 typename DT::storage *__restrict__ gx, int64_t r, int ffn, float p) {
     using S = typename DT::storage;
-    __shared__ float partial[4];
-    const int64_t r = blockIdx.x;
     const int vecs = ffn / VEC;
-    const float p = probs != nullptr ? load_scalar_as_float(probs, r, probs_dtype) : 1.f;
     float dot = 0.f;
     for (int v = threadIdx.x; v < vecs; v += blockDim.x) {
         const int c = v * VEC;
@@ -88,13 +87,33 @@ __global__ __launch_bounds__(256) void swiglu_grad_kernel(const typename DT::sto
         S *dg = gx + r * 2 * ffn + c;
         S *du = dg + ffn;
         if constexpr (VEC * sizeof(S) == 16) {
-            *reinterpret_cast<v16 *>(dg) = *reinterpret_cast<v16 *>(og);
-            *reinterpret_cast<v16 *>(du) = *reinterpret_cast<v16 *>(ou);
+            if constexpr (CACHED) {
+                *reinterpret_cast<v16 *>(dg) = *reinterpret_cast<v16 *>(og);
+                *reinterpret_cast<v16 *>(du) = *reinterpret_cast<v16 *>(ou);
+            } else {
+                MS_NT_STORE(*reinterpret_cast<v16 *>(og), reinterpret_cast<v16 *>(dg));
+                MS_NT_STORE(*reinterpret_cast<v16 *>(ou), reinterpret_cast<v16 *>(du));
+            }
         } else {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) { dg[e] = og[e]; du[e] = ou[e]; }
         }
     }
+    return dot;
+}
+
+template <typename DT, int VEC>
+__global__ __launch_bounds__(256) void swiglu_grad_kernel(const typename DT::storage *__restrict__ gy,
+                                                          const typename DT::storage *__restrict__ x,
+                                                          const void *__restrict__ probs, int probs_dtype,
+                                                          typename DT::storage *__restrict__ gx,
+                                                          void *__restrict__ gprobs, int ffn) {
+    __shared__ float partial[4];
+    const int64_t r = blockIdx.x;
+    const float p = probs != nullptr ? load_scalar_as_float(probs, r, probs_dtype) : 1.f;
+    const int64_t out_bytes = static_cast<int64_t>(gridDim.x) * 2 * ffn * static_cast<int64_t>(sizeof(typename DT::storage));
+    float dot = out_bytes <= kCachedGradBytes ? swiglu_grad_row<DT, VEC, true>(gy, x, gx, r, ffn, p)
+                                              : swiglu_grad_row<DT, VEC, false>(gy, x, gx, r, ffn, p);
     if (gprobs != nullptr) {
 #pragma unroll
         for (int dlt = 32; dlt > 0; dlt >>= 1) dot += __shfl_down(dot, dlt, 64);
