@@ -71,13 +71,14 @@ _SIGNATURES = {
     "ms_gather_rows": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _int, _int, _c_void_p],
     "ms_chunk_sort_map": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _c_void_p],
 }
-# combined forms for this package's own use (csrc/internal.h); not part of the C ABI that the version stands for: msi_interface()
+# combined forms and a diagnostic for this package's own use (csrc/internal.h); not part of the C ABI that the version stands for: msi_interface()
 # names the declarations that a build was made from
 _INTERNAL = {
     "msi_routing_map_permute": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _int, _i64, _int, _c_void_p, _c_void_p,
                                 _c_void_p, _c_void_p, _c_void_p, _int, _c_void_p, _c_void_p, _c_void_p, _size_t],
     "msi_unpermute_grad": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _i64, _i64, _i64, _int, _i64,
                            _c_void_p, _c_void_p, _c_void_p],
+    "msi_gmm_takes_together": [ctypes.POINTER(_i64), _i64, _i64, _i64, _int, _int, ctypes.POINTER(_int)],
 }
 EXPORTED_SYMBOLS = tuple(_SIGNATURES) + ("ms_last_error",)
 

@@ -191,7 +191,7 @@ __device__ __forceinline__ int share_of_eight(int b, int n) {
 // 408, K 7168 1440 / 1483; a group of 6500 rows beside small ones: K 7168 706 / 733, K 4096 703 / 728.  With at most 5 row
 // tiles in a group (one block) no weight panel is read twice at any K (K 28672, 4 row tiles: 1416 / 1397).
 constexpr int kOneBlockRowTiles = 5, kTwoBlockRowTiles = 9, kTogetherRed = 3072, kTogetherGroups = 16;
-__device__ __forceinline__ bool take_together(bool all_one_block, bool all_two_blocks, int k, int num_groups) {
+__host__ __device__ __forceinline__ bool take_together(bool all_one_block, bool all_two_blocks, int k, int num_groups) {
     return all_one_block || (k <= kTogetherRed && (all_two_blocks || num_groups >= kTogetherGroups));
 }
 
@@ -199,10 +199,19 @@ __device__ __forceinline__ bool take_together(bool all_one_block, bool all_two_b
 // matrix cores, small ones by the weights that every one of them streams, and eighths put both on every XCD.  60 groups of 1 to
 // 3100 rows (half of the row tiles small), K 792 / 1584, 18 column tiles: 168 / 174 and 312 / 334 us.  So small tiles are at
 // most a quarter, or no group has twice the average (128 rows each: 298 / 282, 250 each: 399 / 342 and 210 / 185).
-__device__ __forceinline__ bool few_small_tiles(int small, int row_tiles) { return 4 * small <= row_tiles; }
-__device__ __forceinline__ bool much_above_average(int group_row_tiles, int row_tiles, int num_groups) {
+__host__ __device__ __forceinline__ bool few_small_tiles(int small, int row_tiles) { return 4 * small <= row_tiles; }
+__host__ __device__ __forceinline__ bool much_above_average(int group_row_tiles, int row_tiles, int num_groups) {
     return static_cast<int64_t>(group_row_tiles) * num_groups > 2 * static_cast<int64_t>(row_tiles);
 }
+
+// In which launches the two ways to find a tile ask that at all.  From the group list shares are equal in number: with small
+// tiles between the full ones (half of their cost) only up to a tenth of them are close enough to equal shares; with the small
+// ones last any number, but there must be a full tile to place.  From a table they are equal in cost, or with the small tiles
+// last in number, which takes a round of full tiles (the launches with a table that have fewer are decoding ones).
+__host__ __device__ __forceinline__ bool list_places(bool tails_last, int full_tiles, int small, int row_tiles) {
+    return tails_last ? full_tiles != 0 : row_tiles != 0 && 10 * small <= row_tiles;
+}
+__host__ __device__ __forceinline__ bool table_places(bool tails_last, int full_tiles, int cus) { return !tails_last || full_tiles >= cus; }
 
 // Tile number t of the first n, dealt over the XCDs one by one, as one of consecutive ones of its XCD: those in front of the last
 // round's parts, and the tiles that run in parts.
@@ -352,8 +361,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
         const int total_first = tails_last ? (all_rt - all_tails) * C : total;
         if (tails_last && p.part_cus != 0) lr = divide_last_round(total_first, total - total_first, p.part_cus);
         t = tile_of_workgroup(b, lr, part);
-        // (all small: nothing to place.  Small tiles in between cost half of a full one: with more than a tenth of them equal numbers are no equal shares)
-        if (p.small_tails && total_first != 0 && (tails_last || 10 * all_tails <= all_rt) &&
+        if (p.small_tails && list_places(tails_last, total_first, all_tails, all_rt) &&
             take_together(__ballot(row_tiles > kOneBlockRowTiles) == 0, __ballot(row_tiles > kTwoBlockRowTiles) == 0, p.k, p.num_groups) &&
             (few_small_tiles(all_tails, all_rt) || __ballot(much_above_average(row_tiles, all_rt, p.num_groups)) == 0)) {
             in_order = t < total_first;

@@ -1,5 +1,5 @@
-// Entry points for this package's own bindings only: combinations of what include/mindspeed_amd.h declares that save a
-// launch.  Not part of the C ABI that ms_version() stands for.
+// Entry points for this package's own use only: combinations of what include/mindspeed_amd.h declares that save a
+// launch, and a diagnostic.  Not part of the C ABI that ms_version() stands for.
 #pragma once
 
 #include "../../include/mindspeed_amd.h"
@@ -25,6 +25,13 @@ int msi_unpermute_grad(ms_stream_t stream, const void *permuted_tokens, const vo
                        const int32_t *row_id_map, const void *probs, int probs_dtype, int64_t num_tokens, int64_t topk,
                        int64_t hidden, int dtype, int64_t num_rows, const int32_t *sorted_flat, void *grad_permuted,
                        void *grad_probs);
+/* Diagnostic, host only: whether a 16-bit launch split on rows with these group sizes (a host array) gives every XCD
+ * consecutive tiles of the whole launch instead of an eighth of every group's, by the rule of the lookup in the group list
+ * (from_list != 0) or of the schedule kernel's table; num_cus: the GPU's compute units.  Evaluates the functions the kernels
+ * call, so a test can check that a launch takes the order it is meant to.  (A table falls back to eighths where shares equal
+ * in cost need more workgroups than the launch has, and makes no such shares where it deals out whole groups.) */
+int msi_gmm_takes_together(const int64_t *rows, int64_t num_groups, int64_t k, int64_t n, int from_list, int num_cus,
+                           int *together);
 
 #ifdef __cplusplus
 }
