@@ -186,13 +186,29 @@ __device__ __forceinline__ int share_of_eight(int b, int n) {
 // of 750 rows, bf16, us per launch with eighths and with consecutive tiles: K 2048, 3072 columns 143 / 139; K 1536, 2048 columns
 // 79 / 70; K 3072 145 / 138; K 2048, 1536 columns 81 / 66.  8 groups of 2048 rows, K 2048, 28 column tiles 379 / 361; 64 groups of
 // 0 to 6600 rows, K 1408 to 2816 360 to 655 / 352 to 640.
-// Not where the XCDs' blocks come back to panels that the last-level cache (256 MB) no longer holds: eight XCDs in as many groups
-// have 8 x 12 panels of 512 K bytes under way, while eighths of one large group share theirs.  8 groups of 2048 rows: K 4096 402 /
-// 408, K 7168 1440 / 1483; a group of 6500 rows beside small ones: K 7168 706 / 733, K 4096 703 / 728.  With at most 5 row
-// tiles in a group (one block) no weight panel is read twice at any K (K 28672, 4 row tiles: 1416 / 1397).
+// Not where an eighth of a group is about a block by itself: the XCDs then share the group's panels, while eight XCDs in as many
+// groups come back to panels that the last-level cache (256 MB) may no longer hold (8 x 12 of them, 512 K bytes each, are under
+// way).  So from 6 row tiles on there is a limit on the reduction, and on the largest of few groups (row tiles times K) or the tiles
+// in the average one of many.  Rows per group, eighths / consecutive, us per launch:
+//   8 groups of 1600 (7 row tiles): K 3072, 2048 columns 148 / 140; 4096 columns: K 2560 232 / 225, 2816 254 / 250, 3072 278 / 282,
+//   3584 318 / 319; 8 of 2100 (9): K 2048 240 / 234.5, 2816 319 / 324, 7168 (2048 rows) 1440 / 1483
+//   16 groups of 2000 (8 or 9): 2048 columns: K 1536 190 / 183, 3072 346 / 344; 4096 columns: K 1536 365 / 357, 2048 467 / 465, 2560
+//   564 / 575, 3072 660 / 666; of 2816 (11 or 12): 2048 columns: K 1536 257 / 248, 3072 461 / 455; 4096 columns: K 1536 483 / 488, 2048
+//   616 / 624, 2560 750 / 764; of 4000 (16): 2048 columns: K 1536 347 / 365, 3072 650 / 667; 4096 columns: K 1024 497 / 505, 1536 670 /
+//   696, 2560 1025 / 1055; of 100 to 2900 (6): K 1536, 2048 columns 127 / 122
+//   64 and 128 groups of 65536 rows together: K 1408 to 3072, 2048 and 2816 columns 2 to 5 % less time, K 4096 level
+// Up to 5 row tiles (one block) there is none: 16 of 750, K 5120, 2048 columns 251 / 237; 8 of 1200, K 4096 to 14336 275 to 917 / 267 to
+// 900; 8 of 1024, K 28672 1416 / 1397 (small tiles that come last read their panels again in either order, and two XCDs read the
+// panels at the border of their shares).
 constexpr int kOneBlockRowTiles = 5, kTwoBlockRowTiles = 9, kTogetherRed = 3072, kTogetherGroups = 16;
-__host__ __device__ __forceinline__ bool take_together(bool all_one_block, bool all_two_blocks, int k, int num_groups) {
-    return all_one_block || (k <= kTogetherRed && (all_two_blocks || num_groups >= kTogetherGroups));
+constexpr int kLargestRowTilesRed = 7 * kTogetherRed, kAverageTiles = 112;
+__host__ __device__ __forceinline__ int together_row_tiles(int k) {       // .. of the largest group
+    if (k > kTogetherRed) return kOneBlockRowTiles;
+    return kTwoBlockRowTiles * k <= kLargestRowTilesRed ? kTwoBlockRowTiles : (8 * k <= kLargestRowTilesRed ? 8 : 7);
+}
+// none_larger: no group has more than together_row_tiles; tiles: of all groups
+__host__ __device__ __forceinline__ bool take_together(bool none_larger, int tiles, int k, int num_groups) {
+    return none_larger || (k <= kTogetherRed && num_groups >= kTogetherGroups && tiles <= kAverageTiles * num_groups);
 }
 
 // ... and not where an XCD would have the tiles of a large group and another those of many small ones: full tiles are bound by the
@@ -362,7 +378,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
         if (tails_last && p.part_cus != 0) lr = divide_last_round(total_first, total - total_first, p.part_cus);
         t = tile_of_workgroup(b, lr, part);
         if (p.small_tails && list_places(tails_last, total_first, all_tails, all_rt) &&
-            take_together(__ballot(row_tiles > kOneBlockRowTiles) == 0, __ballot(row_tiles > kTwoBlockRowTiles) == 0, p.k, p.num_groups) &&
+            take_together(__ballot(row_tiles > together_row_tiles(p.k)) == 0, total, p.k, p.num_groups) &&
             (few_small_tiles(all_tails, all_rt) || __ballot(much_above_average(row_tiles, all_rt, p.num_groups)) == 0)) {
             in_order = t < total_first;
             if (in_order) t = consecutive_tile(t, total_first, lr);

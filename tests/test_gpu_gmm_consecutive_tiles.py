@@ -19,13 +19,18 @@ CASES = {
     "few_small_tiles_between": ("list, by number", 29, RED, [2048 + 30 * g for g in range(8)], 300),       # 8 rounds, 4 of 71 small
     "a_fifth_small_tiles_between": ("list, eighths", 52, RED, [1024 + 3 * g + 1 for g in range(8)], 0),
     "many_small_tiles_between": ("list, eighths", 90, RED, [257, 300, 520, 256, 70, 513, 1] * 2, 0),
-    "two_blocks_short_reduction": ("list, by number", 12, 3072, [1500 + g for g in range(8)], 10),
-    "two_blocks_long_reduction": ("list, eighths", 12, 3080, [1500 + g for g in range(8)], 10),
+    "seven_row_tiles_short_reduction": ("list, by number", 12, 3072, [1700 + g for g in range(8)], 10),
+    "six_row_tiles_long_reduction": ("list, eighths", 12, 3080, [1500 + g for g in range(8)], 10),
+    "nine_row_tiles_short_reduction": ("list, by number", 12, 2384, [2100, 1800, 2300, 2200], 0),
+    "nine_row_tiles_long_reduction": ("list, eighths", 12, 2392, [2100, 1800, 2300, 2200], 0),
     "sixteen_groups_one_large": ("list, by number", 12, RED, [2600] + [250] * 15, 0),
     "fifteen_groups_one_large": ("list, eighths", 12, RED, [2600] + [250] * 14, 0),
     # from the table
     "seventy_groups": ("table, by number", 8, RED, [300 + g for g in range(70)], 33),
     "seventy_groups_of_one_round": ("table, eighths", 4, RED, [200, 100] * 35, 0),
+    "sixteen_groups_of_112_tiles": ("table, by cost", 8, 136, [3584 + 256 * (g % 3 - 1) for g in range(16)], 0),
+    "sixteen_groups_of_more": ("table, eighths", 8, 136, [3584 + 256 * (g % 3 - 1) for g in range(15)] + [3600], 0),
+    "sixteen_large_groups": ("table, eighths", 13, 72, [2560] * 16, 0),
     "tails_in_parts": ("table, by number in parts", 16, 4168, [1024 + 10 * (g % 2) for g in range(8)], 5),
     "shares_by_cost": ("table, by cost", 28, RED, [2305] + [230 + 57 * g for g in range(19)], 130),          # seven rounds
     "shares_by_cost_one_block": ("table, by cost", 110, RED, [1024 + 7 * g for g in range(8)], 0),        # 17 rounds
