@@ -213,7 +213,8 @@ int ms_gmm_tile_order(int num_row_tiles, int num_col_tiles, int index, int *row_
  * grid) that ms_gmm launches for the tiles of a 16-bit problem of these sizes.  lists: the launch may deal whole
  * groups out to single XCDs (16 to 256 groups); split: it may split the reduction of its tail tiles.  The function
  * the launch itself calls: a test can check with it that no table the schedule kernel writes needs more slots than
- * the launch has.  The common table needs an eighth of all tiles, rounded up; with per-XCD lists and a split on the
+ * the launch has.  The common table needs an eighth of all tiles, rounded up (shares of consecutive tiles that are equal in
+ * cost may need more, and are only taken where they fit); with per-XCD lists and a split on the
  * reduction dim (group_type 2) the fullest XCD holds ceil(num_groups / 8) whole output blocks.  A split on rows of
  * few rounds of tiles comes with another three quarters of a workgroup per compute unit, for the parts that it may
  * divide the tiles of its last round into. */

@@ -42,7 +42,7 @@ constexpr int kMaxListGroups = 256;      // most groups that may be dealt out wh
                                          // dealt out by one thread)
 
 struct TileTable {
-    int slots_per_xcd;       // an eighth of all tiles, rounded up; per-XCD lists: slots of the longest one
+    int slots_per_xcd;       // an eighth of all tiles, rounded up; shares by cost and per-XCD lists: slots of the longest one
     int num_entries;
     int num_split_tails;     // tail tile rows whose reduction was split (entries of the SplitTail array in use)
     int lists_off;           // 0, or the byte offset from the table to eight lists of entries, one per XCD (whole groups
@@ -183,8 +183,8 @@ __device__ __forceinline__ int share_of_eight(int b, int n) {
 // Split on rows: whether every XCD takes consecutive tiles of the whole launch, entries laid end to end, or an eighth of every
 // entry's.  Consecutive ones are blocks of 4 x 8 tiles out of one or two groups, 12 operand panels for the 32 compute units;
 // eighths of small groups are pieces of many (three row tiles by 12 columns: five panels for four and a half tiles).  16 groups
-// of 750 rows, bf16, us per launch with eighths and with consecutive tiles: K 2048, 3072 columns 143 / 139; K 1536, 2048 columns
-// 79 / 70; K 3072 145 / 138; K 2048, 1536 columns 81 / 66.  8 groups of 2048 rows, K 2048, 28 column tiles 379 / 361; 64 groups of
+// of 710 to 790 rows, bf16, us per launch with eighths and with consecutive tiles: K 2048, 3072 columns 147 / 143 (weights along
+// K 141 / 136); K 1536, 2048 columns 84 / 75 (81 / 72).  8 groups of 2048 rows, K 2048, 28 column tiles 379 / 361; 64 groups of
 // 0 to 6600 rows, K 1408 to 2816 360 to 655 / 352 to 640.
 // Not where an eighth of a group is about a block by itself: the XCDs then share the group's panels, while eight XCDs in as many
 // groups come back to panels that the last-level cache (256 MB) may no longer hold (8 x 12 of them, 512 K bytes each, are under
@@ -311,10 +311,12 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
 // Rows of the small tile that a remainder of `rem` rows of a group goes to, 0 for a full one.
 __host__ __device__ __forceinline__ int small_tile_rows(int rem) { return rem <= 64 ? 64 : (rem <= 128 ? 128 : 0); }
 
-// The same tile as from a table without per-XCD lists and split tails (gmm_schedule_kernel), found by every wavefront
-// for itself out of a group list of at most 64 groups: lane g holds group g, the running quantities are prefix sums over
-// the lanes, and the entry that holds this workgroup's tile comes out of one ballot.  One load instead of the table's two
-// dependent ones, and no launch in front of the matmul.
+// A tile of the launch, found by every wavefront for itself out of a group list of at most 64 groups: the entries and tile numbers
+// of a table without per-XCD lists and split tails (gmm_schedule_kernel).  Lane g holds group g, the running quantities are
+// prefix sums over the lanes, and the entry that holds this workgroup's tile comes out of one ballot.  One load instead of the
+// table's two dependent ones, and no launch in front of the matmul.  Which tile number a workgroup takes may differ from a
+// table's: consecutive tiles are shared out by number here, by cost there, and asked for in other launches (list_places,
+// table_places).
 constexpr int kMaxDirectGroups = 64;
 template <bool SPLIT_RED>
 __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {

@@ -184,9 +184,9 @@ __device__ __forceinline__ void interleave(std::integer_sequence<int, G...>) {
 //   !RED operand: [64 reduction][256 outer], 512-byte rows; WIDE: as in memory; else chunk c of row r holds memory chunk
 //                 c ^ ((r & 3) << 2) ^ (((r >> 3) & 1) << 1)
 // (the first keeps 8 consecutive rows of one chunk column on 8 different bank groups for ds_read_b128, the last the
-// rows of one ds_read_b64_tr_b16 on different 32-byte bank groups).  Whole kernels still count conflicts: 0.09 (forward),
-// 0.07 (dX) and 0.3 (dW, both operands of the second kind) conflict clocks per clock of LDS instructions (Mixtral shape),
-// of fragment reads, incoming transfers and staged epilogue together; which of them was not taken apart.
+// rows of one ds_read_b64_tr_b16 on different 32-byte bank groups).  Whole kernels, conflict clocks per clock of LDS
+// instructions (8 groups, 4096 x 14336): dW, both operands WIDE, none (0.31 with the transposing reads); forward 0.04 (0.09), dX
+// 0.03 (K 28672) and 0.16 (K 4096); which of fragment reads, incoming transfers and staged epilogue was not taken apart.
 constexpr int kStageTile = 256 * BK * 2;      // bytes of one operand in one stage (32 KB)
 constexpr int kAStages = 2, kBStages = 3;     // 5 x 32 KB: the compute unit's whole 160 KB
 constexpr int kDmaBytes = (kAStages + kBStages) * kStageTile;
@@ -338,14 +338,6 @@ __device__ __forceinline__ void settle(f32x4 (&acc)[TM][TN]) {
     pin(acc);
 }
 
-// K loop of a 256 x 256 tile: 2 x 2 wavefronts of 128 x 128 = 8 x 8 blocks of 16 x 16, K steps of 64 = two 32-wide
-// slices.  acc[i][j][e] = C[wm*128 + i*16 + (lane & 15)][wn*128 + j*16 + 4*(lane >> 4) + e].
-//
-// Step kt multiplies slice 0 (its fragments are in registers already) while slice 1's fragments are read, then, after
-// the step's only barrier, slice 1 while slice 0 of tile kt+1 is read.  At the barrier every wavefront has all of tile
-// kt in registers and all its transfers of tile kt+1 have landed, so behind it tile kt's stages are free (the transfers
-// of A's tile kt+2 go there at once; B, with three stages, has its tile kt+2 requested in the first half of the step
-// after the one that freed it) and tile kt+1 can be read.
 // Slots of a slice (64 products) that take raw reads apart, and how many of them lie ahead of slot u: none beside a read, none
 // beside a request (slot busy of every eight) or right behind it.  (Two dwords in every slot from the twelfth on, whatever
 // else is in it: dW 1150 instead of 1177 TFLOP/s, forward 1349 instead of 1389.)
@@ -358,6 +350,15 @@ constexpr int idle_before(int u, int busy) {
 constexpr int kBusyB = 5, kBusyA = 1;       // slots of every eight that request a transfer of B (slice 0) and of A (slice 1)
 static_assert(idle_before(64, kBusyB) >= 32 && idle_before(64, kBusyA) >= 32, "both operands' dwords find their slots");
 
+// K loop of a 256 x 256 tile: 2 x 2 wavefronts of 128 x 128 = 8 x 8 blocks of 16 x 16, K steps of 64 = two 32-wide
+// slices.  acc[i][j][e] = C[wm*128 + row][wn*128 + col], with r = lane & 15 and c = 4*(lane >> 4) + e: row = i*16 + r, or 8*r + i of
+// an A that is not reduction-contiguous (its blocks hold every eighth row); col = j*16 + c, or 8*c + j likewise.
+//
+// Step kt multiplies slice 0 (its fragments are in registers already) while slice 1's fragments are read, then, after
+// the step's only barrier, slice 1 while slice 0 of tile kt+1 is read.  At the barrier every wavefront has all of tile
+// kt in registers and all its transfers of tile kt+1 have landed, so behind it tile kt's stages are free (the transfers
+// of A's tile kt+2 go there at once; B, with three stages, has its tile kt+2 requested in the first half of the step
+// after the one that freed it) and tile kt+1 can be read.
 template <int DT, bool A_RED, bool B_RED, bool SWIGLU>
 __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc, char *lds, int row0, int col0,
                                            f32x4 (&acc)[8][8]) {
@@ -827,7 +828,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
         if (kt + 1 == nk) { k_step(std::false_type{}, std::false_type{}, std::false_type{}); ++kt; }
     }
 
-    // Epilogue.  sums.quad(i, q)[e] = C[row0 + wm*TM*32 + i*MB + lane % MB][col0 + wn*TN*32 + col(q) + e]
+    // Epilogue.  sums.quad(i, q)[e] = C[row0 + wm*TM*32 + real_row(i*MB + lane % MB)][col0 + wn*TN*32 + col(q) + e]
     MS_TRACE(4);
     using Acc = decltype(sums);
     const int qrow = lane & (Acc::MB - 1);
@@ -835,7 +836,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     constexpr int WR = TM * 32, WC = TN * 32;       // this wavefront's block of the tile
     if constexpr (OUT == OUT_SAME || OUT == OUT_SWIGLU || OUT == OUT_SWIGLU_GRAD) {
         // 16-bit output: each wavefront stages its block in its own LDS region (row pitch WC*2 + 16 bytes, so that the
-        // 8-byte column-slice writes of a 16 x 16 block start on different banks in all its rows) and writes it out as
+        // column-slice writes of a 16 x 16 block, 8 bytes or 16 of a WIDE B, start on different banks in all its rows) and writes it out as
         // 16 bytes per lane, WC*2 contiguous bytes per row.
         constexpr int SP = WC * 2 + 16;
         static_assert(WR * SP <= kStagePerWave, "staging region too small");
