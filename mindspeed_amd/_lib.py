@@ -78,6 +78,9 @@ _INTERNAL = {
                                 _c_void_p, _c_void_p, _c_void_p, _int, _c_void_p, _c_void_p, _c_void_p, _size_t],
     "msi_unpermute_grad": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _i64, _i64, _i64, _int, _i64,
                            _c_void_p, _c_void_p, _c_void_p],
+    "msi_gmm_backward_workspace_size": [_i64, _i64, _i64, _i64, _int, _int, _int, ctypes.POINTER(_size_t)],
+    "msi_gmm_backward": [_c_void_p, _c_void_p, _i64, _i64, _c_void_p, _i64, _i64, _c_void_p, _i64, _i64, _i64, _c_void_p, _c_void_p,
+                         _c_void_p, _int, _i64, _i64, _i64, _i64, _int, _int, _int, _c_void_p, _size_t],
     "msi_gmm_takes_together": [ctypes.POINTER(_i64), _i64, _i64, _i64, _int, _int, ctypes.POINTER(_int)],
 }
 EXPORTED_SYMBOLS = tuple(_SIGNATURES) + ("ms_last_error",)

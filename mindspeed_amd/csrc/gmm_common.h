@@ -255,10 +255,9 @@ __device__ __forceinline__ void deal_tile(TileCoord &tc, int j, int num_col_tile
 // LISTS: the kernel may meet per-XCD lists (the fast kernels of the split on rows); the others are compiled without that
 // path, which costs the weight-gradient kernel 0.3 us per tile at its start when it is merely present.
 template <bool LISTS, bool ROWS>
-__device__ __forceinline__ TileCoord locate_tile(const TileTable *table) {
+__device__ __forceinline__ TileCoord locate_tile(const TileTable *table, int b) {
     TileCoord tc;
     tc.valid = false;
-    const int b = blockIdx.x;
     if ((b >> 3) >= table->slots_per_xcd) return tc;
     if (LISTS && table->num_entries == 0) {     // per-XCD lists (the common table is empty then); no further header
                                                 // field is read on the way to the common case
@@ -319,11 +318,10 @@ __host__ __device__ __forceinline__ int small_tile_rows(int rem) { return rem <=
 // table_places).
 constexpr int kMaxDirectGroups = 64;
 template <bool SPLIT_RED>
-__device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
+__device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p, int b) {
     TileCoord tc;
     tc.valid = false;
     const int lane = threadIdx.x & 63;
-    const int b = blockIdx.x;
     const int C = p.num_col_tiles;
     const unsigned m = static_cast<unsigned>(p.m);
     const bool mine = lane < p.num_groups;
@@ -427,8 +425,8 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p) {
 // compiled for one of the two.
 template <bool SPLIT_RED>
 __device__ __forceinline__ TileCoord locate(const GmmArgs &p) {
-    if (p.group_list != nullptr) return tile_from_list<SPLIT_RED>(p);
-    return locate_tile<false, !SPLIT_RED>(p.table);
+    if (p.group_list != nullptr) return tile_from_list<SPLIT_RED>(p, blockIdx.x);
+    return locate_tile<false, !SPLIT_RED>(p.table, blockIdx.x);
 }
 // ... nor for one kind of split
 __device__ __forceinline__ TileCoord locate_any(const GmmArgs &p) { return p.group_type == 2 ? locate<true>(p) : locate<false>(p); }
@@ -474,11 +472,15 @@ __device__ __forceinline__ const char *uniform(const char *p) {
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 
-// Fast 16-bit kernels (gmm_fast.hip).  Returns MS_OK after launching, or -1 if
+// Fast 16-bit kernels (gmm_fast.hip, gmm_pair.hip).  Returns MS_OK after launching, or -1 if
 // this problem does not meet the fast kernels' alignment conditions.
 // lists: the table may come as per-XCD lists (only asked of the weight-gradient product, whose common kernel is compiled
 // without that lookup; the kernels of the split on rows always have it).
 int launch_gmm16_fast(hipStream_t stream, const GmmArgs &args, int dtype, int out_mode, bool a_red, bool b_red,
                       unsigned grid, bool lists = false);
+// dX (both operands contiguous along the reduction dim) and dW (neither) of one matmul in one launch (gmm_pair.hip); out_mode:
+// dW's.  dw_first: its workgroups come first.  direct: tiles from the group list, else from the two tables.
+int launch_gmm16_pair(hipStream_t stream, const GmmArgs &dx, unsigned dx_grid, const GmmArgs &dw, unsigned dw_grid, int dtype,
+                      int out_mode, bool dw_first, bool direct);
 
 }  // namespace ms

@@ -25,6 +25,16 @@ int msi_unpermute_grad(ms_stream_t stream, const void *permuted_tokens, const vo
                        const int32_t *row_id_map, const void *probs, int probs_dtype, int64_t num_tokens, int64_t topk,
                        int64_t hidden, int dtype, int64_t num_rows, const int32_t *sorted_flat, void *grad_permuted,
                        void *grad_probs);
+/* Both gradients of one grouped matmul y = x w (split on rows): dx [m, k] = grad w^T and dw [num_groups, k, n] = x^T grad (fp32
+ * with accumulate: added to), the two ms_gmm calls of the backward pass in one.  grad [m, n], x [m, k], weight [num_groups, k, n]
+ * by strides; dx and dw contiguous. */
+int msi_gmm_backward_workspace_size(int64_t num_groups, int64_t m, int64_t k, int64_t n, int dtype, int dw_dtype,
+                                    int accumulate, size_t *bytes);
+int msi_gmm_backward(ms_stream_t stream, const void *grad, int64_t grad_stride0, int64_t grad_stride1, const void *x,
+                     int64_t x_stride0, int64_t x_stride1, const void *weight, int64_t w_stride_group, int64_t w_stride0,
+                     int64_t w_stride1, void *dx, void *dw, const int64_t *group_list, int group_list_type,
+                     int64_t num_groups, int64_t m, int64_t k, int64_t n, int dtype, int dw_dtype, int accumulate,
+                     void *workspace, size_t workspace_bytes);
 /* Diagnostic, host only: whether a 16-bit launch split on rows with these group sizes (a host array) gives every XCD
  * consecutive tiles of the whole launch instead of an eighth of every group's, by the rule of the lookup in the group list
  * (from_list != 0) or of the schedule kernel's table; num_cus: the GPU's compute units.  Evaluates the functions the kernels

@@ -51,6 +51,8 @@ struct Api {
     MS_API(ms_swiglu_grad)
     MS_API(msi_routing_map_permute)
     MS_API(msi_unpermute_grad)
+    MS_API(msi_gmm_backward_workspace_size)
+    MS_API(msi_gmm_backward)
 #undef MS_API
 } api;
 
@@ -88,6 +90,8 @@ void bind(const std::string &path, py::object error) {
     MS_FIND(ms_swiglu_grad)
     MS_FIND(msi_routing_map_permute)
     MS_FIND(msi_unpermute_grad)
+    MS_FIND(msi_gmm_backward_workspace_size)
+    MS_FIND(msi_gmm_backward)
 #undef MS_FIND
     error_class = error.release().ptr();
 }
@@ -154,6 +158,23 @@ bool gmm_out(const Tensor &x, const Tensor &w, const Tensor &gl, int64_t group_t
     if (code(x) < 0) return false;
     const c10::DeviceGuard guard(x.device());
     return gmm_launch(x, w, gl, group_type, list_type, out, accumulate);
+}
+
+OptTensor gmm_backward(const Tensor &grad, const Tensor &x, const Tensor &w, const Tensor &gl, int64_t list_type, const Tensor &dw,
+                       bool accumulate) {
+    if (code(x) < 0) return {};
+    const c10::DeviceGuard guard(x.device());
+    const int64_t m = x.size(0), k = x.size(1), n = w.size(2), groups = gl.numel();
+    const int dw_dtype = dw.scalar_type() == at::kFloat ? MS_FP32 : code(x);
+    const Tensor dx = at::empty({m, k}, x.options());
+    size_t bytes = 0;
+    check(api.msi_gmm_backward_workspace_size(groups, m, k, n, code(x), dw_dtype, accumulate, &bytes), "msi_gmm_backward_workspace_size");
+    const Tensor ws = workspace(bytes, x);
+    check(api.msi_gmm_backward(stream_of(x), ptr(grad), grad.stride(0), grad.stride(1), ptr(x), x.stride(0), x.stride(1), ptr(w),
+                               w.stride(0), w.stride(1), w.stride(2), ptr(dx), ptr(dw), gl.const_data_ptr<int64_t>(),
+                               static_cast<int>(list_type), groups, m, k, n, code(x), dw_dtype, accumulate, ptr(ws), ws.numel()),
+          "ms_gmm");
+    return dx;
 }
 
 std::optional<std::tuple<Tensor, Tensor>> gmm_swiglu(const Tensor &x, const Tensor &w, const Tensor &gl, int64_t list_type,
@@ -332,6 +353,7 @@ PYBIND11_MODULE(_host, mod) {
     const py::call_guard<py::gil_scoped_release> no_gil;      // (a launch may wait for a full queue)
     mod.def("gmm", &gmm, no_gil);
     mod.def("gmm_out", &gmm_out, no_gil);
+    mod.def("gmm_backward", &gmm_backward, no_gil);
     mod.def("gmm_swiglu", &gmm_swiglu, no_gil);
     mod.def("moe_token_permute", &token_permute, no_gil);
     mod.def("moe_token_permute_grad", &token_permute_grad, no_gil);

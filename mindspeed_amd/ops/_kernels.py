@@ -105,6 +105,33 @@ _define("gmm_out(Tensor x, Tensor weight, Tensor group_list, int group_type, int
         "Tensor(a!) out, bool accumulate) -> ()", _gmm_out, lambda *a: None)
 
 
+def _gmm_backward(grad, x, weight, group_list, group_list_type, dw, accumulate):
+    if flop_counter.recording():                 # (each product by itself, so that each has an entry of its own)
+        _gmm_launch(x.t(), grad, group_list, 2, group_list_type, dw, accumulate)
+        return _gmm(grad, weight.transpose(1, 2), group_list, 0, group_list_type)
+    lib = _lib.load()
+    dev = x.device
+    (m, k), n, num_groups = x.shape, weight.size(2), group_list.numel()
+    dtype = _lib.dtype_code(x.dtype, "x")
+    dw_dtype = _lib.MS_FP32 if dw.dtype == torch.float32 else dtype
+    dx = torch.empty((m, k), dtype=x.dtype, device=dev)
+    nbytes = ctypes.c_size_t(0)
+    _lib.check(lib.msi_gmm_backward_workspace_size(num_groups, m, k, n, dtype, dw_dtype, 1 if accumulate else 0,
+                                                   ctypes.byref(nbytes)), "msi_gmm_backward_workspace_size")
+    ws = _lib.workspace(nbytes.value, dev)
+    with _lib.on(dev):
+        _lib.check(lib.msi_gmm_backward(
+            _lib.stream_ptr(dev), _lib.ptr(grad), *grad.stride(), _lib.ptr(x), *x.stride(), _lib.ptr(weight), *weight.stride(),
+            _lib.ptr(dx), _lib.ptr(dw), _lib.ptr(group_list), group_list_type, num_groups, m, k, n, dtype, dw_dtype,
+            1 if accumulate else 0, _lib.ptr(ws), ws.numel()), "ms_gmm")
+    return dx
+
+
+_define("gmm_backward(Tensor grad, Tensor x, Tensor weight, Tensor group_list, int group_list_type, Tensor(a!) dw, "
+        "bool accumulate) -> Tensor", _gmm_backward,
+        lambda grad, x, weight, group_list, group_list_type, dw, accumulate: x.new_empty((x.size(0), x.size(1))))
+
+
 # ---- token permute / unpermute -----------------------------------------------------------------------------
 def _permute_shapes(tokens, indices, num_out, num_experts, want_sorted, want_counts):
     num_tokens, hidden = tokens.shape

@@ -18,7 +18,7 @@ import torch
 
 from .. import _lib, flop_counter
 from ._kernels import K, _plain
-from .npu_groupmatmul_add import add_weight_gradient
+from .npu_groupmatmul_add import add_weight_gradient, gradient_list
 
 __all__ = ["npu_gmm", "npu_gmm_v2", "GMMFunction"]
 
@@ -92,6 +92,31 @@ def gmm_raw(x, weight, group_list, group_type, group_list_type, out=None, accumu
     return out
 
 
+def _one_call(grad, x, weight, gl, dw) -> bool:
+    """Whether both gradients of ``y [M, N] = x [M, K] weight [E, K, N]`` can be one kernel call as the operands are; what
+    cannot, mistakes included, goes through :func:`gmm_raw` product by product."""
+    if x.dim() != 2 or grad.dim() != 2 or weight.dim() != 3 or gl.dim() != 1 or gl.dtype != torch.int64:
+        return False
+    dtype, dev = x.dtype, x.device
+    if dtype not in (torch.bfloat16, torch.float16, torch.float32) or dev.type not in ("cuda", "meta"):
+        return False
+    (m, k), (groups, wk, n) = x.shape, weight.shape
+    return (grad.dtype == dtype and weight.dtype == dtype and grad.device == dev and weight.device == dev and dw.device == dev
+            and grad.size(0) == m and grad.size(1) == n and wk == k and groups == gl.numel()
+            and dw.dtype in (torch.float32, dtype) and dw.is_contiguous() and dw.numel() == groups * k * n
+            and all(_unit_stride_view(t) is t for t in (grad, x, weight)))
+
+
+def gmm_backward_raw(grad, x, weight, group_list, group_list_type, dw, accumulate=False):
+    """The gradients of ``y = gmm_raw(x, weight, group_list, 0)``: returns ``dx`` and fills ``dw`` (contiguous, of the
+    weight's size, in x's dtype or fp32; with ``accumulate`` the result is added, fp32 only)."""
+    gl = _group_list_tensor(group_list, x.device)
+    if (dw.dtype == torch.float32 or not accumulate) and _one_call(grad, x, weight, gl, dw):
+        return K.gmm_backward(grad, x, weight, gl, group_list_type, dw, bool(accumulate))
+    gmm_raw(x.transpose(-1, -2), grad, gl, 2, group_list_type, out=dw, accumulate=accumulate)
+    return gmm_raw(grad, weight.transpose(-1, -2), gl, 0, group_list_type)
+
+
 def gmm_raw_weight_list(x, weights, group_list, group_list_type, transposed=False):
     """``y[rows of group g] = x[rows of g] @ W_g`` with one separately allocated matrix per group.
 
@@ -132,11 +157,10 @@ def gmm_raw_weight_list(x, weights, group_list, group_list_type, transposed=Fals
 
 
 # dX and dW of one grouped matmul are independent; each is a full-chip kernel whose last round of tiles may leave
-# compute units idle.  With MINDSPEED_AMD_OVERLAP_WGRAD=1 the weight-gradient product is launched on a second stream
-# (default priority) between two joins with the caller's stream, so its tiles fill the other kernel's tail and vice
-# versa.  Off by default: since the dX launch cuts its last-round tail tiles into parts along the reduction it ends
-# with a full round by itself, and running the two kernels one after the other measures 0.8 % faster per step on the
-# Mixtral and DeepSeek-share shapes (equal on the Qwen-like one).
+# compute units idle.  By default they are one kernel call (gmm_backward_raw), whose tiles fill each other's last round.
+# With MINDSPEED_AMD_OVERLAP_WGRAD=1 the weight-gradient product is launched on a second stream (default priority)
+# between two joins with the caller's stream instead, which fills the last rounds too but has the two kernels' tiles
+# take each other's panels out of the L2s all along, and costs the host two events per pair.
 OVERLAP_WGRAD = os.environ.get("MINDSPEED_AMD_OVERLAP_WGRAD", "0") != "0"
 _side_streams = {}
 
@@ -241,7 +265,11 @@ class _RawGmmModule:
         w = weight[0]
         num_groups = len(group_list) if not isinstance(group_list, torch.Tensor) else group_list.numel()
         dw = torch.empty((num_groups, x[0].size(-1), grad[0].size(-1)), dtype=x[0].dtype, device=x[0].device)
-        with _beside(grad[0]) as side:
+        side = _beside(grad[0])
+        if not side.active:
+            dx = gmm_backward_raw(grad[0], x[0], w, group_list, glt, dw)
+            return [dx], [dw.reshape(w.shape)], []
+        with side:
             gmm_raw(x[0].transpose(-1, -2), grad[0], group_list, 2, glt, out=dw)
         dx = gmm_raw(grad[0], w.transpose(-1, -2), group_list, 0, glt)
         side.join()
@@ -308,12 +336,18 @@ class GMMFunction(torch.autograd.Function):
             (dx,), (dw,), dbias = module.npu_gmm_backward([grad_y], [x], [weight], group_list, ctx.group_list_type)
             return None, dx, dw, (dbias[0] if dbias else None), None
         # gemm_fusion (gmm.py:56-89): the weight gradient is added into original_weight.main_grad (fp32) by the
-        # accumulate form of the dW product, here on the side stream beside dX; what autograd gets for the weight is
+        # accumulate form of the dW product, in one launch with dX or on the side stream beside it; what autograd gets for the weight is
         # a placeholder (zeros if the parameter asks for it) and the flag the optimizer wrapper looks at is set.
-        with _beside(grad_y) as side:
-            add_weight_gradient(x, grad_y, group_list, ctx.group_list_type, original_weight.main_grad)
-        (dx,), _, dbias = module.npu_gmm_backward_fusion([grad_y], [weight], group_list, ctx.group_list_type)
-        side.join()
+        side = _beside(grad_y)
+        if side.active:
+            with side:
+                add_weight_gradient(x, grad_y, group_list, ctx.group_list_type, original_weight.main_grad)
+            (dx,), _, dbias = module.npu_gmm_backward_fusion([grad_y], [weight], group_list, ctx.group_list_type)
+            side.join()
+        else:
+            main_grad = original_weight.main_grad
+            gl = gradient_list(x, grad_y, group_list, main_grad)
+            dx, dbias = gmm_backward_raw(grad_y, x, weight, gl, ctx.group_list_type, main_grad, accumulate=True), []
         placeholder = None
         if hasattr(original_weight, "grad_added_to_main_grad"):
             make = torch.zeros if getattr(weight, "zero_out_wgrad", False) else torch.empty

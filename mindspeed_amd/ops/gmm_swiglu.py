@@ -21,7 +21,7 @@ import torch
 
 from .. import _lib
 from ._kernels import K
-from .gmm import _beside, _group_list_tensor, _tracing, gmm_raw
+from .gmm import _beside, _group_list_tensor, _tracing, gmm_backward_raw, gmm_raw
 
 __all__ = ["gmm_swiglu", "GmmSwigluFunction", "grouped_mlp", "GroupedMLPFunction"]
 
@@ -75,11 +75,15 @@ class GmmSwigluFunction(torch.autograd.Function):
         dx = dw = None
         if ctx.needs_input_grad[1]:
             dw = torch.empty(weight.shape, dtype=weight.dtype, device=dev)
-            with _beside(d_fc1) as side:
-                gmm_raw(x.t(), d_fc1, gl, 2, glt, out=dw)
-            if ctx.needs_input_grad[0]:
-                dx = gmm_raw(d_fc1, weight.transpose(1, 2), gl, 0, glt)
-            side.join()
+            side = _beside(d_fc1)
+            if ctx.needs_input_grad[0] and not side.active:
+                dx = gmm_backward_raw(d_fc1, x, weight, gl, glt, dw)
+            else:
+                with side:
+                    gmm_raw(x.t(), d_fc1, gl, 2, glt, out=dw)
+                if ctx.needs_input_grad[0]:
+                    dx = gmm_raw(d_fc1, weight.transpose(1, 2), gl, 0, glt)
+                side.join()
         elif ctx.needs_input_grad[0]:
             dx = gmm_raw(d_fc1, weight.transpose(1, 2), gl, 0, glt)
         gp_out = gp.view(ctx.probs_shape) if (gp is not None and ctx.needs_input_grad[4]) else None
@@ -182,19 +186,25 @@ class GroupedMLPFunction(torch.autograd.Function):
         dw1 = torch.empty(w1.shape, dtype=w1.dtype, device=dev) if ctx.needs_input_grad[1] else None
         dw2 = torch.empty(w2.shape, dtype=w2.dtype, device=dev) if ctx.needs_input_grad[2] else None
         side = _beside(dy)
-        with side:                                   # dW2 needs only act and dy
-            if dw2 is not None:
-                gmm_raw(act.t(), dy, gl, 2, glt, out=dw2)
         if ctx.fused_kernels:
             w2 = _vector_rows(w2)
-        dact = gmm_raw(dy, w2.transpose(1, 2), gl, 0, glt)
+        if dw2 is not None and not side.active:
+            dact = gmm_backward_raw(dy, act, w2, gl, glt, dw2)
+        else:
+            with side:                               # dW2 needs only act and dy
+                if dw2 is not None:
+                    gmm_raw(act.t(), dy, gl, 2, glt, out=dw2)
+            dact = gmm_raw(dy, w2.transpose(1, 2), gl, 0, glt)
         d_fc1, gp = _swiglu_grad_from_fc1(dact, fc1, p)
         del dact
-        with side.again():                           # dW1 needs d_fc1: the side stream picks up from here
-            if dw1 is not None:
-                gmm_raw(x.t(), d_fc1, gl, 2, glt, out=dw1)
-        dx = gmm_raw(d_fc1, w1.transpose(1, 2), gl, 0, glt) if ctx.needs_input_grad[0] else None
-        side.join()
+        if dw1 is not None and ctx.needs_input_grad[0] and not side.active:
+            dx = gmm_backward_raw(d_fc1, x, w1, gl, glt, dw1)
+        else:
+            with side.again():                       # dW1 needs d_fc1: the side stream picks up from here
+                if dw1 is not None:
+                    gmm_raw(x.t(), d_fc1, gl, 2, glt, out=dw1)
+            dx = gmm_raw(d_fc1, w1.transpose(1, 2), gl, 0, glt) if ctx.needs_input_grad[0] else None
+            side.join()
         gp_out = gp.view(ctx.probs_shape) if (gp is not None and ctx.needs_input_grad[5]) else None
         return dx, dw1, dw2, None, None, gp_out, None, None, None
 

@@ -17,10 +17,8 @@ def npu_groupmatmul_add_fp32(x, dy, grouplist, grad):
     return None
 
 
-def add_weight_gradient(x, dy, grouplist, group_list_type, grad):
-    """The same for either kind of group list (0: cumulative offsets, 1: counts)."""
-    from .gmm import gmm_raw  # deferred: gmm.py imports this module
-
+def gradient_list(x, dy, grouplist, grad):
+    """``grouplist`` as a tensor, once ``grad`` is known to take the weight gradient of ``x`` and ``dy`` in place."""
     if grad.dtype != torch.float32:
         raise TypeError(f"grad must be float32, got {grad.dtype}")
     if not grad.is_contiguous():
@@ -30,4 +28,12 @@ def add_weight_gradient(x, dy, grouplist, group_list_type, grad):
     num_groups = grouplist.shape[0]
     if grad.numel() != num_groups * x.shape[-1] * dy.shape[-1]:
         raise ValueError(f"grad has {grad.numel()} elements, expected {num_groups}x{x.shape[-1]}x{dy.shape[-1]}")
+    return grouplist
+
+
+def add_weight_gradient(x, dy, grouplist, group_list_type, grad):
+    """The same for either kind of group list (0: cumulative offsets, 1: counts)."""
+    from .gmm import gmm_raw  # deferred: gmm.py imports this module
+
+    grouplist = gradient_list(x, dy, grouplist, grad)
     gmm_raw(x.transpose(-1, -2), dy, grouplist, 2, group_list_type, out=grad, accumulate=True)

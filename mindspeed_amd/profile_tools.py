@@ -48,6 +48,7 @@ GEMM_KEYS = {  # first template arguments <dtype, A reduction-contiguous, B redu
     "gmm16_fast_kernel<0, false, false, 0,": "gmm_dw",
     "gmm16_fast_kernel<0, true, false, 3,": "gmm_fwd_swiglu",
     "gmm16_fast_kernel<0, true, true, 4,": "gmm_dx_swiglu",
+    "gmm16_pair_kernel<0, 0,": "gmm_dx_and_dw",
 }
 
 

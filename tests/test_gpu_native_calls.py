@@ -36,6 +36,8 @@ CALLS = {
     "gmm_transposed": lambda i: ("gmm", i.dy, i.w.transpose(1, 2), i.counts, 0, 1),
     "gmm_out": lambda i: ("gmm_out", i.x.t(), i.dy, i.counts, 2, 1, i.out, False),
     "gmm_out_accumulate": lambda i: ("gmm_out", i.x.t(), i.dy, i.counts, 2, 1, i.acc, True),
+    "gmm_backward": lambda i: ("gmm_backward", i.dy, i.x, i.w, i.counts, 1, torch.empty_like(i.w), False),
+    "gmm_backward_accumulate": lambda i: ("gmm_backward", i.dy, i.x, i.w, i.counts.cumsum(0), 0, i.acc, True),
     "gmm_swiglu": lambda i: ("gmm_swiglu", i.x, i.w, i.counts, 1, None, True),
     "gmm_swiglu_probs_no_fc1": lambda i: ("gmm_swiglu", i.x, i.w, i.counts, 1, i.p100, False),
     "permute": lambda i: ("moe_token_permute", i.tokens, i.index, 100, 4, True, True),
@@ -71,6 +73,8 @@ def test_equals_the_python_function(case):
     if name == "gmm_out":
         assert got is True and want is None
         want, got = clones[5], args[5]
+    if name == "gmm_backward":
+        want, got = (want, clones[5]), (got, args[5])
     for a, b in zip(_flat(want), _flat(got)):
         assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
     assert len(_flat(want)) == len(_flat(got))
