@@ -11,6 +11,8 @@ from __future__ import annotations
 import torch
 
 from .ops import (fused_swiglu, grouped_mlp, moe_token_permute_with_aux, npu_gmm_v2, npu_moe_token_unpermute)
+from .ops import gmm as gmm_ops
+from .ops._kernels import native_form
 
 __all__ = ["experts_computation", "dispatch_mlp_combine"]
 
@@ -54,6 +56,12 @@ def dispatch_mlp_combine(hidden_states, top_k_index, top_k_weights, weights, num
                          fuse_activation=None, gemm_fusion=False):
     gate_up_weights, down_weights = weights
     num_experts = gate_up_weights.size(0) if num_global_experts is None else num_global_experts
+    # the same ops in one native call, wherever nothing but autograd is to see them
+    if not gemm_fusion and not gmm_ops.OVERLAP_WGRAD and num_experts.__class__ is int:
+        fused = not torch.is_grad_enabled() if fuse_activation is None else bool(fuse_activation)
+        out = native_form("layer", hidden_states, top_k_index, top_k_weights, gate_up_weights, down_weights, num_experts, fused)
+        if out is not None:
+            return out
     permuted, row_id_map, _, tokens_per_expert = moe_token_permute_with_aux(
         hidden_states, top_k_index, num_experts=num_experts)
     out = experts_computation(permuted, tokens_per_expert, gate_up_weights, down_weights, fuse_activation, gemm_fusion)

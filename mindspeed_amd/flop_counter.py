@@ -73,13 +73,28 @@ class Recorder:
 
 @contextlib.contextmanager
 def record(timing=True):
-    global _active
     prev, rec = _active, Recorder(timing)
-    _active = rec
+    _activate(rec)
     try:
         yield rec
     finally:
-        _active = prev
+        _activate(prev)
+
+
+_listeners = []
+
+
+def _activate(rec):
+    global _active
+    _active = rec
+    for listener in _listeners:
+        listener(rec is not None)
+
+
+def on_change(listener):
+    """``listener(whether a recorder takes note of every op)``, now and whenever that changes."""
+    _listeners.append(listener)
+    listener(recording())
 
 
 def timing_active() -> bool:

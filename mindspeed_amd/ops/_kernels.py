@@ -671,9 +671,21 @@ def _load_native():
         _native = {}
         return _native
     _host.bind(_lib.LIB_PATH, _lib.MindSpeedAmdError)
+    _host.record_through(_DEVICE_FNS)
+    flop_counter.on_change(_host.set_recording)
     _plain_check = _host.plain
-    _native = {name: getattr(_host, name) for name in _DEVICE_FNS if hasattr(_host, name)}
+    _native = {name: getattr(_host, name) for name in (*_DEVICE_FNS, "layer", "map_permute", "map_unpermute") if hasattr(_host, name)}
     return _native
+
+
+def native_form(name, *args):
+    """What the native function ``name`` (``layer``, ``map_permute``, ``map_unpermute``: several ops with their autograd
+    nodes) returns, None where the call has to go op by op: a compiler is tracing, a Recorder wants every op, or the function
+    does not take these arguments."""
+    if flop_counter.recording() or torch.compiler.is_compiling():
+        return None
+    fn = (_native if _native is not None else _load_native()).get(name)
+    return None if fn is None else fn(*args)
 
 
 class _Ops:

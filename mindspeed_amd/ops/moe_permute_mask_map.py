@@ -34,7 +34,7 @@ import weakref
 import torch
 
 from .. import _lib
-from ._kernels import K
+from ._kernels import K, native_form
 
 __all__ = ["permute", "unpermute", "MoePermuteMaskMap", "MoeUnpermuteMaskMap", "routing_map_row_maps"]
 
@@ -287,6 +287,30 @@ class MoeUnpermuteMaskMap(torch.autograd.Function):
         return grad_permuted, None, None, grad_probs, None, None
 
 
+def _permute(tokens, routing_map, probs, num_out_tokens, drop_and_pad):
+    """:class:`MoePermuteMaskMap`, in native code where that takes the call."""
+    out = native_form("map_permute", tokens, routing_map, probs, num_out_tokens, bool(drop_and_pad))
+    if out is None:
+        return MoePermuteMaskMap.apply(tokens, routing_map, probs, num_out_tokens, drop_and_pad)
+    permuted, row_id_map, sorted_flat, permuted_probs, sorted_indices, num_rows = out
+    _remember_row_map(routing_map, num_rows, drop_and_pad, row_id_map, sorted_flat, sorted_indices)
+    return permuted, permuted_probs, sorted_indices
+
+
+def _unpermute_by_kept_map(permuted_tokens, sorted_indices, restore_shape, probs, routing_map, drop_and_pad):
+    """:class:`MoeUnpermuteMaskMap` in native code, for a mask whose row map an earlier ``permute`` left behind and indices
+    that are known to agree with it; None for any other call."""
+    if permuted_tokens.__class__ is not torch.Tensor or routing_map.__class__ is not torch.Tensor or permuted_tokens.dim() != 2:
+        return None
+    rows = permuted_tokens.size(0)
+    if getattr(routing_map, "_ms_row_maps", None) is None or sorted_indices.numel() != rows:
+        return None
+    kept = _recall_row_map(routing_map, rows, drop_and_pad)
+    if kept is None or (_CHECK_SORTED_INDICES and not _is_known(kept[2], sorted_indices)):
+        return None
+    return native_form("map_unpermute", permuted_tokens, kept[0], kept[1], probs, routing_map, int(restore_shape[0]), bool(drop_and_pad))
+
+
 def permute(tokens, routing_map, probs: Optional[torch.Tensor] = None, num_out_tokens: Optional[int] = None,
             fused: bool = False, drop_and_pad: bool = False):
     """``(permuted_tokens, permuted_probs, sorted_indices)`` for a bool ``routing_map`` ``[T, E]``.
@@ -306,13 +330,12 @@ def permute(tokens, routing_map, probs: Optional[torch.Tensor] = None, num_out_t
     mixed = (fused and isinstance(probs, torch.Tensor)
              and (tokens.dtype == torch.float32) != (probs.dtype == torch.float32))
     if not mixed:
-        return MoePermuteMaskMap.apply(tokens, routing_map, probs, num_out_tokens, drop_and_pad)
+        return _permute(tokens, routing_map, probs, num_out_tokens, drop_and_pad)
     if tokens.dtype != torch.float32:          # 16-bit tokens, fp32 probabilities: both results in the tokens' dtype
-        permuted, permuted_probs, sorted_indices = MoePermuteMaskMap.apply(
-            tokens, routing_map, probs, num_out_tokens, drop_and_pad)
+        permuted, permuted_probs, sorted_indices = _permute(tokens, routing_map, probs, num_out_tokens, drop_and_pad)
         return permuted, permuted_probs.to(tokens.dtype), sorted_indices
     low = probs.dtype                          # fp32 tokens, 16-bit probabilities: both results in the probs' dtype
-    permuted, permuted_probs, sorted_indices = MoePermuteMaskMap.apply(
+    permuted, permuted_probs, sorted_indices = _permute(
         tokens, routing_map, probs.to(torch.float32), num_out_tokens, drop_and_pad)
     return permuted.to(low), permuted_probs.to(low), sorted_indices
 
@@ -323,4 +346,7 @@ def unpermute(permuted_tokens: torch.Tensor, sorted_indices: torch.Tensor, resto
     """``out[t] = sum_e probs[t, e] * permuted_tokens[row of (t, e)]`` over the mapped entries of token ``t``
     (weights 1 without ``probs``); fp32 accumulation, one rounding.  ``routing_map`` is required: the row
     of an entry is recomputed from it on the device."""
+    out = _unpermute_by_kept_map(permuted_tokens, sorted_indices, restore_shape, probs, routing_map, drop_and_pad)
+    if out is not None:
+        return out
     return MoeUnpermuteMaskMap.apply(permuted_tokens, sorted_indices, restore_shape, probs, routing_map, drop_and_pad)
