@@ -921,7 +921,16 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
                 const int r = pass * RPP + lane / LPR;
                 const int row = row0 + wm * WR + r;
                 const v16 v = *reinterpret_cast<const v16 *>(stg + Acc::staged_row(r) * SP + chunk * 16);
-                if (col_ok && row < row_end) *reinterpret_cast<v16 *>(cbase + static_cast<int64_t>(row) * ldc) = v;
+                if (col_ok && row < row_end) {
+                    v16 *dst = reinterpret_cast<v16 *>(cbase + static_cast<int64_t>(row) * ldc);
+                    // Weight gradients go past the last-level cache: nothing on the way reads them, and as ordinary
+                    // stores they put out what the next kernel reads and have it wait for their write-back.  us per
+                    // training pass, ordinary / non-temporal: 16 experts x 750 rows x 2048 x 1536 752 / 732, 64 of 0 to
+                    // 7700 rows x 2048 x 1408 3506 / 3483, 8 x 2048 rows x 7168 x 2048 3510 / 3497, 8 x 1024 rows x 4096 x
+                    // 14336 7117 / 7110.
+                    if constexpr (A_RED) *dst = v;
+                    else MS_NT_STORE(v, dst);
+                }
             }
         }
         if constexpr (SWIGLU) {
