@@ -105,6 +105,14 @@ __device__ __forceinline__ void store_float_as(void *p, int64_t i, int dtype, fl
     }
 }
 
+// 1 / (1 + exp(-x)) of a 16-bit value, for results that are rounded to 16 bits.  The reciprocal instruction (1 ulp) and one Newton
+// step, four instructions where the division takes ten.  Past exp's overflow the step's factor is NaN, which fmaxf takes out: 0.
+__device__ __forceinline__ float sigmoid16(float x) {
+    const float d = 1.f + __expf(-x);
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaxf(fmaf(-d, r, 1.f), -1.f), r, r);
+}
+
 // ---- prefix sums over the lanes of a wavefront ----------------------------------
 // v moved over the lanes (data-parallel primitives: 8 clocks each, a shuffle through LDS takes a hundred); lanes without a
 // source get 0.

@@ -7,7 +7,11 @@
 namespace ms {
 namespace {
 
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
+template <typename DT>
+__device__ __forceinline__ float sigmoid_of(float x) {
+    if constexpr (sizeof(typename DT::storage) == 2) return sigmoid16(x);
+    else return 1.f / (1.f + __expf(-x));
+}
 
 template <typename DT, int VEC>
 __global__ __launch_bounds__(256) void swiglu_kernel(const typename DT::storage *__restrict__ x,
@@ -34,7 +38,7 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const typename DT::storage 
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             const float gf = DT::to_float(g[e]);
-            o[e] = DT::from_float(gf * sigmoidf_(gf) * DT::to_float(u[e]) * p);
+            o[e] = DT::from_float(gf * sigmoid_of<DT>(gf) * DT::to_float(u[e]) * p);
         }
         S *dst = y + r * ffn + c;
         if constexpr (VEC * sizeof(S) == 16) {
@@ -77,7 +81,7 @@ __device__ __forceinline__ float swiglu_grad_row(const typename DT::storage *__r
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             const float gf = DT::to_float(g[e]), uf = DT::to_float(u[e]), df = DT::to_float(d[e]);
-            const float sig = sigmoidf_(gf);
+            const float sig = sigmoid_of<DT>(gf);
             const float act = gf * sig;
             dot = fmaf(df, act * uf, dot);
             const float dp = df * p;

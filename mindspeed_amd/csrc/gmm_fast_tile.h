@@ -210,10 +210,12 @@ struct DmaOperand {
     unsigned tsel[8];       // !RED: swizzled 32-byte column-group offset of fragment t
 
     // outer0: first outer index of the tile; outer_last: clamp bound (RED: last valid outer index, !RED: last valid
-    // start of an 8-wide chunk); wave_outer: this wavefront's first outer index in the tile.  split (!RED only, fused
-    // SwiGLU form): the second half of the tile's outer indices lies `split` elements further on in memory than the
-    // first half's continuation would (gate columns c0 .. c0+127 and up columns ffn+c0 .. ffn+c0+127 side by side in one
-    // tile: split = ffn - 128), with the clamp bound moved along by ffn.
+    // start of an 8-wide chunk); wave_outer: this wavefront's first outer index in the tile.  The fused SwiGLU form
+    // (!RED only) has gate columns c0 .. c0+127 and up columns ffn+c0 .. ffn+c0+127 in one tile, split_last = ffn.
+    // WIDE: every wavefront has 64 gate columns and the up columns of the same numbers behind them, and its reads are
+    // dealt so that a lane's accumulators hold both of a pair (swiglu_tile).  Else the second half of the tile's outer indices
+    // lies `split` elements further on in memory than the first half's continuation would (split = ffn - 128).
+    template <bool GATE_UP = false>
     __device__ __forceinline__ void init(int64_t stride_outer, int64_t stride_red, int outer0, int outer_last,
                                          int wave_outer, int wave, int split = 0, int split_last = 0) {
         const int lane = threadIdx.x & 63;
@@ -236,14 +238,16 @@ struct DmaOperand {
             for (int i = 0; i < NX; ++i) {
                 const int rr = key + 2 * i;
                 const int cg = WIDE ? lane & 31 : (lane & 31) ^ ((rr & 3) << 2) ^ (((rr >> 3) & 1) << 1);
-                const bool second = cg >= 16;
-                int outer = outer0 + cg * 8 + (second ? split : 0);
+                const bool second = WIDE && GATE_UP ? (cg & 8) != 0 : cg >= 16;
+                int outer = outer0 + (WIDE && GATE_UP ? (cg >> 4) * 64 + (cg & 7) * 8 + (second ? split_last : 0) : cg * 8 + (second ? split : 0));
                 const int last = outer_last + (second ? split_last : 0);
                 outer = outer > last ? last : outer;
                 off[i] = static_cast<unsigned>((static_cast<int64_t>(rr) * stride_red + (outer - outer0)) * 2);
             }
             if constexpr (WIDE) {
-                frag_off = 8 * (lane >> 4) * 512 + wave_outer * 2 + (lane & 15) * 16;
+                const int r = lane & 15;
+                const int chunk = GATE_UP ? (r >> 2) * 2 + (r & 1) + (r & 2) * 4 : r;
+                frag_off = 8 * (lane >> 4) * 512 + wave_outer * 2 + chunk * 16;
                 return;
             }
             // transposing read: in each group of 16 lanes, lane L supplies the 4-element segment at
@@ -377,7 +381,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     la.init(p.a_stride_row, p.a_stride_red, row0, A_RED ? tc.e.row_end - 1 : tc.e.row_end - 8, wm * 128, wave);
     if constexpr (SWIGLU) {
         static_assert(!SWIGLU || !B_RED, "the fused SwiGLU form reads the weight along its columns");
-        lb.init(p.b_stride_col, p.b_stride_red, col0, p.cols - 8, wn * 128, wave, p.cols - BN / 2, p.cols);
+        lb.template init<true>(p.b_stride_col, p.b_stride_red, col0, p.cols - 8, wn * 128, wave, 0, p.cols);
     } else {
         lb.init(p.b_stride_col, p.b_stride_red, col0, B_RED ? p.cols - 1 : p.cols - 8, wn * 128, wave);
     }
@@ -676,6 +680,85 @@ struct Acc16 {                                  // 16 x 16 blocks
     __device__ __forceinline__ static int staged_row(int row) { return A_WIDE ? ((row & 7) << 4) + (row >> 3) : row; }
 };
 
+// Epilogue of a 256-row tile of the fused SwiGLU form, for a wavefront's 128 rows from row0 on and its 64 activation columns from
+// acol0 on: act = silu(gate) * up * prob of the rounded fc1 values, exactly what the stand-alone SwiGLU kernel computes from the
+// stored fc1 output, and that output itself where it is kept (p.c).
+// acc[i][j] holds, of row i * 16 + (lane & 15) and with g = lane >> 4, the gate columns 16 g + j and 16 g + 8 + j and the up
+// columns of the same numbers: the activation is computed where the sums are, and only what is stored passes through LDS.
+// What bounds it: 17 vector instructions per activation on compute units whose matrix cores wait.  Gate and up blocks in different
+// wavefronts, both staged, read back by the partners and divided with the division's ten instructions took 8 to 12 us per tile
+// beside 2.5 to 3 of the plain epilogue; us per pass with that and with this: inference, 1777 tokens over 32 experts, 2880 x 2880,
+// fp16 443.5 / 438.4; 24 tokens over 64, 2048 x 1408 (small tiles, the sigmoid only) 197.5 / 196.6.  In two halves, each staged and
+// written by itself, and one block of rows at a time: all of them at once cost 135 spilled registers, 470 us.
+template <int DT>
+__device__ __forceinline__ void swiglu_tile(const GmmArgs &p, const f32x4 (&acc)[8][8], char *lds, int row0, int row_end, int acol0,
+                                            int wave) {
+    using T = std::conditional_t<DT == MS_BF16, BF16, FP16>;
+    const int lane = threadIdx.x & 63, qrow = lane & 15, g = lane >> 4;
+    constexpr int HP = 256 + 16, AP = 128 + 16;         // LDS bytes per row of fc1 values and of activations
+    constexpr int ROWS = 64;                            // staged and written at a time
+    static_assert(ROWS * (HP + AP) <= kStagePerWave, "staging region too small");
+    float prob[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int row = row0 + i * 16 + qrow;
+        prob[i] = p.probs != nullptr && row < row_end ? load_scalar_as_float(p.probs, row, p.probs_dtype) : 1.f;
+    }
+    const bool keep = p.c != nullptr;
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();          // every wavefront is done reading the operand stages
+    char *fc1 = lds + wave * kStagePerWave;             // (private to this wavefront)
+    char *act = fc1 + ROWS * HP;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int m = 0; m < ROWS / 16; ++m) {
+            const int i = half * (ROWS / 16) + m;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                __attribute__((aligned(16))) uint16_t gate[8], up[8], o[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    gate[j] = T::from_float(acc[i][j][e]);
+                    up[j] = T::from_float(acc[i][j][e + 2]);
+                    const float x = T::to_float(gate[j]);
+                    o[j] = T::from_float(x * sigmoid16(x) * T::to_float(up[j]) * prob[i]);
+                }
+                *reinterpret_cast<v16 *>(act + (m * 16 + qrow) * AP + g * 32 + e * 16) = *reinterpret_cast<v16 *>(o);
+                if (keep) {
+                    char *dst = fc1 + (m * 16 + qrow) * HP + g * 32 + e * 16;
+                    *reinterpret_cast<v16 *>(dst) = *reinterpret_cast<v16 *>(gate);
+                    *reinterpret_cast<v16 *>(dst + 128) = *reinterpret_cast<v16 *>(up);
+                }
+                __builtin_amdgcn_sched_barrier(0);      // (or the sums of all rows are taken out of their registers first)
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        const int first = row0 + half * ROWS;
+        {
+            const int acol = acol0 + (lane & 7) * 8;
+            uint16_t *dst = static_cast<uint16_t *>(p.act) + acol;
+#pragma unroll
+            for (int pass = 0; pass < ROWS / 8; ++pass) {
+                const int r = pass * 8 + (lane >> 3);
+                const v16 v = *reinterpret_cast<const v16 *>(act + r * AP + (lane & 7) * 16);
+                if (acol < p.cols && first + r < row_end) *reinterpret_cast<v16 *>(dst + static_cast<int64_t>(first + r) * p.act_stride_row) = v;
+            }
+        }
+        if (keep) {
+            const int acol = acol0 + (lane & 7) * 8;
+            uint16_t *dst = static_cast<uint16_t *>(p.c) + acol + (qrow >= 8 ? p.cols : 0);
+#pragma unroll 4
+            for (int pass = 0; pass < ROWS / 4; ++pass) {
+                const int r = pass * 4 + g;
+                const v16 v = *reinterpret_cast<const v16 *>(fc1 + r * HP + qrow * 16);
+                if (acol < p.cols && first + r < row_end) *reinterpret_cast<v16 *>(dst + static_cast<int64_t>(first + r) * p.c_stride_row) = v;
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);             // the rows have been read before the next ones overwrite them
+    }
+}
+
 // One macro tile of TBM x 256 outputs.  TBM = 256: 2x2 wavefronts of 128x128; TBM = 128 / 64: 1x4 wavefronts
 // of 128x64 / 64x64.
 template <int DT, bool A_RED, bool B_RED, int OUT, int TBM>
@@ -837,7 +920,9 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     const int qrow = lane & (Acc::MB - 1);
     const int64_t ldc = p.c_stride_row;
     constexpr int WR = TM * 32, WC = TN * 32;       // this wavefront's block of the tile
-    if constexpr (OUT == OUT_SAME || OUT == OUT_SWIGLU || OUT == OUT_SWIGLU_GRAD) {
+    if constexpr (SWIGLU && TBM == 256) {
+        swiglu_tile<DT>(p, sums.v, lds, row0 + wm * WR, row_end, col0 + wn * (WC / 2), wave);
+    } else if constexpr (OUT == OUT_SAME || OUT == OUT_SWIGLU || OUT == OUT_SWIGLU_GRAD) {
         // 16-bit output: each wavefront stages its block in its own LDS region (row pitch WC*2 + 16 bytes, so that the
         // column-slice writes of a 16 x 16 block, 8 bytes or 16 of a WIDE B, start on different banks in all its rows) and writes it out as
         // 16 bytes per lane, WC*2 contiguous bytes per row.
@@ -894,7 +979,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const float gf = DTT::to_float(g[e]), uf = DTT::to_float(u[e]), df = DTT::to_float(d[e]);
-                        const float sig = 1.f / (1.f + __expf(-gf));
+                        const float sig = sigmoid16(gf);
                         const float act = gf * sig;
                         dot = fmaf(df, act * uf, dot);
                         const float dp = df * pr;
@@ -956,7 +1041,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const float gf = DTT::to_float(g[e]);
-                        o[e] = DTT::from_float(gf * (1.f / (1.f + __expf(-gf))) * DTT::to_float(u[e]) * pr);
+                        o[e] = DTT::from_float(gf * sigmoid16(gf) * DTT::to_float(u[e]) * pr);
                     }
                     *reinterpret_cast<v16 *>(abase + static_cast<int64_t>(row) * p.act_stride_row) = *reinterpret_cast<v16 *>(o);
                 }
