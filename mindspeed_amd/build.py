@@ -112,7 +112,7 @@ def compile_trace() -> str:
 
 
 def build_trace(verbose: bool = False, force: bool = True) -> str:
-    """The diagnostic variant of the library: the grouped-matmul fast kernels compiled with MS_TRACE_TILES (every
+    """The diagnostic variant of the library: the bf16 grouped-matmul fast kernels compiled with MS_TRACE_TILES (every
     workgroup records time stamps of its phases, read back with ms_trace_read; see profile_tools timeline).  Not
     loaded by anything else; select it with MINDSPEED_AMD_LIB."""
     os.makedirs(OBJ_DIR, exist_ok=True)

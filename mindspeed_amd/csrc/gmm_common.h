@@ -478,6 +478,7 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // without that lookup; the kernels of the split on rows always have it).
 int launch_gmm16_fast(hipStream_t stream, const GmmArgs &args, int dtype, int out_mode, bool a_red, bool b_red,
                       unsigned grid, bool lists = false);
+int launch_gmm16_fast_fp16(hipStream_t stream, const GmmArgs &args, int out_mode, bool a_red, bool b_red, unsigned grid, bool lists);
 // dX (both operands contiguous along the reduction dim) and dW (neither) of one matmul in one launch (gmm_pair.hip); out_mode:
 // dW's.  dw_first: its workgroups come first.  direct: tiles from the group list, else from the two tables.
 int launch_gmm16_pair(hipStream_t stream, const GmmArgs &dx, unsigned dx_grid, const GmmArgs &dw, unsigned dw_grid, int dtype,

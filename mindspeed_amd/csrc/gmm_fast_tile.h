@@ -199,7 +199,7 @@ constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 1
 
 using lds_ptr = char __attribute__((address_space(3))) *;
 
-template <bool RED, int ROWS = 256, bool WIDE = false>
+template <bool RED, int ROWS = 256, bool WIDE = false, int BLOCK_STEP = 16>
 struct DmaOperand {
     static_assert(!WIDE || (!RED && ROWS == 256), "the wide form reads 256-byte pieces of 512-byte rows");
     static_assert(RED || ROWS == 256, "the swizzle of an operand that is contiguous along its outer dim is made for 512-byte rows");
@@ -284,7 +284,7 @@ struct DmaOperand {
     // 8 * (l >> 4) .. + 7 of outer index l & 15.
     __device__ __forceinline__ v16 frag(const char *tile, int kk, int t) const {
         if constexpr (RED) {
-            return *reinterpret_cast<const v16 *>(tile + (frag_off ^ (kk << 6)) + t * 16 * 128);
+            return *reinterpret_cast<const v16 *>(tile + (frag_off ^ (kk << 6)) + t * BLOCK_STEP * 128);
         } else {
             const char *p = tile + frag_off + tsel[t] + kk * 32 * 512;
             const uint2 lo = lds_read_tr(p);
@@ -358,7 +358,8 @@ constexpr int kBusyB = 5, kBusyA = 1;       // slots of every eight that request
 static_assert(idle_before(64, kBusyB) >= 32 && idle_before(64, kBusyA) >= 32, "both operands' dwords find their slots");
 
 // K loop of a 256 x 256 tile: 2 x 2 wavefronts of 128 x 128 = 8 x 8 blocks of 16 x 16, K steps of 64 = two 32-wide
-// slices.  acc[i][j][e] = C[wm*128 + row][wn*128 + col], with r = lane & 15 and c = 4*(lane >> 4) + e: row = i*16 + r, or 8*r + i of
+// slices.  acc[i][j][e] = C[row][wn*128 + col], with r = lane & 15 and c = 4*(lane >> 4) + e: row = (2*i + wm)*16 + r (the two
+// wavefronts' blocks alternate, so that both have fewer where the tile has fewer rows: RB of eight), or wm*128 + 8*r + i of
 // an A that is not reduction-contiguous (its blocks hold every eighth row); col = j*16 + c, or 8*c + j likewise.
 //
 // Step kt multiplies slice 0 (its fragments are in registers already) while slice 1's fragments are read, then, after
@@ -366,7 +367,7 @@ static_assert(idle_before(64, kBusyB) >= 32 && idle_before(64, kBusyA) >= 32, "b
 // kt in registers and all its transfers of tile kt+1 have landed, so behind it tile kt's stages are free (the transfers
 // of A's tile kt+2 go there at once; B, with three stages, has its tile kt+2 requested in the first half of the step
 // after the one that freed it) and tile kt+1 can be read.
-template <int DT, bool A_RED, bool B_RED, bool SWIGLU>
+template <int DT, bool A_RED, bool B_RED, bool SWIGLU, int RB>
 __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc, char *lds, int row0, int col0,
                                            f32x4 (&acc)[8][8]) {
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -376,9 +377,9 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     const int nk = (red_len + BK - 1) / BK;
     if (nk <= 0) return clear(acc);
 
-    DmaOperand<A_RED, 256, !A_RED> la;
+    DmaOperand<A_RED, 256, !A_RED, A_RED ? 32 : 16> la;
     DmaOperand<B_RED, 256, !B_RED> lb;
-    la.init(p.a_stride_row, p.a_stride_red, row0, A_RED ? tc.e.row_end - 1 : tc.e.row_end - 8, wm * 128, wave);
+    la.init(p.a_stride_row, p.a_stride_red, row0, A_RED ? tc.e.row_end - 1 : tc.e.row_end - 8, A_RED ? wm * 16 : wm * 128, wave);
     if constexpr (SWIGLU) {
         static_assert(!SWIGLU || !B_RED, "the fused SwiGLU form reads the weight along its columns");
         lb.template init<true>(p.b_stride_col, p.b_stride_red, col0, p.cols - 8, wn * 128, wave, 0, p.cols);
@@ -425,7 +426,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
     // 1428.  8192 x 4096 x 28672 in 8 groups.)
     auto mfma = [&](int set, int u) {
         const int i = u >> 3, j = (i & 1) ? 7 - (u & 7) : (u & 7);
-        mfma16x16<DT>(bf[set][j], af[set][i], acc[i][j]);
+        if (i < RB) mfma16x16<DT>(bf[set][j], af[set][i], acc[i][j]);
     };
     // What slot u does for the fragments of the next slice to be multiplied (slice kk of the stages a, b, into set `set`): one
     // read every other slot, B's eight and then A's; of an operand that lies along its outer dim, the pairs of raw reads are
@@ -438,7 +439,7 @@ __device__ __forceinline__ void dma_k_loop(const GmmArgs &p, const TileCoord &tc
                 if constexpr (B_RED) bf[set][f] = lb.frag(b, kk, f);
                 else rb[f] = lb.raw(b, kk, f);
             } else {
-                if constexpr (A_RED) af[set][f - 8] = la.frag(a, kk, f - 8);
+                if constexpr (A_RED) { if (f - 8 < RB) af[set][f - 8] = la.frag(a, kk, f - 8); }
                 else ra[f - 8] = la.raw(a, kk, f - 8);
             }
         }
@@ -701,7 +702,7 @@ __device__ __forceinline__ void swiglu_tile(const GmmArgs &p, const f32x4 (&acc)
     float prob[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int row = row0 + i * 16 + qrow;
+        const int row = row0 + i * 32 + qrow;
         prob[i] = p.probs != nullptr && row < row_end ? load_scalar_as_float(p.probs, row, p.probs_dtype) : 1.f;
     }
     const bool keep = p.c != nullptr;
@@ -734,7 +735,7 @@ __device__ __forceinline__ void swiglu_tile(const GmmArgs &p, const f32x4 (&acc)
             }
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);
-        const int first = row0 + half * ROWS;
+        auto row_at = [&](int r) { return row0 + (half * (ROWS / 16) + (r >> 4)) * 32 + (r & 15); };
         {
             const int acol = acol0 + (lane & 7) * 8;
             uint16_t *dst = static_cast<uint16_t *>(p.act) + acol;
@@ -742,7 +743,7 @@ __device__ __forceinline__ void swiglu_tile(const GmmArgs &p, const f32x4 (&acc)
             for (int pass = 0; pass < ROWS / 8; ++pass) {
                 const int r = pass * 8 + (lane >> 3);
                 const v16 v = *reinterpret_cast<const v16 *>(act + r * AP + (lane & 7) * 16);
-                if (acol < p.cols && first + r < row_end) *reinterpret_cast<v16 *>(dst + static_cast<int64_t>(first + r) * p.act_stride_row) = v;
+                if (acol < p.cols && row_at(r) < row_end) *reinterpret_cast<v16 *>(dst + static_cast<int64_t>(row_at(r)) * p.act_stride_row) = v;
             }
         }
         if (keep) {
@@ -752,17 +753,17 @@ __device__ __forceinline__ void swiglu_tile(const GmmArgs &p, const f32x4 (&acc)
             for (int pass = 0; pass < ROWS / 4; ++pass) {
                 const int r = pass * 4 + g;
                 const v16 v = *reinterpret_cast<const v16 *>(fc1 + r * HP + qrow * 16);
-                if (acol < p.cols && first + r < row_end) *reinterpret_cast<v16 *>(dst + static_cast<int64_t>(first + r) * p.c_stride_row) = v;
+                if (acol < p.cols && row_at(r) < row_end) *reinterpret_cast<v16 *>(dst + static_cast<int64_t>(row_at(r)) * p.c_stride_row) = v;
             }
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);             // the rows have been read before the next ones overwrite them
     }
 }
 
-// One macro tile of TBM x 256 outputs.  TBM = 256: 2x2 wavefronts of 128x128; TBM = 128 / 64: 1x4 wavefronts
-// of 128x64 / 64x64.
-template <int DT, bool A_RED, bool B_RED, int OUT, int TBM>
-__device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc, char *lds) {
+// One macro tile of TBM x 256 outputs.  TBM = 256: 2x2 wavefronts of 128x128, of which the first RB blocks of 16 rows are
+// computed; TBM = 128 / 64: 1x4 wavefronts of 128x64 / 64x64.
+template <int DT, bool A_RED, bool B_RED, int OUT, int TBM, int RB = 8>
+__device__ __forceinline__ void gmm16_tile_rows(const GmmArgs &p, const TileCoord &tc, char *lds) {
     constexpr int WAVES_M = TBM == 256 ? 2 : 1;
     constexpr int WAVES_N = 4 / WAVES_M;
     constexpr int TM = TBM / WAVES_M / 32;      // 32-row MFMA blocks per wavefront
@@ -789,7 +790,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     std::conditional_t<DMA, Acc16<2 * TM, 2 * TN, TBM == 256 && !A_RED, TBM == 256 && !B_RED>, Acc32<TM, TN>> sums;
     auto &acc = sums.v;
     if constexpr (DMA) {
-        if constexpr (TBM == 256) dma_k_loop<DT, A_RED, B_RED, SWIGLU>(p, tc, lds, row0, col0, acc);
+        if constexpr (TBM == 256) dma_k_loop<DT, A_RED, B_RED, SWIGLU, RB>(p, tc, lds, row0, col0, acc);
         else dma_small_k_loop<DT, B_RED, SWIGLU, TBM>(p, tc, lds, row0, col0, acc);
     } else {
 #pragma unroll
@@ -920,8 +921,10 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
     const int qrow = lane & (Acc::MB - 1);
     const int64_t ldc = p.c_stride_row;
     constexpr int WR = TM * 32, WC = TN * 32;       // this wavefront's block of the tile
+    // row of the tile's row r of this wavefront's block
+    auto row_at = [&](int r) { return row0 + (A_RED && TBM == 256 ? (r >> 4) * 32 + wm * 16 + (r & 15) : wm * WR + r); };
     if constexpr (SWIGLU && TBM == 256) {
-        swiglu_tile<DT>(p, sums.v, lds, row0 + wm * WR, row_end, col0 + wn * (WC / 2), wave);
+        swiglu_tile<DT>(p, sums.v, lds, row0 + wm * 16, row_end, col0 + wn * (WC / 2), wave);
     } else if constexpr (OUT == OUT_SAME || OUT == OUT_SWIGLU || OUT == OUT_SWIGLU_GRAD) {
         // 16-bit output: each wavefront stages its block in its own LDS region (row pitch WC*2 + 16 bytes, so that the
         // column-slice writes of a 16 x 16 block, 8 bytes or 16 of a WIDE B, start on different banks in all its rows) and writes it out as
@@ -966,7 +969,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll 2
             for (int pass = 0; pass < WR / RPP; ++pass) {
                 const int r = pass * RPP + lane / LPR;
-                const int row = row0 + wm * WR + r;
+                const int row = row_at(r);
                 const bool ok = col_ok && row < row_end;
                 uint16_t d[8], g[8], u[8], og[8], ou[8];
                 *reinterpret_cast<v16 *>(d) = *reinterpret_cast<const v16 *>(stg + r * SP + chunk * 16);
@@ -1004,7 +1007,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll 4
             for (int pass = 0; pass < WR / RPP; ++pass) {
                 const int r = pass * RPP + lane / LPR;
-                const int row = row0 + wm * WR + r;
+                const int row = row_at(r);
                 const v16 v = *reinterpret_cast<const v16 *>(stg + Acc::staged_row(r) * SP + chunk * 16);
                 if (col_ok && row < row_end) {
                     v16 *dst = reinterpret_cast<v16 *>(cbase + static_cast<int64_t>(row) * ldc);
@@ -1032,7 +1035,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll 4
             for (int pass = 0; pass < WR / 2 / RPP; ++pass) {
                 const int r = rbase + pass * RPP + lane / LPR;
-                const int row = row0 + wm * WR + r;
+                const int row = row_at(r);
                 uint16_t g[8], u[8], o[8];
                 *reinterpret_cast<v16 *>(g) = *reinterpret_cast<const v16 *>(gstg + r * SP + chunk * 16);
                 *reinterpret_cast<v16 *>(u) = *reinterpret_cast<const v16 *>(ustg + r * SP + chunk * 16);
@@ -1071,7 +1074,7 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
         auto load_old = [&](f32x4 (&dst)[NP], int i) {
 #pragma unroll
             for (int pass = 0; pass < NP; ++pass) {
-                int row = row0 + wm * WR + Acc::real_row(i * 32 + pass * RPP + lane / LPR);
+                int row = row_at(Acc::real_row(i * 32 + pass * RPP + lane / LPR));
                 row = row < row_end ? row : row_end - 1;
                 dst[pass] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(lbase + static_cast<int64_t>(row) * ldc));
             }
@@ -1091,13 +1094,33 @@ __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc
 #pragma unroll
             for (int pass = 0; pass < NP; ++pass) {
                 const int r = pass * RPP + lane / LPR;
-                const int row = row0 + wm * WR + Acc::real_row(i * 32 + r);
+                const int row = row_at(Acc::real_row(i * 32 + r));
                 f32x4 o = *reinterpret_cast<const f32x4 *>(stg + r * SPF + c4);
                 if constexpr (OUT == ACC_F32) o += old[i & 1][pass];
                 if (col_ok && row < row_end) __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(cbase + static_cast<int64_t>(row) * ldc));
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);    // the strip has been read before the next one overwrites it
         }
+    }
+}
+
+// A 256-row tile of fewer rows computes them in as many blocks of 32 (16 of each of the two wavefronts of a column half) as they
+// take: a group's last tile holds 129 to 256.  What the rest would cost is energy, which bounds the long launches, and matrix
+// time in the others.  All groups of so many rows, bf16, with eight blocks always and with as many as needed, us: 32 groups, 2880 x
+// 5760, forward / dX 140 rows 253 / 258 -> 224 / 241, 170 rows 251 / 261 -> 232 / 248, 200 rows 256 / 260 -> 242 / 256, 250 rows 266 /
+// 271 -> 265 / 271; five blocks beside six 230 -> 224 and 243 -> 241 (140 rows).  The A rows past the end are still requested (one
+// wait count for all wavefronts).  Not for the weight gradient (its tiles' rows are the weight's, whole but for the last) nor
+// for fp32 output.
+template <int DT, bool A_RED, bool B_RED, int OUT, int TBM>
+__device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc, char *lds) {
+    if constexpr (A_RED && TBM == 256 && (OUT == OUT_SAME || OUT == OUT_SWIGLU)) {
+        const int rows = tc.e.row_end - tc.e.row_begin - tc.row_tile * BM;
+        if (rows > 224) gmm16_tile_rows<DT, A_RED, B_RED, OUT, TBM>(p, tc, lds);
+        else if (rows > 192) gmm16_tile_rows<DT, A_RED, B_RED, OUT, TBM, 7>(p, tc, lds);
+        else if (rows > 160) gmm16_tile_rows<DT, A_RED, B_RED, OUT, TBM, 6>(p, tc, lds);
+        else gmm16_tile_rows<DT, A_RED, B_RED, OUT, TBM, 5>(p, tc, lds);
+    } else {
+        gmm16_tile_rows<DT, A_RED, B_RED, OUT, TBM>(p, tc, lds);
     }
 }
 
