@@ -22,7 +22,8 @@ struct GroupEntry {
     int num_tiles;           // num_row_tiles * column tiles
     int share;               // entry of an XCD's own list: tiles of it that every XCD handles (whole: all of them)
     int split;               // 0, or 1 + the part number of a small tail tile whose reduction is split: such a
-                             // tile writes fp32 partial sums to the split workspace (c_off then points there)
+                             // tile writes fp32 partial sums to the split workspace (c_off then points there);
+                             // kEvened: the last two row tiles share their rows (even_out)
     int whole;               // entry of an XCD's own list: 1 = that XCD takes all tiles of the group, 0 = its eighth
     int64_t b_off;           // element offset of the group's weight block
     int64_t c_off;           // element offset of the group's output block
@@ -88,6 +89,7 @@ struct GmmArgs {
     int m, k;
     int tile_rows;              // rows per full tile, a power of two: 256 for 16-bit operands; 32, 64 or 128 in fp32
     int small_tails;            // a group's last row tile may be a smaller one
+    int even_tails;             // ... or the last two share their rows (small_tail_of)
     int tails_last_below;       // launches of fewer tiles take their small tiles last
     int part_cus;               // compute units if the last round may be divided (LastRound), else 0
 };
@@ -236,11 +238,38 @@ __device__ __forceinline__ int consecutive_tile(int t, int n, const LastRound &l
     return t < whole ? share_of_eight(t, whole) : whole + share_of_eight(t - whole, n - whole);
 }
 
+// Rows of the small tile that a remainder of `rem` rows of a group goes to, 0 for a full one.
+__host__ __device__ __forceinline__ int small_tile_rows(int rem) { return rem <= 64 ? 64 : (rem <= 128 ? 128 : 0); }
+
+// A group of more than one row tile whose last one would be a small one may instead share the rows of its last two between
+// them (`even`), 160 and up to 160 or 192 and up to 192: two tiles of five or six of the eight row blocks (gmm16_tile).
+// What bounds a small tile is its own pass over the weight panel: it takes 0.45 to 0.65 of a full tile's time for a quarter
+// or half of its products, and leaves the step of the tiles beside it.
+constexpr int kEvened = -1;
+__host__ __device__ __forceinline__ int small_tail_of(int rem, int row_tiles, bool even) {
+    return even && row_tiles > 1 ? 0 : small_tile_rows(rem);
+}
+__device__ __forceinline__ bool shares_last_two(int rem, int row_tiles, bool even) {
+    return even && row_tiles > 1 && small_tile_rows(rem) != 0;
+}
+// The rows of such a tile, as those of an entry in which it begins where its number says.
+__device__ __forceinline__ void even_out(TileCoord &tc) {
+    const int T = tc.e.tile_rows, n = tc.e.num_row_tiles;
+    tc.e.split = 0;
+    if (tc.row_tile < n - 2) return;
+    const int rem = tc.e.row_end - tc.e.row_begin - (n - 1) * T;
+    const int rows = rem <= 64 ? 160 : 192;
+    const int from = tc.e.row_begin + (n - 2) * T + (tc.row_tile == n - 1 ? rows : 0);
+    tc.e.row_end = from + rows < tc.e.row_end ? from + rows : tc.e.row_end;
+    tc.e.row_begin = from - tc.row_tile * T;
+}
+
 // Tile number j of an entry: of the entry's tiles every XCD (workgroup number modulo 8) takes consecutive ones of the
 // blocked order, the odd ones dealt in turn; in_order: the j-th one.
 __device__ __forceinline__ void deal_tile(TileCoord &tc, int j, int num_col_tiles, bool in_order = false) {
     tile_order(in_order ? j : share_of_eight(j, tc.e.num_tiles), tc.e.num_row_tiles, num_col_tiles, tc.row_tile, tc.col_tile);
     tc.tile_rows = (tc.e.tail_rows != 0 && tc.row_tile == tc.e.num_row_tiles - 1) ? tc.e.tail_rows : tc.e.tile_rows;
+    if (tc.e.split == kEvened) even_out(tc);
     tc.valid = true;
 }
 
@@ -272,6 +301,7 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table, int b) 
         if (r >= tc.e.num_tiles || (tc.e.whole == 0 && slot - tc.e.tile_begin >= tc.e.share)) return tc;
         tile_order(r, tc.e.num_row_tiles, tc.e.num_tiles / tc.e.num_row_tiles, tc.row_tile, tc.col_tile);
         tc.tile_rows = (tc.e.tail_rows != 0 && tc.row_tile == tc.e.num_row_tiles - 1) ? tc.e.tail_rows : tc.e.tile_rows;
+        if (tc.e.split == kEvened) even_out(tc);
         tc.valid = true;
         return tc;
     }
@@ -306,9 +336,6 @@ __device__ __forceinline__ TileCoord locate_tile(const TileTable *table, int b) 
     if (t >= lr.from && t < lr.from + lr.count) take_part(tc, part, lr.shift);
     return tc;
 }
-
-// Rows of the small tile that a remainder of `rem` rows of a group goes to, 0 for a full one.
-__host__ __device__ __forceinline__ int small_tile_rows(int rem) { return rem <= 64 ? 64 : (rem <= 128 ? 128 : 0); }
 
 // A tile of the launch, found by every wavefront for itself out of a group list of at most 64 groups: the entries and tile numbers
 // of a table without per-XCD lists and split tails (gmm_schedule_kernel).  Lane g holds group g, the running quantities are
@@ -365,7 +392,8 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p, int b) {
         e.tile_begin = q * e.num_tiles;
     } else {
         const int row_tiles = (len + T - 1) >> shift;
-        const int tail = p.small_tails && len > 0 ? small_tile_rows(len - (row_tiles - 1) * T) : 0;
+        const int rem = len - (row_tiles - 1) * T;
+        const int tail = p.small_tails && len > 0 ? small_tail_of(rem, row_tiles, p.even_tails != 0) : 0;
         const unsigned packed = static_cast<unsigned>(row_tiles) | (tail != 0 ? 1u << 25 : 0u);   // (fewer than 2^25 row tiles, at most 64 tails)
         const unsigned incl = wave_scan(packed, [](unsigned x, unsigned y) { return x + y; });
         const unsigned sums = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
@@ -411,6 +439,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p, int b) {
             e.row_end = full_only ? g_prev + g_full * T : g_end;
             e.num_row_tiles = first ? g_full : 1;
             e.tail_rows = full_only ? 0 : g_tail;
+            if (__builtin_amdgcn_readlane(p.small_tails && shares_last_two(rem, row_tiles, p.even_tails != 0) ? 1 : 0, g)) e.split = kEvened;
             e.num_tiles = e.num_row_tiles * C;
             e.tile_begin = __builtin_amdgcn_readlane(begin, g);
             e.b_off = p.b_offsets != nullptr ? p.b_offsets[g] : g * p.b_stride_group;
