@@ -89,7 +89,7 @@ struct GmmArgs {
     int m, k;
     int tile_rows;              // rows per full tile, a power of two: 256 for 16-bit operands; 32, 64 or 128 in fp32
     int small_tails;            // a group's last row tile may be a smaller one
-    int even_tails;             // ... or the last two share their rows (small_tail_of)
+    int even_tails;             // ... or the last two share their rows (EVEN_..)
     int tails_last_below;       // launches of fewer tiles take their small tiles last
     int part_cus;               // compute units if the last round may be divided (LastRound), else 0
 };
@@ -242,15 +242,16 @@ __device__ __forceinline__ int consecutive_tile(int t, int n, const LastRound &l
 __host__ __device__ __forceinline__ int small_tile_rows(int rem) { return rem <= 64 ? 64 : (rem <= 128 ? 128 : 0); }
 
 // A group of more than one row tile whose last one would be a small one may instead share the rows of its last two between
-// them (`even`), 160 and up to 160 or 192 and up to 192: two tiles of five or six of the eight row blocks (gmm16_tile).
+// them (`even`: EVEN_TWO only in groups of two, EVEN_ALL), 160 and up to 160 or 192 and up to 192: two tiles of five or six of the eight row blocks (gmm16_tile).
 // What bounds a small tile is its own pass over the weight panel: it takes 0.45 to 0.65 of a full tile's time for a quarter
 // or half of its products, and leaves the step of the tiles beside it.
 constexpr int kEvened = -1;
-__host__ __device__ __forceinline__ int small_tail_of(int rem, int row_tiles, bool even) {
-    return even && row_tiles > 1 ? 0 : small_tile_rows(rem);
+enum { EVEN_NONE = 0, EVEN_TWO = 1, EVEN_ALL = 2 };
+__host__ __device__ __forceinline__ bool shares_last_two(int rem, int row_tiles, int even) {
+    return small_tile_rows(rem) != 0 && (even == EVEN_ALL ? row_tiles > 1 : even == EVEN_TWO && row_tiles == 2);
 }
-__device__ __forceinline__ bool shares_last_two(int rem, int row_tiles, bool even) {
-    return even && row_tiles > 1 && small_tile_rows(rem) != 0;
+__host__ __device__ __forceinline__ int small_tail_of(int rem, int row_tiles, int even) {
+    return shares_last_two(rem, row_tiles, even) ? 0 : small_tile_rows(rem);
 }
 // The rows of such a tile, as those of an entry in which it begins where its number says.
 __device__ __forceinline__ void even_out(TileCoord &tc) {
@@ -393,7 +394,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p, int b) {
     } else {
         const int row_tiles = (len + T - 1) >> shift;
         const int rem = len - (row_tiles - 1) * T;
-        const int tail = p.small_tails && len > 0 ? small_tail_of(rem, row_tiles, p.even_tails != 0) : 0;
+        const int tail = p.small_tails && len > 0 ? small_tail_of(rem, row_tiles, p.even_tails) : 0;
         const unsigned packed = static_cast<unsigned>(row_tiles) | (tail != 0 ? 1u << 25 : 0u);   // (fewer than 2^25 row tiles, at most 64 tails)
         const unsigned incl = wave_scan(packed, [](unsigned x, unsigned y) { return x + y; });
         const unsigned sums = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
@@ -439,7 +440,7 @@ __device__ __forceinline__ TileCoord tile_from_list(const GmmArgs &p, int b) {
             e.row_end = full_only ? g_prev + g_full * T : g_end;
             e.num_row_tiles = first ? g_full : 1;
             e.tail_rows = full_only ? 0 : g_tail;
-            if (__builtin_amdgcn_readlane(p.small_tails && shares_last_two(rem, row_tiles, p.even_tails != 0) ? 1 : 0, g)) e.split = kEvened;
+            if (__builtin_amdgcn_readlane(p.small_tails && shares_last_two(rem, row_tiles, p.even_tails) ? 1 : 0, g)) e.split = kEvened;
             e.num_tiles = e.num_row_tiles * C;
             e.tile_begin = __builtin_amdgcn_readlane(begin, g);
             e.b_off = p.b_offsets != nullptr ? p.b_offsets[g] : g * p.b_stride_group;

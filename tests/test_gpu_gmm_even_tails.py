@@ -1,9 +1,10 @@
-"""In long launches, and in the one launch of both gradients, a group whose last row tile would be a small one has its last two
-tiles share their rows.  The same rows in groups that fill their tiles give the same bits, and every row is written once: the
+"""A group whose last row tile would be a small one has its last two tiles share their rows: in long launches and in the one launch
+of both gradients any, elsewhere one of two row tiles.  The same rows in groups that fill their tiles give the same bits, and every row is written once: the
 outputs start as NaN, and rows behind the groups are zero."""
 import pytest
 import torch
 
+from conftest import rel_l2
 from mindspeed_amd.ops._kernels import K
 from mindspeed_amd.ops.gmm import gmm_backward_raw, gmm_raw
 
@@ -57,6 +58,28 @@ def test_equals_tiles_that_are_full(name, k):
     assert torch.equal(y32[:own.numel()], whole32[own])
     fc1, act = K.gmm_swiglu(x, w, short, 1, None, True)
     assert torch.equal(fc1, y) and torch.equal(act, K.swiglu(y, None))
+
+
+# short launches: last rounds divided into parts of such tiles or not, small tiles of other groups beside them, whole or (from a
+# reduction of 4096 on) with their reduction split
+@pytest.mark.parametrize("cols,k,counts", [
+    (1, 72, [300]), (3, 72, [257, 288, 320, 321, 384, 385, 5, 0, 640]), (12, 136, [300, 380] * 6), (16, 72, [1024, 330, 260] * 4),
+    (7, 200, [290] * 70), (5, 4224, [300, 600, 350, 20]), (16, 8256, [512, 380, 600, 257])])
+def test_groups_of_two_row_tiles_in_short_launches(cols, k, counts):
+    n = cols * 256 - 40
+    full, own, x, short, whole = _rows(counts, k)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    w = torch.randn(len(counts), k, n, generator=gen, device="cuda").bfloat16()
+    two = torch.cat([torch.full((c,), 256 < c <= 384, device="cuda") for c in counts])
+    for weight in (w, w.transpose(1, 2).contiguous().transpose(1, 2)):
+        y = torch.full((x.size(0) + 2, n), float("nan"), dtype=x.dtype, device="cuda")
+        gmm_raw(x, weight, short, 0, 1, out=y[:-2])
+        expect = gmm_raw(full, weight, whole, 0, 1)[own]
+        assert torch.equal(y[:-2][two], expect[two])
+        if k < 4096:
+            assert torch.equal(y[:-2], expect)
+        assert rel_l2(y[:-2], expect) <= 4e-3               # (the sums of a split reduction are added in another order)
+        assert bool(y[-2:].isnan().all())
 
 
 @pytest.mark.parametrize("counts", [EDGES, [30, 0, 600, 1100], [300] * 20, EDGES * 4, [1024 + 13 * (g - 4) for g in range(8)]],
