@@ -360,12 +360,14 @@ using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 const Tensor kNone;
 
-// The Python function of an op, for a Recorder.
+// The Python function of an op, for a Recorder.  No Python object leaves it (the caller does not hold the interpreter's lock).
 template <typename Result, typename... Args>
 Result recorded(const char *name, Args &&...args) {
+    static_assert(!std::is_base_of_v<py::handle, Result>, "it would be given back without the interpreter's lock");
     const py::gil_scoped_acquire gil;
     try {
-        return py::cast<Result>(py::handle(device_fns)[name](std::forward<Args>(args)...));
+        const py::object out = py::handle(device_fns)[name](std::forward<Args>(args)...);
+        if constexpr (!std::is_void_v<Result>) return py::cast<Result>(out);
     } catch (py::error_already_set &e) {
         e.restore();
         python_error err;
@@ -426,7 +428,7 @@ struct GmmNode : torch::autograd::Function<GmmNode> {
             if (want_x && want_w) {
                 dx = recording ? recorded<Tensor>("gmm_backward", grad, x, w, counts, 1, dw, false) : *gmm_backward(grad, x, w, counts, 1, dw, false);
             } else if (want_w) {
-                if (recording) recorded<py::object>("gmm_out", x.t(), grad, counts, 2, 1, dw, false);
+                if (recording) recorded<void>("gmm_out", x.t(), grad, counts, 2, 1, dw, false);
                 else gmm_out(x.t(), grad, counts, 2, 1, dw, false);
             } else if (want_x) {
                 dx = recording ? recorded<Tensor>("gmm", grad, w.transpose(1, 2), counts, 0, 1) : *gmm(grad, w.transpose(1, 2), counts, 0, 1);

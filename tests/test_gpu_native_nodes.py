@@ -270,6 +270,24 @@ def test_a_recorder_sees_every_op(taken, monkeypatch):
     assert equal(run_layer(args), plain) and taken == []
 
 
+@pytest.mark.parametrize("wanted", [(3,), (3, 4), (0,), (2,), (0, 3)])
+def test_a_recorder_around_the_backward_pass_alone(wanted, taken):
+    """The native forward's nodes call the Python functions from the autograd thread, whichever gradients are wanted."""
+    args = layer_inputs()
+    plain = run_layer(args, wanted)
+    leaves = [a.detach() for a in args]
+    for i in wanted:
+        leaves[i].requires_grad_(True)
+    y = dispatch_mlp_combine(*leaves[:3], leaves[3:])
+    with flop_counter.record(timing=False) as rec:
+        grads = torch.autograd.grad(y, [leaves[i] for i in wanted], torch.ones_like(y))
+    assert taken == ["layer", "layer"] and equal([y.detach(), *grads], plain)
+    names = [c[0] for c in rec.calls]
+    # (a matmul's gradients: by what lies in front of it and whether its weight is wanted)
+    in_front = [0 in wanted, bool({0, 3} & set(wanted))]
+    assert names.count("gmm_dx") == sum(in_front) and names.count("gmm_dw") == (3 in wanted) + (4 in wanted)
+
+
 def test_a_failed_call_in_the_backward_pass(taken, monkeypatch):
     """The library's refusal reaches the caller as the package's error whichever thread met it."""
     args = layer_inputs()
