@@ -106,11 +106,13 @@ __device__ __forceinline__ void store_float_as(void *p, int64_t i, int dtype, fl
 }
 
 // 1 / (1 + exp(-x)) of a 16-bit value, for results that are rounded to 16 bits.  The reciprocal instruction (1 ulp) and one Newton
-// step, four instructions where the division takes ten.  Past exp's overflow the step's factor is NaN, which fmaxf takes out: 0.
+// step, five instructions where the division takes ten.  The instruction has no subnormal results, but x times one is a normal
+// bfloat16 (x = -87.5, -88, -88.5): it sees a quarter of 1 + exp(-x), at most 2^126, and the last product is the only one that
+// rounds to a subnormal.  Past exp's overflow the step's factor is NaN, which fmaxf takes out: 0, as the division gives.
 __device__ __forceinline__ float sigmoid16(float x) {
-    const float d = 1.f + __expf(-x);
+    const float d = fmaf(__expf(-x), 0.25f, 0.25f);
     const float r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaxf(fmaf(-d, r, 1.f), -1.f), r, r);
+    return fmaf(fmaxf(fmaf(-d, r, 1.f), -1.f), r, r) * 0.25f;
 }
 
 // ---- prefix sums over the lanes of a wavefront ----------------------------------
