@@ -56,8 +56,9 @@ def dispatch_mlp_combine(hidden_states, top_k_index, top_k_weights, weights, num
                          fuse_activation=None, gemm_fusion=False):
     gate_up_weights, down_weights = weights
     num_experts = gate_up_weights.size(0) if num_global_experts is None else num_global_experts
-    # the same ops in one native call, wherever nothing but autograd is to see them
-    if not gemm_fusion and not gmm_ops.OVERLAP_WGRAD and num_experts.__class__ is int:
+    # the same ops in one native call, wherever nothing but autograd is to see them and the products are this package's
+    if (not gemm_fusion and not gmm_ops.OVERLAP_WGRAD and num_experts.__class__ is int
+            and gmm_ops.built_in(gmm_ops.GMMFunction.builder2.load(), "npu_gmm", "npu_gmm_backward")):
         fused = not torch.is_grad_enabled() if fuse_activation is None else bool(fuse_activation)
         out = native_form("layer", hidden_states, top_k_index, top_k_weights, gate_up_weights, down_weights, num_experts, fused)
         if out is not None:

@@ -282,6 +282,19 @@ class _RawGmmModule:
         return [dx], [], []
 
 
+# The products that gmm_backward_raw and the native layer stand for: a module that brings others (a subclass, a wrapper, a method
+# put in their place) is called for them instead.
+_BUILT_IN = {name: getattr(_RawGmmModule, name) for name in ("npu_gmm", "npu_gmm_backward", "npu_gmm_backward_fusion")}
+
+
+def built_in(module, *names) -> bool:
+    """Whether these functions of a module are the ones of this package."""
+    for name in names:
+        if getattr(module, name, None) is not _BUILT_IN[name]:
+            return False
+    return True
+
+
 class _Builder:
     _module = _RawGmmModule()
 
@@ -336,10 +349,11 @@ class GMMFunction(torch.autograd.Function):
             (dx,), (dw,), dbias = module.npu_gmm_backward([grad_y], [x], [weight], group_list, ctx.group_list_type)
             return None, dx, dw, (dbias[0] if dbias else None), None
         # gemm_fusion (gmm.py:56-89): the weight gradient is added into original_weight.main_grad (fp32) by the
-        # accumulate form of the dW product, in one launch with dX or on the side stream beside it; what autograd gets for the weight is
-        # a placeholder (zeros if the parameter asks for it) and the flag the optimizer wrapper looks at is set.
+        # accumulate form of the dW product, in one launch with dX (where that is this package's too) or on the side stream beside
+        # it; what autograd gets for the weight is a placeholder (zeros if the parameter asks for it) and the flag the optimizer
+        # wrapper looks at is set.
         side = _beside(grad_y)
-        if side.active:
+        if side.active or not built_in(module, "npu_gmm_backward_fusion"):
             with side:
                 add_weight_gradient(x, grad_y, group_list, ctx.group_list_type, original_weight.main_grad)
             (dx,), _, dbias = module.npu_gmm_backward_fusion([grad_y], [weight], group_list, ctx.group_list_type)
