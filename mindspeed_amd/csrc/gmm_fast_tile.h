@@ -1105,15 +1105,20 @@ __device__ __forceinline__ void gmm16_tile_rows(const GmmArgs &p, const TileCoor
 }
 
 // A 256-row tile of fewer rows computes them in as many blocks of 32 (16 of each of the two wavefronts of a column half) as they
-// take: a group's last tile holds 129 to 256.  What the rest would cost is energy, which bounds the long launches, and matrix
+// take: a group's last tile holds 129 to 256, two that share their rows (shares_last_two) 97 to 192 each.  What the rest would cost
+// is energy, which bounds the long launches, and matrix
 // time in the others.  All groups of so many rows, bf16, with eight blocks always and with as many as needed, us: 32 groups, 2880 x
 // 5760, forward / dX 140 rows 253 / 258 -> 224 / 241, 170 rows 251 / 261 -> 232 / 248, 200 rows 256 / 260 -> 242 / 256, 250 rows 266 /
-// 271 -> 265 / 271; five blocks beside six 230 -> 224 and 243 -> 241 (140 rows).  The A rows past the end are still requested (one
-// wait count for all wavefronts).  Not for the weight gradient (its tiles' rows are the weight's, whole but for the last) nor
-// for fp32 output.
+// 271 -> 265 / 271; five blocks beside six 230 -> 224 and 243 -> 241 (140 rows).  fp32 output / `+=` / SwiGLU backward in the
+// epilogue, 2880 x 2880 32 of 170 rows 156 / 152 / 176 -> 144 / 146 / 172; sharing rows pays by them alone (small tiles; shared,
+// eight blocks; shared): 32 of 290 rows, 2880 x 2880 217 / 234 / 286; 231 / 246 / 270; 188 / 203 / 242, 8 of 300, 4096 x 28672
+// 670 / 700 / 838; 747 / 771 / 828; 599 / 628 / 713, 128 of 300, 2048 x 3072 638 / 691 / 929; 700 / 749 / 867; 587 / 644 / 802, 16 of
+// 1100, 2048 x 6144 422 / 464 / 576; 441 / 489 / 618; 417 / 458 / 590 (the one of 15 sizes where a mode has small tiles 2 % faster).
+// The A rows past the end are still requested (one wait count for all wavefronts).  Not for the weight gradient (its tiles' rows
+// are the weight's, whole but for the last).
 template <int DT, bool A_RED, bool B_RED, int OUT, int TBM>
 __device__ __forceinline__ void gmm16_tile(const GmmArgs &p, const TileCoord &tc, char *lds) {
-    if constexpr (A_RED && TBM == 256 && (OUT == OUT_SAME || OUT == OUT_SWIGLU)) {
+    if constexpr (A_RED && TBM == 256) {
         const int rows = tc.e.row_end - tc.e.row_begin - tc.row_tile * BM;
         if (rows > 224) gmm16_tile_rows<DT, A_RED, B_RED, OUT, TBM>(p, tc, lds);
         else if (rows > 192) gmm16_tile_rows<DT, A_RED, B_RED, OUT, TBM, 7>(p, tc, lds);
