@@ -39,10 +39,12 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "gmm_hbm_traffic.json")
 GEMM_KERNEL_NAMES = {
     "gmm_fwd": "gmm16_fast_kernel<bf16, A reduction-contiguous, B column-contiguous> (forward grouped matmul; one "
                "launch each for fc1 and fc2, averaged)",
+    "gmm_dx_and_dw": "gmm16_pair_kernel<bf16> (dX and dW of one grouped matmul in one launch; one launch each for fc1 and "
+                     "fc2, averaged)",
     "gmm_dx": "gmm16_fast_kernel<bf16, A reduction-contiguous, B reduction-contiguous> (dX grouped matmul on the "
-              "transposed weight view; one launch each for fc1 and fc2, averaged)",
+              "transposed weight view, by itself; one launch each for fc1 and fc2, averaged)",
     "gmm_dw": "gmm16_fast_kernel<bf16, A row-contiguous, B column-contiguous> (dW grouped matmul, split on the "
-              "reduction dim; one launch each for fc1 and fc2, averaged)",
+              "reduction dim, by itself; one launch each for fc1 and fc2, averaged)",
     "gmm_fwd_swiglu": "gmm16_fast_kernel<bf16, A reduction-contiguous, B column-contiguous, SwiGLU epilogue> (fc1 "
                       "forward grouped matmul, one launch per step)",
     "gmm_dx_swiglu": "gmm16_fast_kernel<bf16, A, B reduction-contiguous, SwiGLU-backward epilogue> (fc2 dX grouped "
@@ -180,9 +182,8 @@ def threads_on_one_core():
     """Confine every thread of this process to one core for the duration.  The host work of an eager step is serial —
     the main thread issues the forward pass, then waits while torch's autograd thread issues the backward pass — so
     nothing is lost, and the core never goes idle between the two hand-overs of a step.  With the threads on different
-    cores each hand-over wakes an idle core, which on these hosts costs about 70 us: the small configuration's step
-    reads 0.27 ms as the scheduler places the threads and 0.17 ms on one core.  (The core is the lowest of
-    the process's share; on another host the step read 0.28 ms and, confined to it, 0.41 ms.)"""
+    cores each hand-over wakes an idle core: the small configuration's step reads 0.09 to 0.15 ms as the scheduler places
+    the threads and 0.09 ms on one core, the lowest of the process's share."""
     saved = {}
     for name in os.listdir("/proc/self/task"):
         try:
@@ -263,7 +264,6 @@ def run_layer(cfg, device, steps, warmup, fuse_activation=False, per_kernel=True
     the event brackets or None, per-kernel table or None, the inputs).
     accumulate: None, or how the weight gradients reach fp32 `main_grad` buffers of the weights: "fused" = added by
     the weight-gradient product itself (gemm_fusion), "separate" = 16-bit weight gradients and one torch add each."""
-    from mindspeed_amd import flop_counter
     from mindspeed_amd.dispatcher import dispatch_mlp_combine
 
     x, p, idx, w1, w2, gy = make_inputs(cfg, device)
@@ -294,7 +294,20 @@ def run_layer(cfg, device, steps, warmup, fuse_activation=False, per_kernel=True
     if not per_kernel:
         return ms_per_step, None, None, (x, p, idx)
 
-    with flop_counter.record(timing=True) as rec:
+    # the launches of the timed steps; then dX and dW, which those make in one launch, each by itself
+    ms_events, kernels = _recorded_steps(cfg, steps, step, pairs=True)
+    if "gmm_dx_and_dw" in kernels:
+        apart = _recorded_steps(cfg, steps, step, pairs=False)[1]
+        kernels.update({name: dict(apart[name], apart=True) for name in ("gmm_dx", "gmm_dw")
+                        if name in apart and name not in kernels})
+    return ms_per_step, ms_events, kernels, (x, p, idx)
+
+
+def _recorded_steps(cfg, steps, step, pairs):
+    """`steps` steps with every op between two events: ms per step, and per op its time and rate."""
+    from mindspeed_amd import flop_counter
+
+    with flop_counter.record(timing=True, pairs=pairs) as rec:
         t0 = time.perf_counter()
         for _ in range(steps):
             step()
@@ -316,7 +329,7 @@ def run_layer(cfg, device, steps, warmup, fuse_activation=False, per_kernel=True
             entry["bytes_per_launch"] = work
             entry["frac_of_hbm_peak"] = round(entry["gbs"] / HBM_PEAK_GBS, 4)
         kernels[name] = entry
-    return ms_per_step, ms_events, kernels, (x, p, idx)
+    return ms_events, kernels
 
 
 def forward_only_ms(cfg, device, fuse_activation, steps=20, warmup=10):
@@ -416,13 +429,14 @@ def main():
 
     # dominant kernel: the grouped-matmul flavour with the largest share of the step
     peak = MFMA_PEAK_TFLOPS[cfg["dtype"]]
-    gemms = {k: v for k, v in kernels.items() if "tflops" in v}
+    launched = {k: v for k, v in kernels.items() if "apart" not in v}
+    gemms = {k: v for k, v in launched.items() if "tflops" in v}
     dom_name = max(gemms, key=lambda k: gemms[k]["ms_per_step"])
     dom = gemms[dom_name]
     kname = GEMM_KERNEL_NAMES.get(dom_name, dom_name) if cfg["dtype"] == "bf16" else \
         f"gmm32_kernel ({dom_name}, fp32 inputs)"
     roofline = {"bound": "mfma", "kernel": kname, "kernel_key": dom_name,
-                "share_of_step": round(dom["ms_per_step"] / sum(v["ms_per_step"] for v in kernels.values()), 4),
+                "share_of_step": round(dom["ms_per_step"] / sum(v["ms_per_step"] for v in launched.values()), 4),
                 "achieved": dom["tflops"], "peak": peak, "unit": "TFLOP/s", "frac": dom["frac_of_mfma_peak"],
                 "traffic": measured_traffic(args.workload, dom_name)}
 
@@ -446,7 +460,8 @@ def main():
         "roofline": roofline,
         "kernels": kernels,
         "kernels_note": "single launches inside the layer step, each between two events on its stream; an empty "
-                        f"bracket reads {empty_bracket_ms * 1e3:.1f} us on this box",
+                        f"bracket reads {empty_bracket_ms * 1e3:.1f} us on this box; `apart`: from steps whose dX and dW "
+                        "are launches of their own, which the timed steps do not make",
     }
     if args.copy_calibration:
         from mindspeed_amd import microbench_kernels
@@ -525,16 +540,16 @@ def main():
         ms, _, ok, _ = run_layer(ocfg, device, steps=300 if small else 10, warmup=100 if small else 10)
         others[name] = {"workload": ocfg["desc"], "ms_per_step": round(ms, 4),
                         "tokens_per_s": round(ocfg["T"] / (ms / 1e3), 1),
-                        "gemm_tflops": {k: ok[k]["tflops"] for k in ("gmm_fwd", "gmm_dx", "gmm_dw") if k in ok},
+                        "gemm_tflops": {k: ok[k]["tflops"] for k in ("gmm_fwd", "gmm_dx_and_dw", "gmm_dx", "gmm_dw") if k in ok},
                         "gemm_frac_of_mfma_peak": {k: ok[k]["frac_of_mfma_peak"]
-                                                   for k in ("gmm_fwd", "gmm_dx", "gmm_dw") if k in ok}}
+                                                   for k in ("gmm_fwd", "gmm_dx_and_dw", "gmm_dx", "gmm_dw") if k in ok}}
         if small:
             # the same steps with the process's threads on one core (see threads_on_one_core)
             with threads_on_one_core():
                 ms1, _, _, _ = run_layer(ocfg, device, steps=300, warmup=100, per_kernel=False)
             others[name]["ms_per_step_threads_on_one_core"] = round(ms1, 4)
-            others[name]["note"] = ("ms_per_step: threads placed by the scheduler; the step is host-bound and reads "
-                                    "0.17-0.41 ms depending on the host and on whether the main and the autograd thread share a core")
+            others[name]["note"] = ("ms_per_step: threads placed by the scheduler; host and device take about as long, and the step reads "
+                                    "0.09-0.15 ms depending on whether the main and the autograd thread share a core")
 
     def graph_section():
         others["plumbing"]["graph_replay_ms_per_step"] = graph_replay_ms(WORKLOADS["plumbing"], device)
@@ -547,6 +562,7 @@ def main():
         for how in ("fused", "separate"):
             ms, _, ok, _ = run_layer(cfg, device, steps=10, warmup=5, accumulate=how)
             acc[how] = {"ms_per_step": round(ms, 4),
+                        "gmm_dx_and_dw_tflops": ok["gmm_dx_and_dw"]["tflops"] if "gmm_dx_and_dw" in ok else None,
                         "gmm_dw_tflops": ok["gmm_dw"]["tflops"] if "gmm_dw" in ok else None}
             torch.cuda.empty_cache()
         others["mixtral_fp32_grad_accumulation"] = acc

@@ -53,10 +53,12 @@ def swiglu_bytes(rows, ffn, elem, backward=False):
 
 
 class Recorder:
-    """Collects (name, work, unit, start event, end event) for every op call while active."""
+    """Collects (name, work, unit, start event, end event) for every op call while active.  ``pairs``: the two gradients of
+    a grouped matmul as the one call that an unrecorded backward pass makes, else each by itself."""
 
-    def __init__(self, timing=True):
+    def __init__(self, timing=True, pairs=False):
         self.timing = timing
+        self.pairs = pairs
         self.calls = []
 
     def summary(self):
@@ -72,8 +74,8 @@ class Recorder:
 
 
 @contextlib.contextmanager
-def record(timing=True):
-    prev, rec = _active, Recorder(timing)
+def record(timing=True, pairs=False):
+    prev, rec = _active, Recorder(timing, pairs)
     _activate(rec)
     try:
         yield rec
@@ -101,6 +103,11 @@ def timing_active() -> bool:
     """True while a recorder is bracketing every op with events (ops then keep to one stream, so that the
     per-op durations are those of kernels running alone)."""
     return _active is not None and _active.timing
+
+
+def splits_pairs() -> bool:
+    """True while a recorder wants the two gradients of a grouped matmul each by itself."""
+    return _active is not None and not _active.pairs
 
 
 def recording() -> bool:

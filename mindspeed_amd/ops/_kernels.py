@@ -106,7 +106,7 @@ _define("gmm_out(Tensor x, Tensor weight, Tensor group_list, int group_type, int
 
 
 def _gmm_backward(grad, x, weight, group_list, group_list_type, dw, accumulate):
-    if flop_counter.recording():                 # (each product by itself, so that each has an entry of its own)
+    if flop_counter.splits_pairs():              # (each product by itself, so that each has an entry of its own)
         _gmm_launch(x.t(), grad, group_list, 2, group_list_type, dw, accumulate)
         return _gmm(grad, weight.transpose(1, 2), group_list, 0, group_list_type)
     lib = _lib.load()
@@ -119,7 +119,7 @@ def _gmm_backward(grad, x, weight, group_list, group_list_type, dw, accumulate):
     _lib.check(lib.msi_gmm_backward_workspace_size(num_groups, m, k, n, dtype, dw_dtype, 1 if accumulate else 0,
                                                    ctypes.byref(nbytes)), "msi_gmm_backward_workspace_size")
     ws = _lib.workspace(nbytes.value, dev)
-    with _lib.on(dev):
+    with _lib.on(dev), flop_counter.op("gmm_dx_and_dw", 2 * flop_counter.gmm_flops(m, k, n), "flop", dev):
         _lib.check(lib.msi_gmm_backward(
             _lib.stream_ptr(dev), _lib.ptr(grad), *grad.stride(), _lib.ptr(x), *x.stride(), _lib.ptr(weight), *weight.stride(),
             _lib.ptr(dx), _lib.ptr(dw), _lib.ptr(group_list), group_list_type, num_groups, m, k, n, dtype, dw_dtype,
