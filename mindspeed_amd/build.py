@@ -112,12 +112,12 @@ def compile_trace() -> str:
 
 
 def build_trace(verbose: bool = False, force: bool = True) -> str:
-    """The diagnostic variant of the library: the bf16 grouped-matmul fast kernels compiled with MS_TRACE_TILES (every
-    workgroup records time stamps of its phases, read back with ms_trace_read; see profile_tools timeline).  Not
-    loaded by anything else; select it with MINDSPEED_AMD_LIB."""
+    """The diagnostic variant of the library: the bf16 grouped-matmul fast kernels and those of both gradients (one
+    translation unit then) compiled with MS_TRACE_TILES (every workgroup records time stamps of its phases, read back with
+    ms_trace_read; see profile_tools timeline).  Not loaded by anything else; select it with MINDSPEED_AMD_LIB."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     objs = [_compile(s, force, ("-DMS_TRACE_TILES",), "_trace") if s.endswith("gmm_fast.hip") else _compile(s, False)
-            for s in sources()]
+            for s in sources() if not s.endswith("gmm_pair.hip")]
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", TRACE_LIB_PATH, *objs]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

@@ -1,5 +1,8 @@
 // One product per launch on the fast 16-bit tiles: the bf16 kernels, and the choice of the type (fp16: gmm_fast_fp16.hip).
 #include "gmm_fast_kernel.h"
+#ifdef MS_TRACE_TILES
+#include "gmm_pair.hip"      // (the stamps of both in one array; the diagnostic library does without the unit of its own)
+#endif
 
 namespace ms {
 

@@ -34,17 +34,7 @@ __global__ __launch_bounds__(256) void gmm16_fast_kernel(const GmmArgs p) {
     } else {
         gmm16_tile<DT, A_RED, B_RED, OUT, 64>(p, tc, lds);
     }
-#ifdef MS_TRACE_TILES
-    if (threadIdx.x == 0) {
-        unsigned hw_id, xcc_id;
-        asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID)" : "=s"(hw_id));
-        asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc_id));
-        long long *rec = g_tile_trace + (blockIdx.x % kTraceSlots) * 8;
-        rec[0] = (static_cast<long long>(xcc_id & 0xf) << 32) | ((hw_id >> 8) & 0xff) | (1ll << 40);   // XCC, CU/SH/SE bits, "valid"
-        rec[5] = wall_clock64();
-        rec[6] = tc.tile_rows;
-    }
-#endif
+    MS_TRACE_END(tc.tile_rows, !A_RED);
 }
 
 template <int DT, int OUT>

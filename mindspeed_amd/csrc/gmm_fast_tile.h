@@ -53,15 +53,30 @@
 #ifdef MS_TRACE_TILES
 // Diagnostic build only (python -m mindspeed_amd.build --trace): every workgroup of the fast kernels records when it
 // started, found its tile, had its first operands in LDS, left the K loop and finished (100 MHz wall clock), plus the
-// compute unit it ran on; ms_trace_read copies the records of the last launches out.  The record of workgroup b is
-// slot b % kTraceSlots, so a launch with more workgroups than that overwrites its own early records.
+// compute unit it ran on, the tile's height and whether it was one of a weight gradient; ms_trace_read copies the records of
+// the last launches out.  The record of workgroup b is slot b % kTraceSlots, so a launch with more workgroups than that
+// overwrites its own early records.  One translation unit: gmm_fast.hip takes gmm_pair.hip in.
 namespace ms {
 constexpr int kTraceSlots = 16384;
 __device__ long long g_tile_trace[kTraceSlots * 8];
 }  // namespace ms
 #define MS_TRACE(i) do { if (threadIdx.x == 0) ms::g_tile_trace[(blockIdx.x % ms::kTraceSlots) * 8 + (i)] = wall_clock64(); } while (0)
+#define MS_TRACE_END(height, weight_gradient) \
+    do { \
+        if (threadIdx.x == 0) { \
+            unsigned hw_id, xcc_id; \
+            asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID)" : "=s"(hw_id)); \
+            asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc_id)); \
+            long long *rec = ms::g_tile_trace + (blockIdx.x % ms::kTraceSlots) * 8; \
+            rec[0] = (static_cast<long long>(xcc_id & 0xf) << 32) | ((hw_id >> 8) & 0xff) | (1ll << 40);   /* XCC, CU/SH/SE bits, "valid" */ \
+            rec[5] = wall_clock64(); \
+            rec[6] = (height); \
+            rec[7] = (weight_gradient) ? 1 : 0; \
+        } \
+    } while (0)
 #else
 #define MS_TRACE(i)
+#define MS_TRACE_END(height, weight_gradient)
 #endif
 
 namespace ms {
@@ -1015,7 +1030,12 @@ __device__ __forceinline__ void gmm16_tile_rows(const GmmArgs &p, const TileCoor
                     // stores they put out what the next kernel reads and have it wait for their write-back.  us per
                     // training pass, ordinary / non-temporal: 16 experts x 750 rows x 2048 x 1536 752 / 732, 64 of 0 to
                     // 7700 rows x 2048 x 1408 3506 / 3483, 8 x 2048 rows x 7168 x 2048 3510 / 3497, 8 x 1024 rows x 4096 x
-                    // 14336 7117 / 7110.
+                    // 14336 7117 / 7110.  Of any size, also where the gradient is read right behind (left alone; added to
+                    // one; copied): 64 x 256 rows x 1024 x 256 (dW 64 and 32 MB) 237 294 282 / 226 297 277, 16 x 750 x 2048 x
+                    // 768 (96 and 48) 467 553 528 / 454 554 519, 8 x 1024 x 4096 x 768 (96 and 48) 595 683 655 / 585 692 652, 16
+                    // x 750 x 2048 x 256 (32 and 16) 253 309 290 / 246 308 282, 8 x 512 x 1024 x 1024 (32 and 16) 163 191 179 /
+                    // 161 192 182; two products of 8 and 16 MB by themselves 18.3 and 28.0 / 17.2 and 27.1, with the
+                    // read 23.1 and 36.2 / 22.5 and 36.3.  No line in the size has one kind on one side.
                     if constexpr (A_RED) *dst = v;
                     else MS_NT_STORE(v, dst);
                 }

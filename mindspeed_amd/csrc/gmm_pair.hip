@@ -1,5 +1,6 @@
 // Both gradients of one grouped matmul in one launch on the fast 16-bit tiles (gmm_fast_tile.h): dX, both operands contiguous
-// along the reduction dim, and dW, neither.
+// along the reduction dim, and dW, neither.  The form with tables and a 16-bit dW keeps four
+// registers in scratch through the last K step, one store and one load per tile; the K loops have none.
 #include "gmm_fast_tile.h"
 
 namespace ms {
@@ -11,14 +12,17 @@ __device__ __forceinline__ void pair_tile(const GmmArgs &p, int b, char *lds) {
     if constexpr (DIRECT) tc = tile_from_list<!RED>(p, b);
     else tc = locate_tile<true, RED>(p.table, b);
     if (!tc.valid) return;
+    MS_TRACE(2);
     if (tc.tile_rows == 256) gmm16_tile<DT, RED, RED, OUT, 256>(p, tc, lds);
     else if (tc.tile_rows == 128) gmm16_tile<DT, RED, RED, OUT, 128>(p, tc, lds);
     else gmm16_tile<DT, RED, RED, OUT, 64>(p, tc, lds);
+    MS_TRACE_END(tc.tile_rows, !RED);
 }
 
 template <int DT, int OUT, bool DIRECT>
 __global__ __launch_bounds__(256) void gmm16_pair_kernel(const GmmArgs dx, const GmmArgs dw, int first, int dw_first) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
+    MS_TRACE(1);
     const int b = blockIdx.x;
     const bool second = b >= first;
     const int own = second ? b - first : b;

@@ -38,7 +38,8 @@ int msi_gmm_backward(ms_stream_t stream, const void *grad, int64_t grad_stride0,
 /* Diagnostic, host only: whether a 16-bit launch split on rows with these group sizes (a host array) gives every XCD
  * consecutive tiles of the whole launch instead of an eighth of every group's, by the rule of the lookup in the group list
  * (from_list != 0) or of the schedule kernel's table; num_cus: the GPU's compute units.  Evaluates the functions the kernels
- * call, so a test can check that a launch takes the order it is meant to.  (A table falls back to eighths where shares equal
+ * call, so a test can check that a launch takes the order it is meant to: a launch of its own, not dX in the launch of both
+ * gradients, where more groups share the rows of their last tiles.  (A table falls back to eighths where shares equal
  * in cost need more workgroups than the launch has, and makes no such shares where it deals out whole groups.) */
 int msi_gmm_takes_together(const int64_t *rows, int64_t num_groups, int64_t k, int64_t n, int from_list, int num_cus,
                            int *together);

@@ -353,14 +353,14 @@ def cmd_power(args):
             time.sleep(1.0)
 
 
-def _products(dev, data, gen, counts=None):
-    """fc1-shaped products of the Mixtral expert MLP: name -> (callable, flops).  counts: rows per expert (eight equal
-    groups by default)."""
+def _products(dev, data, gen, counts=None, dims=(4096, 28672)):
+    """One matmul's products, by default the Mixtral expert MLP's fc1: mode -> callable, and the flops of one product.
+    counts: rows per expert (eight equal groups by default); dims: K and N of the forward product."""
     import torch
 
-    from .ops.gmm import gmm_raw
+    from .ops.gmm import gmm_backward_raw, gmm_raw
 
-    T, H, F, E = 8192, 4096, 14336, 8
+    T, E, H, F = 8192, 8, dims[0], dims[1] // 2
     bf = torch.bfloat16
     if counts:
         T, E = sum(counts), len(counts)
@@ -383,6 +383,10 @@ def _products(dev, data, gen, counts=None):
         if mode == "dw1":
             x, dy = operand(T, H), operand(T, 2 * F)
             return lambda: gmm_raw(x.t(), dy, counts, 2, 1)
+        if mode == "pair1":                            # both gradients in one launch
+            x, dy, w = operand(T, H), operand(T, 2 * F), operand(E, H, 2 * F)
+            dw = torch.empty_like(w)
+            return lambda: gmm_backward_raw(dy, x, w, counts, 1, dw)
         raise SystemExit(f"unknown mode {mode}")
     return make, 2 * T * H * 2 * F
 
@@ -410,13 +414,15 @@ def cmd_timeline(args):
     slots = 16384
     counts = [int(c) for c in args.counts.split(",")] if args.counts else None
     groups = f"{sum(counts)} rows in groups of {args.counts}" if counts else "8192 rows in 8 equal groups"
-    print(f"Mixtral-shape fc1 products ({groups}, hidden 4096, 2*ffn 28672, bf16), one launch each; "
+    dims = [int(d) for d in args.dims.split(",")]
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    print(f"Grouped-matmul products ({groups}, hidden {dims[0]}, 2*ffn {dims[1]}, bf16), one launch each; "
           "times in microseconds from a 100 MHz clock, averaged over the workgroups that held a tile"
-          + (" of the given height (rows)" if counts else ""))
+          + (" of the given height (rows), of dW where so marked" if counts else "") + "; busy: those times over compute units x span")
     print(f"{'product':8s} {'operands':8s} {'tiles':>6s} {'find tile':>10s} {'first data':>11s} {'K loop':>9s} {'epilogue':>9s} "
-          f"{'tile total':>11s} {'idle gap':>9s} {'launch span':>12s} {'MFMA share':>11s}")
+          f"{'tile total':>11s} {'idle gap':>9s} {'launch span':>12s} {'MFMA share':>11s} {'busy':>6s}")
     for data in args.data.split(","):
-        make, flops = _products(dev, data, gen, counts)
+        make, one_product = _products(dev, data, gen, counts, dims)
         for mode in args.modes.split(","):
             fn = make(mode)
             for _ in range(3):
@@ -433,14 +439,19 @@ def cmd_timeline(args):
             if len(rec) == 0:
                 print(f"{mode:8s} {data:8s} no records")
                 continue
-            heights = sorted(set(int(h) for h in rec[:, 6]), reverse=True)
-            if len(heights) > 1:                       # ragged groups: the phases of each tile height by itself
-                for h in heights:
-                    sub = rec[rec[:, 6] == h]
+            flops = 2 * one_product if mode.startswith("pair") else one_product
+            kinds = sorted(set((int(w), -int(h)) for h, w in rec[:, 6:8]))
+            if len(kinds) > 1:                         # ragged groups, two products: the phases of each kind of tile by itself
+                for w, h in kinds:
+                    sub = rec[(rec[:, 6] == -h) & (rec[:, 7] == w) & (rec[:, 3] > 0)]
+                    if len(sub) == 0:
+                        continue
                     ush = lambda a, b: float((sub[:, a] - sub[:, b]).mean()) / 100.0     # noqa: E731
-                    print(f"{mode + ' ' + str(h):8s} {data:8s} {len(sub):6d} {ush(2, 1):10.2f} {ush(3, 2):11.2f} {ush(4, 3):9.2f} "
+                    name = f"{mode} {-h}" + (" dW" if w and mode.startswith("pair") else "")
+                    print(f"{name:8s} {data:8s} {len(sub):6d} {ush(2, 1):10.2f} {ush(3, 2):11.2f} {ush(4, 3):9.2f} "
                           f"{ush(5, 4):9.2f} {ush(5, 1):11.2f}", flush=True)
-            us = lambda a, b: float((rec[:, a] - rec[:, b]).mean()) / 100.0     # noqa: E731
+            looped = rec[rec[:, 3] > 0]                # (a tile of an empty group has no K loop)
+            us = lambda a, b: float((looped[:, a] - looped[:, b]).mean()) / 100.0     # noqa: E731
             gaps = []
             by_cu = {}
             for r in rec:
@@ -455,7 +466,7 @@ def cmd_timeline(args):
             total = us(5, 1)
             print(f"{mode:8s} {data:8s} {tiles_total:6d} {us(2, 1):10.2f} {us(3, 2):11.2f} {us(4, 3):9.2f} {us(5, 4):9.2f} "
                   f"{total:11.2f} {(sum(gaps) / len(gaps) / 100.0) if gaps else float('nan'):9.2f} {span:12.1f} "
-                  f"{mfma_us / total:11.3f}", flush=True)
+                  f"{mfma_us / total:11.3f} {float((rec[:, 5] - rec[:, 1]).sum()) / 100.0 / (cus * span):6.3f}", flush=True)
             del fn
 
 
@@ -483,9 +494,10 @@ def main():
     w.add_argument("--modes", default="fwd1,dx1,dw1")
     w.add_argument("--data", default="randn,small,zeros")
     tl = sub.add_parser("timeline")
-    tl.add_argument("--modes", default="fwd1,dx1,dw1")
+    tl.add_argument("--modes", default="fwd1,dx1,dw1", help="also pair1: dX and dW in one launch")
     tl.add_argument("--data", default="randn,zeros")
     tl.add_argument("--counts", default="", help="comma-separated rows per expert instead of eight equal groups")
+    tl.add_argument("--dims", default="4096,28672", help="K and N of the forward product")
     args = ap.parse_args()
     {"traffic": cmd_traffic, "counters": cmd_counters, "power": cmd_power, "timeline": cmd_timeline,
      "in-layer": cmd_in_layer, "products": cmd_products}[args.cmd](args)
